@@ -12,7 +12,7 @@ The roofline object is the cell stage as the survey's measurement section
 defines it: algorithmic bytes B = 4 N + 24 V + 17 Q (the field read once,
 FP32 position and normal per vertex, an int4 quadrilateral and its colour
 byte) over the summed device time of the cell-stage kernels (k_sweep,
-k_rows, k_vertices, k_vertices_slow, k_quads and the scans between them),
+k_cells, k_vertices, k_vertices_slow, k_quads and the scans between them),
 timed with HIP events on the engine's stream over the timed steps.
 `kernels` lists the main kernels with their own byte models and fractions.
 The CPU baseline is the reference cpp_dmc compiled from its sources
@@ -42,7 +42,7 @@ HBM_PEAK_GBS = 8000.0
 # 1.14 GB, k_vertices (its 3-wave form) 11.46 GB, k_quads 8.27 GB, the cell
 # scans 0.47 GB.
 TRAFFIC = {"schwarz_1024": 27_100_000_000}
-CELL_KERNELS = ("k_sweep", "k_scan_cells", "k_vol_abase", "k_rows", "k_vol_bounds", "k_vertices", "k_vertices_slow",
+CELL_KERNELS = ("k_sweep", "k_scan_cells", "k_vol_abase", "k_cells", "k_vol_bounds", "k_vertices", "k_vertices_slow",
                 "k_quads")
 
 
@@ -620,7 +620,7 @@ def main():
     R = (grid.ny - 1) * (grid.nz - 1)
     models = {
         "k_sweep": (4 * nvox, "4 N (field read once)"),
-        "k_rows": (4 * A + 20 * A + 8 * R, "4 A list entries read + 20 A per-cell words + 8 R row totals written"),
+        "k_cells": (4 * A + 16 * A, "4 A list entries read + 16 A per-cell records written"),
         "k_vertices": (24 * V, "24 V (FP32 position + normal; the engine writes FP64, 48 V)"),
         "k_quads": (17 * Q + 32 * Q, "17 Q (int4 quad + colour) + 32 Q (first halfedge rows)"),
         "k_he_twins": (16 * Q + 32 * Q + 20 * Q + 4 * V,

@@ -75,7 +75,6 @@ __device__ __forceinline__ bool edge_interior(int e, int i, int j, int k, int nx
 // MC polygons, packed: bits 0..15 = four 4-bit contour sizes (0 = absent),
 // bits 16..63 = edge ids, contour after contour.
 // ---------------------------------------------------------------------------
-__device__ __constant__ uint64_t c_case_contours[256] = DMC_CASE_CONTOURS_INIT;
 __device__ __constant__ uint64_t c_ambiguous[4] = DMC_AMBIGUOUS_MASK_INIT;
 
 __device__ __forceinline__ bool case_ambiguous(unsigned icase) {
@@ -101,76 +100,128 @@ __device__ __forceinline__ double asymptotic_decider(double f0, double f1, doubl
 // Polygons of an ambiguous case (cpp_dmc/DualMarchingCubes.cpp:328-461):
 // each face contributes oriented segments, faces with two opposite positive
 // corners are split by the asymptotic decider, and segments are chained into
-// contours starting from the lowest intersected edge.
-__device__ inline uint64_t polygons_decider(double iso, const double F[8]) {
-    uint64_t outs = 0;   // 4-bit successor per edge
-    unsigned set = 0;    // edges touched by a segment
+// contours starting from the lowest intersected edge (chain).  The contours
+// of every case under every outcome of its ambiguous faces' deciders are
+// formed at compile time, so that a cell takes its polygons from a table:
+// chaining them in the kernels is a divergent loop that held up the waves of
+// noisy volumes.  Entry start[case] + dec: bit n of dec is "decider value >=
+// iso" of the case's n-th ambiguous face, in face order.  Cases without a
+// decider have one entry.
+constexpr int kContourEntries = 656;   // 128 + the outcomes of the 128 decided cases
+constexpr int kMaxDecisions = 6;       // a cell's faces
+struct ContourTable {
+    uint64_t w[kContourEntries];
+    uint32_t map[kContourEntries];   // contour of each edge (2 bits per edge) | contours << 24
+    uint16_t start[256];
+    int n;
+    static constexpr int face_case(unsigned icase, int f) {
+        int fc = 0;
+        for (int q = 0; q < 4; q++) fc |= (int)((icase >> kFaceV[f][q]) & 1u) << q;
+        return fc;
+    }
+    // bit n of skip: the n-th ambiguous face's decider is neither above nor
+    // below (NaN), the face has no segments
+    static constexpr uint64_t chain(unsigned icase, unsigned dec, unsigned skip) {
+        // oriented segments (from | to << 4, face edge numbers) of the face
+        // cases; two of them under a decider, whose outcome picks the pair
+        constexpr uint8_t seg[16] = {0, 0x30, 0x01, 0x31, 0x23, 0x20, 0, 0x21, 0x12, 0, 0x02, 0x32, 0x13, 0x10, 0x03, 0};
+        constexpr uint8_t two[2][2][2] = {{{0x01, 0x23}, {0x03, 0x21}}, {{0x30, 0x12}, {0x10, 0x32}}};
+        uint64_t outs = 0;
+        unsigned set = 0;
+        int nd = 0;
+#pragma unroll 1
+        for (int f = 0; f < 6; f++) {
+            const int fc = face_case(icase, f);
+            int ns = fc == 0 || fc == 15 ? 0 : 1;
+            uint8_t sg[2] = {seg[fc], 0};
+            if (fc == 6 || fc == 9) {
+                const int d = (int)((dec >> nd) & 1u);
+                ns = ((skip >> nd) & 1u) ? 0 : 2;
+                nd++;
+                sg[0] = two[fc == 9][d][0];
+                sg[1] = two[fc == 9][d][1];
+            }
+            for (int q = 0; q < ns; q++) {
+                const int a = kFaceE[f][sg[q] & 0xF], b = kFaceE[f][sg[q] >> 4];
+                outs = (outs & ~(0xFull << (4 * a))) | ((uint64_t)b << (4 * a));
+                set |= (1u << a) | (1u << b);
+            }
+        }
+        uint64_t w = 0;
+        int cnt = 0, pos = 0;
+#pragma unroll 1
+        for (int e = 0; e < 12; e++) {
+            if (!((set >> e) & 1u)) continue;
+            if (cnt >= 4 || pos >= 12) break;
+            int size = 1;
+            w |= (uint64_t)e << (16 + 4 * pos);
+            pos++;
+            int to = (int)((outs >> (4 * e)) & 0xF);
+            while (to != e && to < 12 && pos < 12) {
+                w |= (uint64_t)to << (16 + 4 * pos);
+                pos++;
+                size++;
+                const int cur = to;
+                to = (int)((outs >> (4 * cur)) & 0xF);
+                set &= ~(1u << cur);
+            }
+            w |= (uint64_t)size << (4 * cnt);
+            cnt++;
+        }
+        return w;
+    }
+    static constexpr uint32_t map_of(uint64_t w) {
+        uint32_t m = 0, cnt = 0;
+        int pos = 0;
+        for (int t = 0; t < 4; t++) {
+            const int sz = (int)((w >> (4 * t)) & 0xF);
+            for (int q = 0; q < sz; q++) m |= (uint32_t)t << (2 * (int)((w >> (16 + 4 * (pos + q))) & 0xF));
+            pos += sz;
+            cnt += sz != 0;
+        }
+        return m | cnt << 24;
+    }
+    constexpr ContourTable() : w(), map(), start(), n(0) {
+        constexpr uint64_t contours[256] = DMC_CASE_CONTOURS_INIT;
+        constexpr uint64_t amb[4] = DMC_AMBIGUOUS_MASK_INIT;
+        for (int c = 0; c < 256; c++) {
+            start[c] = (uint16_t)n;
+            int nd = 0;
+            for (int f = 0; f < 6; f++) nd += face_case(c, f) == 6 || face_case(c, f) == 9;
+            const bool decided = (amb[c >> 6] >> (c & 63)) & 1ull;
+            for (unsigned d = 0; d < (decided ? 1u << nd : 1u); d++) {
+                w[n] = decided ? chain((unsigned)c, d, 0) : contours[c];
+                map[n] = map_of(w[n]);
+                n++;
+            }
+        }
+    }
+};
+constexpr ContourTable kContours{};
+static_assert(kContours.n == kContourEntries, "entries of the contour table");
+__device__ __constant__ ContourTable c_contours{};
+
+// Outcomes of the deciders of case icase's ambiguous faces: the index into its
+// contours, and above kMaxDecisions the faces whose decider is neither above
+// nor below (NaN), which the table does not hold.
+__device__ __forceinline__ unsigned case_decisions(unsigned icase, double iso, const double F[8]) {
+    unsigned dec = 0;
+    int nd = 0;
 #pragma unroll
     for (int f = 0; f < 6; f++) {
-        const double f0 = F[kFaceV[f][0]], f1 = F[kFaceV[f][1]], f2 = F[kFaceV[f][2]], f3 = F[kFaceV[f][3]];
-        const int e0 = kFaceE[f][0], e1 = kFaceE[f][1], e2 = kFaceE[f][2], e3 = kFaceE[f][3];
-        const unsigned fc = (unsigned)(f0 >= iso) | (unsigned)(f1 >= iso) << 1 |
-                            (unsigned)(f2 >= iso) << 2 | (unsigned)(f3 >= iso) << 3;
-        int a0 = -1, b0 = -1, a1 = -1, b1 = -1;   // up to two segments a->b
-        switch (fc) {
-        case 1: a0 = e0; b0 = e3; break;
-        case 2: a0 = e1; b0 = e0; break;
-        case 3: a0 = e1; b0 = e3; break;
-        case 4: a0 = e3; b0 = e2; break;
-        case 5: a0 = e0; b0 = e2; break;
-        case 6: {
-            const double val = asymptotic_decider(f0, f1, f2, f3);
-            if (val >= iso) { a0 = e3; b0 = e0; a1 = e1; b1 = e2; }
-            else if (val < iso) { a0 = e1; b0 = e0; a1 = e3; b1 = e2; }
-        } break;
-        case 7: a0 = e1; b0 = e2; break;
-        case 8: a0 = e2; b0 = e1; break;
-        case 9: {
-            const double val = asymptotic_decider(f0, f1, f2, f3);
-            if (val >= iso) { a0 = e0; b0 = e1; a1 = e2; b1 = e3; }
-            else if (val < iso) { a0 = e0; b0 = e3; a1 = e2; b1 = e1; }
-        } break;
-        case 10: a0 = e2; b0 = e0; break;
-        case 11: a0 = e2; b0 = e3; break;
-        case 12: a0 = e3; b0 = e1; break;
-        case 13: a0 = e0; b0 = e1; break;
-        case 14: a0 = e3; b0 = e0; break;
-        default: break;
-        }
-        if (a0 >= 0) {
-            outs = (outs & ~(0xFull << (4 * a0))) | ((uint64_t)b0 << (4 * a0));
-            set |= (1u << a0) | (1u << b0);
-        }
-        if (a1 >= 0) {
-            outs = (outs & ~(0xFull << (4 * a1))) | ((uint64_t)b1 << (4 * a1));
-            set |= (1u << a1) | (1u << b1);
-        }
+        const unsigned fc = ((icase >> kFaceV[f][0]) & 1u) | ((icase >> kFaceV[f][1]) & 1u) << 1 |
+                            ((icase >> kFaceV[f][2]) & 1u) << 2 | ((icase >> kFaceV[f][3]) & 1u) << 3;
+        if (fc != 6u && fc != 9u) continue;
+        const double val = asymptotic_decider(F[kFaceV[f][0]], F[kFaceV[f][1]], F[kFaceV[f][2]], F[kFaceV[f][3]]);
+        if (val >= iso) dec |= 1u << nd;
+        else if (!(val < iso)) dec |= 1u << (kMaxDecisions + nd);
+        nd++;
     }
-    uint64_t w = 0;
-    int cnt = 0, pos = 0;
-    for (int e = 0; e < 12; e++) {
-        if (!((set >> e) & 1u)) continue;
-        if (cnt >= 4 || pos >= 12) break;
-        int size = 1;
-        w |= (uint64_t)e << (16 + 4 * pos);
-        pos++;
-        int to = (int)((outs >> (4 * e)) & 0xF);
-        while (to != e && to < 12 && pos < 12) {
-            w |= (uint64_t)to << (16 + 4 * pos);
-            pos++;
-            size++;
-            const int cur = to;
-            to = (int)((outs >> (4 * cur)) & 0xF);
-            set &= ~(1u << cur);
-        }
-        w |= (uint64_t)size << (4 * cnt);
-        cnt++;
-    }
-    return w;
+    return dec;
 }
-
-__device__ __forceinline__ uint64_t cell_polygons(unsigned icase, double iso, const double F[8]) {
-    return case_ambiguous(icase) ? polygons_decider(iso, F) : c_case_contours[icase];
+__device__ __forceinline__ bool undecided(unsigned dec) { return dec >= 1u << kMaxDecisions; }
+__device__ inline uint64_t chained_contours(unsigned icase, unsigned dec) {
+    return ContourTable::chain(icase, dec & ((1u << kMaxDecisions) - 1u), dec >> kMaxDecisions);
 }
 
 // Pick element t of a 4-array without dynamic register indexing.

@@ -102,7 +102,7 @@ struct dmc_context {
     std::string err;
     std::vector<Buf*> bufs;
     // cell sweep
-    Buf segCount, segBase, segMask, lists, acell, acode, aaux, avloc, aqloc, rowV, rowQ, rowBaseV, rowBaseQ;
+    Buf segCount, segBase, segMask, lists, acell, acode, rec, grpNV, grpNQ, grpV, grpQ;
     Buf field, grads, scanPartial, scanState, scanTotal, sizes;
     // volume table of the last extraction (one volume, or a batch) and the
     // per-volume first active cell / vertex / quadrilateral, kept through
@@ -193,7 +193,7 @@ struct dmc_context {
     size_t arena_cap = 0, arena_used = 0;
 
     dmc_context() {
-        Buf* all[] = {&segCount, &segBase, &segMask, &lists, &acell, &acode, &aaux, &avloc, &aqloc, &rowV, &rowQ, &rowBaseV, &rowBaseQ,
+        Buf* all[] = {&segCount, &segBase, &segMask, &lists, &acell, &acode, &rec, &grpNV, &grpNQ, &grpV, &grpQ,
                       &field, &grads, &scanPartial, &scanState, &scanTotal, &sizes, &pos[0], &pos[1], &nrm[0], &nrm[1], &vslot[0], &vslot[1],
                       &quads[0], &quads[1], &colors, &deg, &off, &cursor, &adj, &twin, &flag, &hev, &ovr,
                       &bndrec, &nbnd, &val, &p, &em, &vfirst, &vsecond, &lastT, &lastR, &newV,
@@ -570,7 +570,7 @@ float smallest_float_not_below(double iso) {
     return f;
 }
 
-int64_t* vol_ptr(dmc_context* ctx, int which) {  // 0 waveBase, 1 rowBase, 2 aBase
+int64_t* vol_ptr(dmc_context* ctx, int which) {  // 0 waveBase, 1 grpBase, 2 aBase
     const size_t n = (size_t)ctx->nvol;
     uint8_t* base = static_cast<uint8_t*>(ctx->vtab.p) + n * sizeof(VolDesc);
     return reinterpret_cast<int64_t*>(base) + (size_t)which * (n + 1);
@@ -583,7 +583,7 @@ VolTable vol_table(dmc_context* ctx) {
 
 // What the field sweep leaves for the cell stages.
 struct Swept {
-    int64_t R;      // cell rows (all volumes)
+    int64_t groups; // groups of (row, segment)s (all volumes)
     int64_t cells;  // cells (all volumes)
     VolTable vt;
     VolStat* vstat;
@@ -594,10 +594,18 @@ struct Swept {
 // Host side of a pass: the volume table (built in ctx->vtab_host, uploaded
 // by upload_vtab) and the sweep's tiling.
 struct SweepPlan {
-    int64_t W, R, RS, cells;
+    int64_t W, RS, groups, cells;
     bool vec;
     size_t tab_bytes;
 };
+
+// (row, segment)s per wave of k_cells and k_tmc_cells (2^n), from their total:
+// enough waves to fill the chip come first, cells per wave second.  k_cells
+// with 1 / 2 / 4 / 8 / 16 of them per wave, us: 32^3 (961 in all) 4.6 / 4.6 /
+// 5.2 / 6.4 / 8.0; 201x174x149 (25,752) 17 / 13 / 13 / 18 / 29; 301x257x283
+// (144,384) 107 / 68 / 48 / 39 / 36; 1024^3 (4.2 M) 1606 / 1008 / 799 / 620 /
+// 511.
+int group_shift(int64_t rs) { return rs >= (1 << 16) ? 4 : rs >= (1 << 13) ? 2 : 0; }
 
 template <class T>
 SweepPlan plan_sweep(dmc_context* ctx, const std::vector<HostVol>& hv) {
@@ -634,27 +642,29 @@ SweepPlan plan_sweep(dmc_context* ctx, const std::vector<HostVol>& hv) {
     const size_t tab_bytes = (size_t)n * sizeof(VolDesc) + 3 * (size_t)(n + 1) * sizeof(int64_t);
     ctx->vtab_host.assign(tab_bytes, 0);
     int64_t* waveBase = reinterpret_cast<int64_t*>(ctx->vtab_host.data() + (size_t)n * sizeof(VolDesc));
-    int64_t* rowBase = waveBase + (n + 1);
-    int64_t W = 0, R = 0, RS = 0;
+    int64_t* grpBase = waveBase + (n + 1);
+    int64_t W = 0, RS = 0;
     bool vec = true;
+    int64_t rs_all = 0;
+    for (int v = 0; v < n; v++) rs_all += desc[v].d.R * desc[v].S;
+    const int gsh = group_shift(rs_all);
     for (int v = 0; v < n; v++) {
         VolDesc& D = desc[v];
         D.K = std::min(Kg, D.d.nz - 1);
         D.ntk = (D.d.nz - 1 + D.K - 1) / D.K;
-        D.rowBase = R;
         D.rsBase = RS;
+        D.gsh = gsh;
         waveBase[v] = W;
-        rowBase[v] = R;
+        grpBase[v] = RS >> gsh;
         W += (int64_t)D.S * D.ntj * D.ntk;
-        R += D.d.R;
-        RS += D.d.R * D.S;
+        RS += (D.d.R * D.S + kGroup - 1) / kGroup * kGroup;
         vec = vec && (D.d.nx % 4 == 0) && ((uintptr_t)D.field % (4 * sizeof(T)) == 0);
     }
     waveBase[n] = W;
-    rowBase[n] = R;
+    grpBase[n] = RS >> gsh;
     memcpy(ctx->vtab_host.data(), desc.data(), (size_t)n * sizeof(VolDesc));
     ensure<uint8_t>(ctx, ctx->vtab, tab_bytes);
-    return SweepPlan{W, R, RS, cells, vec, tab_bytes};
+    return SweepPlan{W, RS, RS >> gsh, cells, vec, tab_bytes};
 }
 
 // The volume table to the device (before the pass's launches; a replayed
@@ -670,7 +680,7 @@ void upload_vtab(dmc_context* ctx, const SweepPlan& P) {
 template <class T>
 Swept sweep_cells(dmc_context* ctx, const SweepPlan& P) {
     const int n = ctx->nvol;
-    const int64_t W = P.W, R = P.R, RS = P.RS;
+    const int64_t W = P.W, RS = P.RS;
     const VolTable vt = vol_table(ctx);
     VolStat* vstat = ensure<VolStat>(ctx, ctx->vstat, n);
     Sizes* S = reinterpret_cast<Sizes*>(ensure<uint8_t>(ctx, ctx->sizes, sizeof(Sizes)));
@@ -694,7 +704,7 @@ Swept sweep_cells(dmc_context* ctx, const SweepPlan& P) {
     if (n > 1)
         launch(ctx, "k_vol_abase", k_vol_abase, dim3(grid_for(ctx, n + 1)), dim3(kBlock), vt, segBase, &S->A,
                vol_ptr(ctx, 2));
-    return Swept{R, P.cells, vt, vstat, lists, segCount, segBase, segMask};
+    return Swept{P.groups, P.cells, vt, vstat, lists, segCount, segBase, segMask};
 }
 
 // Capacities of the cell-stage arrays for a pass over the volumes `hv`: per
@@ -746,22 +756,18 @@ void run_cells(dmc_context* ctx, const SweepPlan& P) {
     const Swept sw = sweep_cells<T>(ctx, P);
     const int n = ctx->nvol;
     const int64_t acap = ctx->acap, vcap = ctx->vcap, qcap = ctx->qcap;
-    const int64_t R = sw.R;
+    const int64_t G = sw.groups;
     const VolTable vt = sw.vt;
     Sizes* S = dsizes(ctx);
-    uint32_t* acell = ensure<uint32_t>(ctx, ctx->acell, acap);
-    uint32_t* acode = ensure<uint32_t>(ctx, ctx->acode, acap);
-    uint32_t* aaux = ensure<uint32_t>(ctx, ctx->aaux, acap);
-    uint32_t* avloc = ensure<uint32_t>(ctx, ctx->avloc, acap);
-    uint32_t* aqloc = ensure<uint32_t>(ctx, ctx->aqloc, acap);
-    uint32_t* rowV = ensure<uint32_t>(ctx, ctx->rowV, R);
-    uint32_t* rowQ = ensure<uint32_t>(ctx, ctx->rowQ, R);
-    uint32_t* rowBaseV = ensure<uint32_t>(ctx, ctx->rowBaseV, R);
-    uint32_t* rowBaseQ = ensure<uint32_t>(ctx, ctx->rowBaseQ, R);
-    launch(ctx, "k_rows", k_rows<T>, dim3(grid_for(ctx, R, kBlock / kWave)), dim3(kBlock), vt, R, sw.lists,
-           sw.segCount, sw.segBase, acell, acode, aaux, avloc, aqloc, rowV, rowQ, sw.vstat, S->cpart, (uint32_t)acap);
-    check_launch(ctx, "k_rows");
-    scan_pair(ctx, scan_job(ScanCounts{rowV}, rowBaseV, hn(R), &S->V), scan_job(ScanCounts{rowQ}, rowBaseQ, hn(R), &S->Q),
+    uint4* rec = ensure<uint4>(ctx, ctx->rec, acap);
+    uint32_t* grpNV = ensure<uint32_t>(ctx, ctx->grpNV, G);
+    uint32_t* grpNQ = ensure<uint32_t>(ctx, ctx->grpNQ, G);
+    uint32_t* grpV = ensure<uint32_t>(ctx, ctx->grpV, G);
+    uint32_t* grpQ = ensure<uint32_t>(ctx, ctx->grpQ, G);
+    launch(ctx, "k_cells", k_cells<T>, dim3(grid_for(ctx, G, kBlock / kWave)), dim3(kBlock), vt, G, sw.lists,
+           sw.segCount, sw.segBase, rec, grpNV, grpNQ, sw.vstat, S->cpart, (uint32_t)acap);
+    check_launch(ctx, "k_cells");
+    scan_pair(ctx, scan_job(ScanCounts{grpNV}, grpV, hn(G), &S->V), scan_job(ScanCounts{grpNQ}, grpQ, hn(G), &S->Q),
               "k_scan_cells");
     // cells deferred to the general sampling: slow[0] = count (zeroed by the
     // guard), then cell ids
@@ -772,7 +778,7 @@ void run_cells(dmc_context* ctx, const SweepPlan& P) {
     int64_t* vb = ensure<int64_t>(ctx, ctx->vbound, 2 * (size_t)(n + 1));
     int64_t* qb = ensure<int64_t>(ctx, ctx->qbound, 2 * (size_t)(n + 1));
     if (n > 1)
-        launch(ctx, "k_vol_bounds", k_vol_bounds, dim3(grid_for(ctx, n + 1)), dim3(kBlock), vt, rowBaseV, rowBaseQ, S,
+        launch(ctx, "k_vol_bounds", k_vol_bounds, dim3(grid_for(ctx, n + 1)), dim3(kBlock), vt, grpV, grpQ, S,
                vb, qb);
     ctx->cur = 0;
     ctx->pcur = 0;
@@ -794,20 +800,19 @@ void run_cells(dmc_context* ctx, const SweepPlan& P) {
     // threads (F32 fields: the F64 form would spill at 3 waves)
     const dim3 gv(grid_for(ctx, acap, kBlock, kVerticesBlocks));
     if (std::is_same<T, float>::value && acap > kVerticesBlocks * kBlock)
-        launch(ctx, "k_vertices", k_vertices_wide<T>, gv, dim3(kBlock), vt, acell, acode, aaux, avloc, rowBaseV, A,
-               pos, nrm, deg, slow, &S->qhead);
+        launch(ctx, "k_vertices", k_vertices_wide<T>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, deg,
+               slow, &S->qhead);
     else
-        launch(ctx, "k_vertices", k_vertices<T>, gv, dim3(kBlock), vt, acell, acode, aaux, avloc, rowBaseV, A, pos,
-               nrm, deg, slow, &S->qhead);
+        launch(ctx, "k_vertices", k_vertices<T>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, deg, slow,
+               &S->qhead);
     check_launch(ctx, "k_vertices");
     launch(ctx, "k_vertices_slow", k_vertices_slow<T>, dim3(grid_for(ctx, acap, kBlock, 1024)), dim3(kBlock), vt,
-           acell, acode, aaux, avloc, rowBaseV, slow, pos, nrm, deg, sw.vstat);
+           rec, grpV, slow, pos, nrm, deg, sw.vstat);
     check_launch(ctx, "k_vertices_slow");
     mark(ctx, "quads");
     // the row total must be 4 Q (checked with the pass's sizes at the end)
     scan_to(ctx, ScanCounts{deg}, off, dn(&S->nv, vcap), &S->rows, "k_scan_cells", nullptr, off);
-    launch(ctx, "k_quads", k_quads, dim3(grid_for(ctx, acap)), dim3(kBlock), vt, acell, acode, aaux, avloc, aqloc,
-           rowBaseV, rowBaseQ, A, sw.segMask, sw.segBase, quads, colors, off, adj, (uint64_t)(4 * qcap),
+    launch(ctx, "k_quads", k_quads, dim3(grid_for(ctx, acap)), dim3(kBlock), vt, rec, grpV, grpQ, A, sw.segMask, sw.segBase, quads, colors, off, adj, (uint64_t)(4 * qcap),
            &S->unresolved);
     check_launch(ctx, "k_quads");
     ctx->ready = 1;
@@ -1286,7 +1291,7 @@ void run_tmc(dmc_context* ctx, const std::vector<HostVol>& hv) {
     const Swept sw = sweep_cells<T>(ctx, P);
     const uint64_t A = read_u64(ctx, &dsizes(ctx)->A);
     if (A > 0xFFFFFFFFull) fail(ctx, DMC_ERR_CAPACITY, "too many active cells (%llu)", (unsigned long long)A);
-    const int64_t R = sw.R;
+    const int64_t G = sw.groups;
     uint32_t* acell = ensure<uint32_t>(ctx, ctx->acell, A);
     uint32_t* acode = ensure<uint32_t>(ctx, ctx->acode, A);
     uint32_t* cnt_v = ensure<uint32_t>(ctx, ctx->tcntv, A);
@@ -1297,7 +1302,7 @@ void run_tmc(dmc_context* ctx, const std::vector<HostVol>& hv) {
     uint32_t* amb = ensure<uint32_t>(ctx, ctx->tamb, A + 1);
     fill_u32(ctx, st, hn(6), 0u);
     fill_u32(ctx, amb, hn(1), 0u);
-    launch(ctx, "k_tmc_cells", k_tmc_cells, dim3(grid_for(ctx, R, kBlock / kWave)), dim3(kBlock), sw.vt, R, sw.lists,
+    launch(ctx, "k_tmc_cells", k_tmc_cells, dim3(grid_for(ctx, G, kBlock / kWave)), dim3(kBlock), sw.vt, G, sw.lists,
            sw.segCount, sw.segBase, acell, acode, cnt_v, cnt_t, amb, st);
     check_launch(ctx, "k_tmc_cells");
     if (A > 0) {

@@ -11,10 +11,10 @@
 //   active    a = segBase[r*S + s] + m enumerates the active cells in
 //             (k, j, i) order, the reference's vertex order
 //             (cpp_dmc/DualMarchingCubes.cpp:16-50 with :167-171):
-//             acell[a] (linear cell index), acode[a] (case | edge-to-contour
-//             map << 8), avloc[a] / aqloc[a] (first vertex / quadrilateral
-//             of the cell relative to its row); rowBaseV / rowBaseQ are the
-//             scans of the row totals.
+//             rec[a] (ActRec) holds its linear cell index, case,
+//             edge-to-contour map, interior edges and first vertex /
+//             quadrilateral relative to its group of (row, segment)s;
+//             grpV / grpQ are the scans of the groups' totals.
 #pragma once
 #include <utility>
 
@@ -48,8 +48,8 @@ struct VolDesc {
     double iso_t;          // comparison threshold, exact in the field type
     double rdx2[3];        // 1 / (2 dx), 1 / (2 dy), 1 / (2 dz) correctly rounded, or 0 (divide instead)
     int S, ntj, K, ntk;    // sweep tiling: segments per row, row tiles, planes per wave, plane tiles
-    int64_t rowBase;       // first global cell row
-    int64_t rsBase;        // first global (row, segment)
+    int64_t rsBase;        // first global (row, segment), a multiple of kGroup
+    int gsh;               // (row, segment)s per group (wave of k_cells): 2^gsh, the same for all volumes
 };
 
 struct VolStat {
@@ -60,7 +60,7 @@ struct VolStat {
 struct VolTable {
     const VolDesc* desc;
     const int64_t* waveBase;   // n+1: first sweep wave of each volume
-    const int64_t* rowBase;    // n+1: first global cell row
+    const int64_t* grpBase;    // n+1: first group of (row, segment)s
     const int64_t* aBase;      // n+1: first active cell (set after the sweep's scan)
     int n;
 };
@@ -82,6 +82,7 @@ struct VolTable {
 // float not below iso: the same predicate.
 // ---------------------------------------------------------------------------
 constexpr int kSeg = 256;           // cells per segment (one wave) and list slots per (row, segment)
+constexpr int kGroup = 16;          // most (row, segment)s per wave of k_cells; a volume is padded to whole ones
 #ifndef TMC_SWEEP_ROWS
 #define TMC_SWEEP_ROWS 16
 #endif
@@ -302,6 +303,11 @@ __global__ void __launch_bounds__(kBlock) k_sweep(VolTable vt, int64_t waves, ui
     else
         sweep_march<T, VEC, false>(field, d, k0, k1, j0, nj, S, s, i0, ie, valid, iso_t, lane, lists, segCount,
                                    segMask);
+    // the volume's last wave empties the padding of its last group
+    if (wave == vt.waveBase[v + 1] - vt.waveBase[v] - 1) {
+        const int64_t rs = d.R * S + lane;
+        if (rs < (d.R * S + kGroup - 1) / kGroup * kGroup) segCount[rs] = 0;
+    }
 }
 
 // A volume's field as a global-memory pointer.  The descriptor keeps a
@@ -367,7 +373,7 @@ __device__ __forceinline__ uint32_t contour_spread(uint32_t map, unsigned t) {
     return ~(x | (x >> 1)) & kAllEdgesSpread;
 }
 // Per active cell: interior cut edges (spread, bits 0..23) and used
-// contours (bits 24..27), formed once in k_rows.  Used contours are those
+// contours (bits 24..27), formed once in k_cells.  Used contours are those
 // with at least one interior edge; the others only feed incomplete
 // quadrilaterals and are dropped by removeUnusedVertices
 // (cpp_dmc/DualMarchingCubes.h:685-729).  A vertex's quadrilaterals are
@@ -386,23 +392,89 @@ __device__ __forceinline__ int contour_rank(uint32_t map, uint32_t aux, unsigned
     return __popc(contour_spread(map, t) & aux & c_cut_spread.v[icase] & kAllEdgesSpread & ((1u << (2 * e)) - 1u));
 }
 
+// One active cell, 16 bytes, so that a neighbour lookup is one load.
+struct ActRec {
+    uint32_t cell;   // linear cell index in its volume
+    uint32_t code;   // case | edge-to-contour map << 8
+    uint32_t aux;    // cell_aux | decider outcomes 0..3 << 28
+    uint32_t loc;    // first vertex | undecided << 15 | first quadrilateral << 16 | decider outcomes 4, 5 << 30
+    __device__ __forceinline__ uint32_t vloc() const { return loc & 0x3FFFu; }
+    __device__ __forceinline__ uint32_t qloc() const { return (loc >> 16) & 0x3FFFu; }
+    __device__ __forceinline__ unsigned used() const { return (aux >> 24) & 0xFu; }
+    __device__ __forceinline__ bool undecided() const { return (loc & 0x8000u) != 0u; }
+    __device__ __forceinline__ uint64_t contours() const {
+        return c_contours.w[c_contours.start[code & 0xFFu] + (aux >> 28 | loc >> 30 << 4)];
+    }
+};
+static_assert(4 * kGroup * kSeg <= 1 << 14, "a group's vertices are counted in 14 bits");
+
+__device__ __forceinline__ ActRec load_rec(const uint4* __restrict__ rec, int64_t a) {
+    const uint4 x = rec[a];
+    return ActRec{x.x, x.y, x.z, x.w};
+}
+
+// The (row, segment)s of a group, one per lane below the group's size (the
+// lanes above it start past everything): where each starts in the group's
+// active order and its cell row.
+struct GroupLanes {
+    uint32_t rel;     // active cells of the group before it
+    int j, k;         // cell row
+    uint32_t first;   // (wave-uniform) flat index of the group's first active cell
+    uint32_t total;   // (wave-uniform) active cells of the group
+};
+
+__device__ __forceinline__ GroupLanes load_group(const VolDesc& V, int64_t g, int lane,
+                                                 const uint32_t* __restrict__ segCount,
+                                                 const uint32_t* __restrict__ segBase) {
+    const int last = (1 << V.gsh) - 1;
+    const int64_t rs = (g << V.gsh) + min(lane, last);
+    const uint32_t base = segBase[rs];
+    GroupLanes L;
+    L.first = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+    L.rel = base - L.first;
+    const uint32_t end = L.rel + segCount[rs];
+    L.total = (uint32_t)__builtin_amdgcn_readlane((int)end, last);
+    if (lane > last) L.rel = 0xFFFFFFFFu;
+    const uint32_t r = (uint32_t)(rs - V.rsBase) / (uint32_t)V.S;
+    L.k = (int)(r / (uint32_t)(V.d.ny - 1));
+    L.j = (int)(r - (uint32_t)L.k * (uint32_t)(V.d.ny - 1));
+    return L;
+}
+
+// The (row, segment) of the group that holds the group's x-th active cell:
+// the last one that starts at or before it (an empty one starts where the
+// next does).
+__device__ __forceinline__ int group_seg(const GroupLanes& L, uint32_t x) {
+    int s = 0;
+#pragma unroll
+    for (int q = 1; q < kGroup; q++) s += (uint32_t)__builtin_amdgcn_readlane((int)L.rel, q) <= x;
+    return s;
+}
+
 // ---------------------------------------------------------------------------
-// K2: one wave per row, cells in ascending x: polygons of every active cell
-// -> code, kept vertices and owned quadrilaterals (edges e0, e3, e8 of the
-// cell with all four neighbour cells present) and their prefix inside the
-// row; the flat active arrays; row totals for the row scans.  Counts every
-// contour for the reference's pre-removal vertex count.
+// K2: polygons of every active cell -> its record: case and contour map,
+// kept vertices and owned quadrilaterals (edges e0, e3, e8 of the cell with
+// all four neighbour cells present) as their prefix inside the group; group
+// totals for the scans.  Counts every contour for the reference's
+// pre-removal vertex count.
+//
+// One wave per group of 2^gsh consecutive (row, segment)s, whose active
+// cells it takes 64 at a time in the flat order.  Bound by the latency of a
+// wave's chain (bases, list entry, case table, store), so what counts is
+// active cells per chain: a row of the 1024^3 Schwarz-P volume holds 31, a
+// row of a small volume under ten, and a wave per row left most lanes idle
+// (1024^3: 1009 -> 511 us, 0.95 TB/s of list entries and records; 1,024
+// volumes of 16-96 points per axis: 1508 -> 323 us).  Contours come from the
+// decided table instead of being chained here and again in k_vertices: 512^3
+// blobs with noise, 352 -> 140 us here and 1267 -> 1094 us there.
 // ---------------------------------------------------------------------------
 template <class T>
-__global__ void __launch_bounds__(kBlock) k_rows(VolTable vt, int64_t Rtot, const uint32_t* __restrict__ lists,
-                                                  const uint32_t* __restrict__ segCount,
-                                                  const uint32_t* __restrict__ segBase,
-                                                  uint32_t* __restrict__ acell, uint32_t* __restrict__ acode,
-                                                  uint32_t* __restrict__ aaux,
-                                                  uint32_t* __restrict__ avloc, uint32_t* __restrict__ aqloc,
-                                                  uint32_t* __restrict__ rowV, uint32_t* __restrict__ rowQ,
-                                                  VolStat* __restrict__ vstat, unsigned long long* __restrict__ cpart,
-                                                  uint32_t acap) {
+__global__ void __launch_bounds__(kBlock) k_cells(VolTable vt, int64_t groups, const uint32_t* __restrict__ lists,
+                                                   const uint32_t* __restrict__ segCount,
+                                                   const uint32_t* __restrict__ segBase, uint4* __restrict__ rec,
+                                                   uint32_t* __restrict__ grpV, uint32_t* __restrict__ grpQ,
+                                                   VolStat* __restrict__ vstat, unsigned long long* __restrict__ cpart,
+                                                   uint32_t acap) {
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t wpb = kBlock / kWave;
     // one volume: its contour count is spread over kContourParts counters
@@ -414,9 +486,9 @@ __global__ void __launch_bounds__(kBlock) k_rows(VolTable vt, int64_t Rtot, cons
     };
     unsigned long long total = 0;
     int cur = -1;  // volume whose contour count `total` holds (wave-uniform)
-    for (int64_t g = (int64_t)blockIdx.x * wpb + __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave); g < Rtot;
+    for (int64_t g = (int64_t)blockIdx.x * wpb + __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave); g < groups;
          g += (int64_t)gridDim.x * wpb) {
-        const int v = vol_of(vt.rowBase, vt.n, g);
+        const int v = vol_of(vt.grpBase, vt.n, g);
         if (v != cur) {
             total = wave_sum(total);
             if (lane == 0 && total) atomicAdd(contours(cur), total);
@@ -424,94 +496,52 @@ __global__ void __launch_bounds__(kBlock) k_rows(VolTable vt, int64_t Rtot, cons
             cur = v;
         }
         const VolDesc& V = vt.desc[v];
-        const GPtr<T> field = gfield<T>(V.field);
         const Dims d = V.d;
-        const double iso = V.iso;
-        const int S = V.S;
-        const int64_t r = g - V.rowBase;
-        const int j = (int)(r % (d.ny - 1));
-        const int k = (int)(r / (d.ny - 1));
-        uint32_t cv = 0, cq = 0;
-        // the row's active cells are contiguous in the flat order: process
-        // them 64 at a time across segment boundaries
-        const int64_t rs0 = V.rsBase + r * S;
-        // the row's segment bases, one per lane (rows of at most 64 segments;
-        // wider rows search memory)
-        const bool regs = S <= kWave;
-        const uint32_t mybase = (regs && lane < S) ? segBase[rs0 + lane] : 0u;
-        const uint32_t first = regs ? (uint32_t)__builtin_amdgcn_readfirstlane((int)mybase) : segBase[rs0];
-        const uint32_t last = segBase[rs0 + S - 1] + segCount[rs0 + S - 1];
-        for (uint32_t a0 = first; a0 < last; a0 += kWave) {
-            const uint32_t a = a0 + lane;
-            const bool act = a < last;
-            // segment of a: the last s with segBase[rs0 + s] <= a
-            int seg = 0;
-            uint32_t sbase = first;
-            if (regs) {
-                for (int s2 = 1; s2 < S; s2++) {
-                    const uint32_t b = (uint32_t)__shfl((int)mybase, s2, kWave);
-                    if (b <= a) {
-                        seg = s2;
-                        sbase = b;
-                    }
-                }
-            }
-            uint32_t nv = 0, nq = 0, code = 0, aux = 0;
-            int i = 0;
-            if (act) {
-                if (!regs) {
-                    int lo = 0, hi = S - 1;
-                    while (lo < hi) {
-                        const int mid = (lo + hi + 1) >> 1;
-                        if (segBase[rs0 + mid] <= a) lo = mid;
-                        else hi = mid - 1;
-                    }
-                    seg = lo;
-                    sbase = segBase[rs0 + lo];
-                }
-                const uint32_t x = lists[(rs0 + seg) * kSeg + (a - sbase)];
-                i = (int)(x & 0xFFFFFFu);
-                const unsigned icase = x >> 24;
-                uint64_t w;
+        const GroupLanes L = load_group(V, g, lane, segCount, segBase);
+        uint32_t cvq = 0;   // vertices | quadrilaterals << 16 of the cells before
+        for (uint32_t x0 = 0; x0 < L.total; x0 += kWave) {
+            const uint32_t x = x0 + lane;
+            const int s = group_seg(L, x);
+            const uint32_t rel = (uint32_t)__shfl((int)L.rel, s, kWave);
+            const int j = __shfl(L.j, s, kWave), k = __shfl(L.k, s, kWave);
+            uint32_t nvq = 0, code = 0, aux = 0, cell = 0, bits = 0;
+            if (x < L.total) {
+                const uint32_t e = lists[((g << V.gsh) + s) * kSeg + (x - rel)];
+                const int i = (int)(e & 0xFFFFFFu);
+                const unsigned icase = e >> 24;
+                unsigned dec = 0;
+                uint32_t m;
                 if (case_ambiguous(icase)) {
                     double F[8];
-                    load_corners<T>(field, d, i, j, k, F);
-                    w = polygons_decider(iso, F);
+                    load_corners<T>(gfield<T>(V.field), d, i, j, k, F);
+                    dec = case_decisions(icase, V.iso, F);
+                    if (undecided(dec)) m = ContourTable::map_of(chained_contours(icase, dec));
+                    else m = c_contours.map[c_contours.start[icase] + dec];
                 } else {
-                    w = c_case_contours[icase];
+                    m = c_contours.map[c_contours.start[icase]];
                 }
-                uint32_t map = 0;
-                int pos = 0;
-#pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    const int sz = poly_size(w, t);
-                    for (int q = 0; q < sz; q++) map |= (uint32_t)t << (2 * poly_edge_at(w, pos + q));
-                    pos += sz;
-                }
-                total += (unsigned long long)poly_count(w);
+                const uint32_t map = m & 0xFFFFFFu;
+                total += (unsigned long long)(m >> 24);
                 aux = cell_aux(icase, map, i, j, k, d);
-                nv = (uint32_t)__popc(aux >> 24);
-                nq = (uint32_t)(edge_cut(icase, 0) && j >= 1 && k >= 1) +
-                     (uint32_t)(edge_cut(icase, 3) && i >= 1 && k >= 1) +
-                     (uint32_t)(edge_cut(icase, 8) && i >= 1 && j >= 1);
+                nvq = (uint32_t)__popc(aux >> 24) |
+                      ((uint32_t)(edge_cut(icase, 0) && j >= 1 && k >= 1) +
+                       (uint32_t)(edge_cut(icase, 3) && i >= 1 && k >= 1) +
+                       (uint32_t)(edge_cut(icase, 8) && i >= 1 && j >= 1)) << 16;
                 code = icase | (map << 8);
+                bits = undecided(dec) ? 0x8000u : dec >> 4 << 30;
+                if (!undecided(dec)) aux |= dec << 28;
+                cell = ((uint32_t)k * (uint32_t)(d.ny - 1) + (uint32_t)j) * (uint32_t)d.C + (uint32_t)i;
             }
-            const uint32_t iv = wave_inclusive_scan(nv), iq = wave_inclusive_scan(nq);
+            const uint32_t inc = wave_inclusive_scan(nvq);
             // the counts are exact whatever the capacity; entries past it are
             // left out (the pass is then run again with room for them)
-            if (act && a < acap) {
-                acell[a] = (uint32_t)(r * d.C) + (uint32_t)i;
-                acode[a] = code;
-                aaux[a] = aux;
-                avloc[a] = cv + iv - nv;
-                aqloc[a] = cq + iq - nq;
-            }
-            cv += (uint32_t)__shfl((int)iv, kWave - 1, kWave);
-            cq += (uint32_t)__shfl((int)iq, kWave - 1, kWave);
+            const uint32_t a = L.first + x;
+            if (x < L.total && a < acap) rec[a] = make_uint4(cell, code, aux, (cvq + inc - nvq) | bits);
+            cvq += (uint32_t)__builtin_amdgcn_readlane((int)inc, kWave - 1);
         }
         if (lane == 0) {
-            rowV[g] = cv;
-            rowQ[g] = cq;
+            grpV[g] = cvq & 0xFFFFu;
+            grpQ[g] = cvq >> 16;
         }
     }
     total = wave_sum(total);
@@ -521,22 +551,29 @@ __global__ void __launch_bounds__(kBlock) k_rows(VolTable vt, int64_t Rtot, cons
 // ---------------------------------------------------------------------------
 // K3: vertices (cpp_dmc/DualMarchingCubes.cpp:141-171, UniformGrid.h:286-305).
 // One thread per active cell; position, normal and count of interior cut
-// edges of the vertices of used contours are written from
-// rowBaseV[row] + avloc[a] on.  Cells that need the general sampling (a
+// edges of the vertices of used contours are written from the cell's first
+// vertex (first_vertex) on.  Cells that need the general sampling (a
 // contour whose samples must avoid another contour's box, or a 9 x 9
 // sampling that finds no point) are appended to `slow` (slow[0] = count,
 // entries from slow[1]) and finished by k_vertices_slow, which also counts
 // the failed projections: only those cells can have any.
 // ---------------------------------------------------------------------------
+// Group of cell (i, j, k)'s (row, segment), r its cell row.
+__device__ __forceinline__ int64_t cell_group(const VolDesc& V, uint32_t r, int i) {
+    return (V.rsBase + (int64_t)r * V.S + i / kSeg) >> V.gsh;
+}
+__device__ __forceinline__ uint32_t first_vertex(const VolDesc& V, uint32_t r, int i, const ActRec& R,
+                                                 const uint32_t* __restrict__ grpV) {
+    return grpV[cell_group(V, r, i)] + R.vloc();
+}
+
+// Cell (i, j, k) in row r of an active cell, its corner values in F and in LDS.
 template <class T>
-__device__ __forceinline__ uint64_t cell_corners(const VolDesc& V, uint32_t cellword, uint32_t code,
-                                                 const CornerRef& Fc, int& i, int& j, int& k, uint32_t& r) {
-    const GPtr<T> field = gfield<T>(V.field);
+__device__ __forceinline__ void cell_corners(const VolDesc& V, uint32_t cellword, const CornerRef& Fc, double F[8],
+                                             int& i, int& j, int& k, uint32_t& r) {
     cell_ijk(cellword, V.d, i, j, k, r);
-    double F[8];
-    load_corners<T>(field, V.d, i, j, k, F);
+    load_corners<T>(gfield<T>(V.field), V.d, i, j, k, F);
     Fc.store(F);
-    return cell_polygons(code & 0xFFu, V.iso, F);
 }
 
 // The 24 field values one step beyond cell (i, j, k) along each axis that
@@ -655,10 +692,8 @@ __device__ __forceinline__ void store_vertex(const VolDesc& V, int i, int j, int
 }
 
 template <class T, int kUnroll>
-__device__ __forceinline__ void vertices_run(const VolTable& vt, const uint32_t* __restrict__ acell,
-                                             const uint32_t* __restrict__ acode, const uint32_t* __restrict__ aaux,
-                                             const uint32_t* __restrict__ avloc,
-                                             const uint32_t* __restrict__ rowBaseV, DevN dA,
+__device__ __forceinline__ void vertices_run(const VolTable& vt, const uint4* __restrict__ rec,
+                                             const uint32_t* __restrict__ grpV, DevN dA,
                                              double* __restrict__ vpos, double* __restrict__ vnrm,
                                              uint32_t* __restrict__ vdeg, uint32_t* __restrict__ slow,
                                              unsigned long long* qhead) {
@@ -691,20 +726,23 @@ __device__ __forceinline__ void vertices_run(const VolTable& vt, const uint32_t*
         const int vol = vol_of(vt.aBase, vt.n, a);
         const VolDesc& V = vt.desc[vol];
         const double iso = V.iso;
-        const uint32_t code = acode[a];
+        const ActRec R = load_rec(rec, a);
+        const uint32_t code = R.code;
         int i, j, k;
         uint32_t r;
-        const uint64_t w = cell_corners<T>(V, acell[a], code, Fc, i, j, k, r);
+        double F[8];
+        cell_corners<T>(V, R.cell, Fc, F, i, j, k, r);
+        const uint64_t w = R.contours();
         const int cnt = poly_count(w);
-        bool defer = cell_needs_box_test(w, cnt);
+        bool defer = R.undecided() || cell_needs_box_test(w, cnt);
         if (!defer) {
             // issued before the sampling, which hides their latency
             OuterValues<T> o;
             if (!V.grads) load_outer<T>(V, i, j, k, o);
             cell_boxes(Fc, iso, w, cnt, B);
-            const uint32_t aux = aaux[a];
-            const unsigned used = aux >> 24;
-            uint32_t out = rowBaseV[V.rowBase + r] + avloc[a];
+            const uint32_t aux = R.aux;
+            const unsigned used = R.used();
+            uint32_t out = first_vertex(V, r, i, R, grpV);
             for (int t = 0; t < cnt; t++) {
                 double p[3];
                 if (!contour_representative9<kUnroll>(Fc, iso, w, t, B, p)) {
@@ -734,15 +772,12 @@ __device__ __forceinline__ void vertices_run(const VolTable& vt, const uint32_t*
 // active cell: a row's samples interleaved (the latency of one cell matters
 // most), 2 waves per SIMD.
 template <class T>
-__global__ void __launch_bounds__(kBlock) TMC_VERTICES_ATTR k_vertices(VolTable vt, const uint32_t* __restrict__ acell,
-                                                      const uint32_t* __restrict__ acode,
-                                                      const uint32_t* __restrict__ aaux,
-                                                      const uint32_t* __restrict__ avloc,
-                                                      const uint32_t* __restrict__ rowBaseV, DevN dA,
+__global__ void __launch_bounds__(kBlock) TMC_VERTICES_ATTR k_vertices(VolTable vt, const uint4* __restrict__ rec,
+                                                      const uint32_t* __restrict__ grpV, DevN dA,
                                                       double* __restrict__ vpos, double* __restrict__ vnrm,
                                                       uint32_t* __restrict__ vdeg, uint32_t* __restrict__ slow,
                                                       unsigned long long* qhead) {
-    vertices_run<T, 7>(vt, acell, acode, aaux, avloc, rowBaseV, dA, vpos, vnrm, vdeg, slow, qhead);
+    vertices_run<T, 7>(vt, rec, grpV, dA, vpos, vnrm, vdeg, slow, qhead);
 }
 
 // K3 for larger passes: samples one at a time, which fits 3 waves per SIMD
@@ -752,23 +787,18 @@ __global__ void __launch_bounds__(kBlock) TMC_VERTICES_ATTR k_vertices(VolTable 
 // arithmetic in the same order as k_vertices.
 template <class T>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 3)))
-k_vertices_wide(VolTable vt, const uint32_t* __restrict__ acell, const uint32_t* __restrict__ acode,
-                const uint32_t* __restrict__ aaux, const uint32_t* __restrict__ avloc,
-                const uint32_t* __restrict__ rowBaseV, DevN dA, double* __restrict__ vpos,
-                double* __restrict__ vnrm, uint32_t* __restrict__ vdeg, uint32_t* __restrict__ slow,
+k_vertices_wide(VolTable vt, const uint4* __restrict__ rec, const uint32_t* __restrict__ grpV, DevN dA,
+                double* __restrict__ vpos, double* __restrict__ vnrm, uint32_t* __restrict__ vdeg, uint32_t* __restrict__ slow,
                 unsigned long long* qhead) {
-    vertices_run<T, 1>(vt, acell, acode, aaux, avloc, rowBaseV, dA, vpos, vnrm, vdeg, slow, qhead);
+    vertices_run<T, 1>(vt, rec, grpV, dA, vpos, vnrm, vdeg, slow, qhead);
 }
 
 // General path of K3 for the cells k_vertices deferred: every contour is
 // sampled with the box test at 9 x 9 and, where that finds no point, at
 // 28 x 28; failed projections are counted per volume.
 template <class T>
-__global__ void __launch_bounds__(kBlock) k_vertices_slow(VolTable vt, const uint32_t* __restrict__ acell,
-                                                          const uint32_t* __restrict__ acode,
-                                                          const uint32_t* __restrict__ aaux,
-                                                          const uint32_t* __restrict__ avloc,
-                                                          const uint32_t* __restrict__ rowBaseV,
+__global__ void __launch_bounds__(kBlock) k_vertices_slow(VolTable vt, const uint4* __restrict__ rec,
+                                                          const uint32_t* __restrict__ grpV,
                                                           const uint32_t* __restrict__ slow,
                                                           double* __restrict__ vpos, double* __restrict__ vnrm,
                                                           uint32_t* __restrict__ vdeg, VolStat* __restrict__ vstat) {
@@ -782,17 +812,20 @@ __global__ void __launch_bounds__(kBlock) k_vertices_slow(VolTable vt, const uin
         const int vol = vol_of(vt.aBase, vt.n, a);
         const VolDesc& V = vt.desc[vol];
         const double iso = V.iso;
-        const uint32_t code = acode[a];
+        const ActRec R = load_rec(rec, a);
+        const uint32_t code = R.code;
         int i, j, k;
         uint32_t r;
-        const uint64_t w = cell_corners<T>(V, acell[a], code, Fc, i, j, k, r);
+        double F[8];
+        cell_corners<T>(V, R.cell, Fc, F, i, j, k, r);
+        const uint64_t w = R.undecided() ? chained_contours(code & 0xFFu, case_decisions(code & 0xFFu, iso, F)) : R.contours();
         const int cnt = poly_count(w);
         OuterValues<T> o;
         if (!V.grads) load_outer<T>(V, i, j, k, o);
         cell_boxes(Fc, iso, w, cnt, B);
-        const uint32_t aux = aaux[a];
-        const unsigned used = aux >> 24;
-        uint32_t out = rowBaseV[V.rowBase + r] + avloc[a];
+        const uint32_t aux = R.aux;
+        const unsigned used = R.used();
+        uint32_t out = first_vertex(V, r, i, R, grpV);
         for (int t = 0; t < cnt; t++) {
             double p[3];
             const int fl = contour_representative(Fc, iso, w, cnt, t, B, p);
@@ -843,24 +876,18 @@ __device__ __forceinline__ int64_t find_active(const SegLists& L, const Dims& d,
     return (int64_t)L.base[rs] + rank;
 }
 
-// Final id of the vertex of active cell `a` whose contour contains edge e,
-// and the row of edge e among that contour's interior edges (its slot in the
-// first halfedge CSR).  rowBase points at the volume's first row; r is the
-// cell's row in the volume.
-__device__ __forceinline__ int32_t vertex_slot_of(const uint32_t* __restrict__ acode,
-                                                  const uint32_t* __restrict__ aaux,
-                                                  const uint32_t* __restrict__ avloc,
-                                                  const uint32_t* __restrict__ rowBaseV, int64_t a, int e,
-                                                  int64_t r, int& slot) {
+// Final id of the vertex of active cell `a` (cell (i, ., .) of cell row r)
+// whose contour contains edge e, and the row of edge e among that contour's
+// interior edges (its slot in the first halfedge CSR).
+__device__ __forceinline__ int32_t vertex_slot_of(const uint4* __restrict__ rec, const uint32_t* __restrict__ grpV,
+                                                  const VolDesc& V, int64_t a, int e, int64_t r, int i, int& slot) {
     slot = 0;
     if (a < 0) return -1;
-    const uint32_t code = acode[a], aux = aaux[a];
-    const unsigned icase = code & 0xFFu;
-    const uint32_t map = code >> 8;
+    const ActRec R = load_rec(rec, a);
+    const uint32_t map = R.code >> 8;
     const unsigned t = (map >> (2 * e)) & 3u;
-    slot = contour_rank(map, aux, icase, t, e);
-    const uint32_t vb = rowBaseV[r] + avloc[a];
-    return (int32_t)(vb + __popc((aux >> 24) & ((1u << t) - 1u)));
+    slot = contour_rank(map, R.aux, R.code & 0xFFu, t, e);
+    return (int32_t)(first_vertex(V, (uint32_t)r, i, R, grpV) + __popc(R.used() & ((1u << t) - 1u)));
 }
 
 // ---------------------------------------------------------------------------
@@ -870,13 +897,9 @@ __device__ __forceinline__ int32_t vertex_slot_of(const uint32_t* __restrict__ a
 // (cpp_dmc/DualMarchingCubes.h:215-223, :663-676).  Colour: 3*parity + dir
 // (cpp_dmc/DualMarchingCubes.cpp:180-183).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(kBlock) k_quads(VolTable vt, const uint32_t* __restrict__ acell,
-                                                   const uint32_t* __restrict__ acode,
-                                                   const uint32_t* __restrict__ aaux,
-                                                   const uint32_t* __restrict__ avloc,
-                                                   const uint32_t* __restrict__ aqloc,
-                                                   const uint32_t* __restrict__ rowBaseV0,
-                                                   const uint32_t* __restrict__ rowBaseQ, DevN dA,
+__global__ void __launch_bounds__(kBlock) k_quads(VolTable vt, const uint4* __restrict__ rec,
+                                                   const uint32_t* __restrict__ grpV,
+                                                   const uint32_t* __restrict__ grpQ, DevN dA,
                                                    const unsigned long long* __restrict__ segMask,
                                                    const uint32_t* __restrict__ segBase,
                                                    int32_t* __restrict__ quads, uint8_t* __restrict__ colors,
@@ -888,22 +911,22 @@ __global__ void __launch_bounds__(kBlock) k_quads(VolTable vt, const uint32_t* _
         const VolDesc& V = vt.desc[vol];
         const Dims d = V.d;
         const SegLists L{segMask, segBase, V.S, V.rsBase};
-        const uint32_t* __restrict__ rowBaseV = rowBaseV0 + V.rowBase;
+        const ActRec R = load_rec(rec, a);
         int i, j, k;
         uint32_t r;
-        cell_ijk(acell[a], d, i, j, k, r);
-        const unsigned icase = acode[a] & 0xFFu;
+        cell_ijk(R.cell, d, i, j, k, r);
+        const unsigned icase = R.code & 0xFFu;
         const int bit = (icase & 1u) ? 0 : 1;     // field at the edge origin below iso
         const int parity = (i & 1) | (j & 1) << 1 | (k & 1) << 2;
-        int64_t q = (int64_t)rowBaseQ[V.rowBase + r] + aqloc[a];
+        int64_t q = (int64_t)grpQ[cell_group(V, r, i)] + R.qloc();
         const bool ex = edge_cut(icase, 0) && j >= 1 && k >= 1;
         const bool ey = edge_cut(icase, 3) && i >= 1 && k >= 1;
         const bool ez = edge_cut(icase, 8) && i >= 1 && j >= 1;
         if (!(ex || ey || ez)) continue;
         int s0, s3, s8;
-        const int32_t own0 = vertex_slot_of(acode, aaux, avloc, rowBaseV, a, 0, r, s0);
-        const int32_t own3 = vertex_slot_of(acode, aaux, avloc, rowBaseV, a, 3, r, s3);
-        const int32_t own8 = vertex_slot_of(acode, aaux, avloc, rowBaseV, a, 8, r, s8);
+        const int32_t own0 = vertex_slot_of(rec, grpV, V, a, 0, r, i, s0);
+        const int32_t own3 = vertex_slot_of(rec, grpV, V, a, 3, r, i, s3);
+        const int32_t own8 = vertex_slot_of(rec, grpV, V, a, 8, r, i, s8);
         // rows of the cells (., j-1, k) and (., j, k-1)
         const int64_t rj = (int64_t)r - 1, rk = (int64_t)r - (d.ny - 1);
         // cells of the previous row (j-1) and plane (k-1) found once
@@ -933,9 +956,9 @@ __global__ void __launch_bounds__(kBlock) k_quads(VolTable vt, const uint32_t* _
             const int64_t e = find_active(L, d, i, j - 1, k - 1);
             out[edge_slot(0, bit)] = own0;
             sl[edge_slot(0, bit)] = s0;
-            out[edge_slot(2, bit)] = vertex_slot_of(acode, aaux, avloc, rowBaseV, cjm, 2, rj, sl[edge_slot(2, bit)]);
-            out[edge_slot(4, bit)] = vertex_slot_of(acode, aaux, avloc, rowBaseV, ckm, 4, rk, sl[edge_slot(4, bit)]);
-            out[edge_slot(6, bit)] = vertex_slot_of(acode, aaux, avloc, rowBaseV, e, 6, rk - 1, sl[edge_slot(6, bit)]);
+            out[edge_slot(2, bit)] = vertex_slot_of(rec, grpV, V, cjm, 2, rj, i, sl[edge_slot(2, bit)]);
+            out[edge_slot(4, bit)] = vertex_slot_of(rec, grpV, V, ckm, 4, rk, i, sl[edge_slot(4, bit)]);
+            out[edge_slot(6, bit)] = vertex_slot_of(rec, grpV, V, e, 6, rk - 1, i, sl[edge_slot(6, bit)]);
             emit(0);
         }
         // y edge: cells (i,j,k) e3, (i-1,j,k) e1, (i,j,k-1) e7, (i-1,j,k-1) e5
@@ -943,9 +966,9 @@ __global__ void __launch_bounds__(kBlock) k_quads(VolTable vt, const uint32_t* _
             const int64_t e = ckm > 0 ? ckm - 1 : -1;
             out[edge_slot(3, bit)] = own3;
             sl[edge_slot(3, bit)] = s3;
-            out[edge_slot(1, bit)] = vertex_slot_of(acode, aaux, avloc, rowBaseV, a - 1, 1, r, sl[edge_slot(1, bit)]);
-            out[edge_slot(7, bit)] = vertex_slot_of(acode, aaux, avloc, rowBaseV, ckm, 7, rk, sl[edge_slot(7, bit)]);
-            out[edge_slot(5, bit)] = vertex_slot_of(acode, aaux, avloc, rowBaseV, e, 5, rk, sl[edge_slot(5, bit)]);
+            out[edge_slot(1, bit)] = vertex_slot_of(rec, grpV, V, a - 1, 1, r, i - 1, sl[edge_slot(1, bit)]);
+            out[edge_slot(7, bit)] = vertex_slot_of(rec, grpV, V, ckm, 7, rk, i, sl[edge_slot(7, bit)]);
+            out[edge_slot(5, bit)] = vertex_slot_of(rec, grpV, V, e, 5, rk, i - 1, sl[edge_slot(5, bit)]);
             emit(1);
         }
         // z edge: cells (i,j,k) e8, (i-1,j,k) e9, (i,j-1,k) e11, (i-1,j-1,k) e10
@@ -953,9 +976,9 @@ __global__ void __launch_bounds__(kBlock) k_quads(VolTable vt, const uint32_t* _
             const int64_t e = cjm > 0 ? cjm - 1 : -1;
             out[edge_slot(8, bit)] = own8;
             sl[edge_slot(8, bit)] = s8;
-            out[edge_slot(9, bit)] = vertex_slot_of(acode, aaux, avloc, rowBaseV, a - 1, 9, r, sl[edge_slot(9, bit)]);
-            out[edge_slot(11, bit)] = vertex_slot_of(acode, aaux, avloc, rowBaseV, cjm, 11, rj, sl[edge_slot(11, bit)]);
-            out[edge_slot(10, bit)] = vertex_slot_of(acode, aaux, avloc, rowBaseV, e, 10, rj, sl[edge_slot(10, bit)]);
+            out[edge_slot(9, bit)] = vertex_slot_of(rec, grpV, V, a - 1, 9, r, i - 1, sl[edge_slot(9, bit)]);
+            out[edge_slot(11, bit)] = vertex_slot_of(rec, grpV, V, cjm, 11, rj, i, sl[edge_slot(11, bit)]);
+            out[edge_slot(10, bit)] = vertex_slot_of(rec, grpV, V, e, 10, rj, i - 1, sl[edge_slot(10, bit)]);
             emit(2);
         }
     }
@@ -989,11 +1012,11 @@ __global__ void k_cell_guard(Sizes* S, uint64_t acap, uint64_t vcap, uint64_t qc
 
 // Each volume's first vertex and quadrilateral: [0, n] the live bounds,
 // [n+1, 2n+1] the cell stage's (kept for the per-volume counts).
-__global__ void k_vol_bounds(VolTable vt, const uint32_t* __restrict__ rowBaseV, const uint32_t* __restrict__ rowBaseQ,
+__global__ void k_vol_bounds(VolTable vt, const uint32_t* __restrict__ grpV, const uint32_t* __restrict__ grpQ,
                              const Sizes* S, int64_t* __restrict__ vb, int64_t* __restrict__ qb) {
     for (int v = blockIdx.x * blockDim.x + threadIdx.x; v <= vt.n; v += gridDim.x * blockDim.x) {
-        const int64_t x = v < vt.n ? (int64_t)rowBaseV[vt.desc[v].rowBase] : (int64_t)S->V;
-        const int64_t y = v < vt.n ? (int64_t)rowBaseQ[vt.desc[v].rowBase] : (int64_t)S->Q;
+        const int64_t x = v < vt.n ? (int64_t)grpV[vt.desc[v].rsBase >> vt.desc[v].gsh] : (int64_t)S->V;
+        const int64_t y = v < vt.n ? (int64_t)grpQ[vt.desc[v].rsBase >> vt.desc[v].gsh] : (int64_t)S->Q;
         vb[v] = x;
         qb[v] = y;
         vb[vt.n + 1 + v] = x;

@@ -5,11 +5,11 @@
 // The active cells come from the DMC sweep (same classification, f >= iso,
 // same per-(row, segment) lists, whose flat order is the reference's
 // (k, j, i) cell order).  Then:
-//   k_tmc_cells      one wave per row: each active cell's case, new vertices
+//   k_tmc_cells      each active cell's case, new vertices
 //                    (the cut edges it owns) and table triangles; the
 //                    ambiguous cells listed;
 //   k_tmc_amb_count  the listed cells' inner vertices and triangles from the
-//                    decider slicing (kept out of the row walk, where one
+//                    decider slicing (kept out of the cell walk, where one
 //                    ambiguous lane would hold up its wave);
 //   scans            over the active cells: each cell's first vertex and
 //                    triangle -- the reference's numbering, first sight in
@@ -439,13 +439,13 @@ __device__ __forceinline__ void tmc_corners(const T* __restrict__ field, const D
     for (int c = 0; c < 8; c++) F[c] = (double)p[(c & 1) + ((c >> 1) & 1) * sy + (c >> 2) * sz];
 }
 
-// K_T1: one wave per row, cells in ascending x (the flat active order):
-// per active cell its cell word, case (acode), new vertices (cnt_v: the cut
-// edges it owns) and triangles (cnt_t: the case table's); the ambiguous
-// cells are listed (amb[0] = count, from amb[1]) for k_tmc_amb_count, which
-// adds their inner vertices and sets their triangles.  stats[0] counts
-// them.
-__global__ void __launch_bounds__(kBlock) k_tmc_cells(VolTable vt, int64_t Rtot, const uint32_t* __restrict__ lists,
+// K_T1: one wave per group of (row, segment)s as in k_cells, cells in the
+// flat active order: per active cell its cell word, case (acode), new
+// vertices (cnt_v: the cut edges it owns) and triangles (cnt_t: the case
+// table's); the ambiguous cells are listed (amb[0] = count, from amb[1]) for
+// k_tmc_amb_count, which adds their inner vertices and sets their triangles.
+// stats[0] counts them.
+__global__ void __launch_bounds__(kBlock) k_tmc_cells(VolTable vt, int64_t groups, const uint32_t* __restrict__ lists,
                                                        const uint32_t* __restrict__ segCount,
                                                        const uint32_t* __restrict__ segBase,
                                                        uint32_t* __restrict__ acell, uint32_t* __restrict__ acode,
@@ -455,54 +455,24 @@ __global__ void __launch_bounds__(kBlock) k_tmc_cells(VolTable vt, int64_t Rtot,
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t wpb = kBlock / kWave;
     unsigned long long namb = 0;
-    for (int64_t g = (int64_t)blockIdx.x * wpb + __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave); g < Rtot;
+    for (int64_t g = (int64_t)blockIdx.x * wpb + __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave); g < groups;
          g += (int64_t)gridDim.x * wpb) {
-        const int v = vol_of(vt.rowBase, vt.n, g);
-        const VolDesc& V = vt.desc[v];
+        const VolDesc& V = vt.desc[vol_of(vt.grpBase, vt.n, g)];
         const Dims d = V.d;
-        const int S = V.S;
-        const int64_t r = g - V.rowBase;
-        const int j = (int)(r % (d.ny - 1));
-        const int k = (int)(r / (d.ny - 1));
-        const int64_t rs0 = V.rsBase + r * S;
-        // the row's segment bases, one per lane (rows of at most 64
-        // segments; wider rows search memory)
-        const bool regs = S <= kWave;
-        const uint32_t mybase = (regs && lane < S) ? segBase[rs0 + lane] : 0u;
-        const uint32_t first = regs ? (uint32_t)__builtin_amdgcn_readfirstlane((int)mybase) : segBase[rs0];
-        const uint32_t last = segBase[rs0 + S - 1] + segCount[rs0 + S - 1];
-        for (uint32_t a0 = first; a0 < last; a0 += kWave) {
-            const uint32_t a = a0 + lane;
-            const bool act = a < last;
-            int seg = 0;
-            uint32_t sbase = first;
-            if (regs) {
-                for (int s2 = 1; s2 < S; s2++) {
-                    const uint32_t b = (uint32_t)__shfl((int)mybase, s2, kWave);
-                    if (b <= a) {
-                        seg = s2;
-                        sbase = b;
-                    }
-                }
-            }
+        const GroupLanes L = load_group(V, g, lane, segCount, segBase);
+        for (uint32_t x0 = 0; x0 < L.total; x0 += kWave) {
+            const uint32_t x = x0 + lane, a = L.first + x;
+            const int s = group_seg(L, x);
+            const uint32_t rel = (uint32_t)__shfl((int)L.rel, s, kWave);
+            const int j = __shfl(L.j, s, kWave), k = __shfl(L.k, s, kWave);
             bool isamb = false;
-            if (act) {
-                if (!regs) {
-                    int lo = 0, hi = S - 1;
-                    while (lo < hi) {
-                        const int mid = (lo + hi + 1) >> 1;
-                        if (segBase[rs0 + mid] <= a) lo = mid;
-                        else hi = mid - 1;
-                    }
-                    seg = lo;
-                    sbase = segBase[rs0 + lo];
-                }
-                const uint32_t x = lists[(rs0 + seg) * kSeg + (a - sbase)];
-                const int i = (int)(x & 0xFFFFFFu);
-                const unsigned icase = x >> 24;
+            if (x < L.total) {
+                const uint32_t e = lists[((g << V.gsh) + s) * kSeg + (x - rel)];
+                const int i = (int)(e & 0xFFFFFFu);
+                const unsigned icase = e >> 24;
                 isamb = tmc_ambiguous(icase);
                 namb += isamb;
-                acell[a] = (uint32_t)(r * d.C) + (uint32_t)i;
+                acell[a] = ((uint32_t)k * (uint32_t)(d.ny - 1) + (uint32_t)j) * (uint32_t)d.C + (uint32_t)i;
                 acode[a] = icase;
                 cnt_v[a] = (uint32_t)__popc(tmc_cut_mask(icase) & tmc_owned_mask(i, j, k, d));
                 cnt_t[a] = isamb ? 0u : (uint32_t)(c_tmc_tri[icase] >> 60);
