@@ -25,6 +25,7 @@
 #include "../../include/tmc_dmc.h"
 #include "dmc_extract_kernels.h"
 #include "dmc_mesh_kernels.h"
+#include "dmc_quad_kernels.h"
 #include "tmc_kernels.h"
 
 using namespace tmc;
@@ -116,8 +117,8 @@ struct dmc_context {
     int pcur = 0;  // which positions/normals buffer holds the vertex data
     int scur = 0;  // which slot map is live ...
     bool slots = false;  // ... once a compaction has run (else slots are the identity)
-    // what the next halfedge build starts from: 1 the cell stage's rows in
-    // off/adj, 2 the build a compaction carried over, 0 nothing
+    // what the next halfedge build starts from: 1 the cell stage's build, 2 the
+    // build a compaction carried over, 0 nothing
     int ready = 0;
     bool rows_live = false;   // off/adj hold the rows of the last extraction's final mesh
     bool force_generic = false;   // this extraction's passes pair every build through generic rows
@@ -748,8 +749,10 @@ void plan_caps(dmc_context* ctx, const std::vector<HostVol>& hv, int64_t cells) 
     ctx->reccap = std::max<int64_t>(ctx->reccap, 1024);
 }
 
+// final_build: no simplification follows, the cell stage's halfedges are the
+// final mesh's.
 template <class T>
-void run_cells(dmc_context* ctx, const SweepPlan& P) {
+void run_cells(dmc_context* ctx, const SweepPlan& P, bool final_build) {
     // canonical buffer roles at the start of every pass, so that a pass of
     // the same shape launches on the same pointers (and can be replayed)
     set_pair_order(ctx, 0);
@@ -765,7 +768,8 @@ void run_cells(dmc_context* ctx, const SweepPlan& P) {
     uint32_t* grpV = ensure<uint32_t>(ctx, ctx->grpV, G);
     uint32_t* grpQ = ensure<uint32_t>(ctx, ctx->grpQ, G);
     launch(ctx, "k_cells", k_cells<T>, dim3(grid_for(ctx, G, kBlock / kWave)), dim3(kBlock), vt, G, sw.lists,
-           sw.segCount, sw.segBase, rec, grpNV, grpNQ, sw.vstat, S->cpart, (uint32_t)acap);
+           sw.segCount, sw.segBase, rec, grpNV, grpNQ, sw.vstat, S->cpart,
+           &S->open_cells, (uint32_t)acap);
     check_launch(ctx, "k_cells");
     scan_pair(ctx, scan_job(ScanCounts{grpNV}, grpV, hn(G), &S->V), scan_job(ScanCounts{grpNQ}, grpQ, hn(G), &S->Q),
               "k_scan_cells");
@@ -788,11 +792,24 @@ void run_cells(dmc_context* ctx, const SweepPlan& P) {
     double* nrm = ensure<double>(ctx, ctx->nrm[0], 3 * vcap);
     int32_t* quads = ensure<int32_t>(ctx, ctx->quads[0], 4 * qcap);
     uint8_t* colors = ensure<uint8_t>(ctx, ctx->colors, qcap);
-    // first halfedge CSR straight from the cells: degree of each vertex from
-    // k_vertices, rows filled by k_quads
+    // the first halfedge build straight from the cells: out-degree of each
+    // vertex from k_vertices, the rest from k_quads
     uint32_t* deg = ensure<uint32_t>(ctx, ctx->deg, vcap);
-    uint32_t* off = ensure<uint32_t>(ctx, ctx->off, vcap + 1);
-    int2* adj = ensure<int2>(ctx, ctx->adj, 4 * qcap);
+    uint32_t* arr = final_build ? nullptr : ensure<uint32_t>(ctx, ctx->arr, vcap);
+    QuadOut qo{};
+    qo.quads = quads;
+    qo.colors = colors;
+    qo.twin = ensure<int32_t>(ctx, ctx->twin, 4 * qcap);
+    qo.flag = ensure<uint8_t>(ctx, ctx->flag, 4 * qcap);
+    qo.hev = ensure<int32_t>(ctx, ctx->hev, vcap);
+    qo.arr = arr;
+    qo.recs = ensure<BndRec>(ctx, ctx->bndrec, ctx->reccap);
+    qo.reccap = (uint32_t)ctx->reccap;
+    qo.S = S;
+    if (final_build && n > 1) {
+        qo.vst = ensure<unsigned long long>(ctx, ctx->vhe, 3 * (size_t)n);
+        fill_u32(ctx, qo.vst, hn(6 * (int64_t)n), 0u);
+    }
     const DevN A = dn(&S->acnt, acap);
     mark(ctx, "vertices");
     // persistent: a few rounds of the blocks the chip holds at once; the
@@ -801,19 +818,17 @@ void run_cells(dmc_context* ctx, const SweepPlan& P) {
     const dim3 gv(grid_for(ctx, acap, kBlock, kVerticesBlocks));
     if (std::is_same<T, float>::value && acap > kVerticesBlocks * kBlock)
         launch(ctx, "k_vertices", k_vertices_wide<T>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, deg,
-               slow, &S->qhead);
+               arr, slow, &S->qhead);
     else
-        launch(ctx, "k_vertices", k_vertices<T>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, deg, slow,
-               &S->qhead);
+        launch(ctx, "k_vertices", k_vertices<T>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, deg, arr,
+               slow, &S->qhead);
     check_launch(ctx, "k_vertices");
     launch(ctx, "k_vertices_slow", k_vertices_slow<T>, dim3(grid_for(ctx, acap, kBlock, 1024)), dim3(kBlock), vt,
-           rec, grpV, slow, pos, nrm, deg, sw.vstat);
+           rec, grpV, slow, pos, nrm, deg, arr, sw.vstat);
     check_launch(ctx, "k_vertices_slow");
     mark(ctx, "quads");
-    // the row total must be 4 Q (checked with the pass's sizes at the end)
-    scan_to(ctx, ScanCounts{deg}, off, dn(&S->nv, vcap), &S->rows, "k_scan_cells", nullptr, off);
-    launch(ctx, "k_quads", k_quads, dim3(grid_for(ctx, acap)), dim3(kBlock), vt, rec, grpV, grpQ, A, sw.segMask, sw.segBase, quads, colors, off, adj, (uint64_t)(4 * qcap),
-           &S->unresolved);
+    launch(ctx, "k_quads", n > 1 ? k_quads<true> : k_quads<false>, dim3(grid_for(ctx, acap)), dim3(kBlock), vt, rec,
+           grpV, grpQ, A, sw.segMask, sw.segBase, qo, &S->unresolved);
     check_launch(ctx, "k_quads");
     ctx->ready = 1;
 }
@@ -823,18 +838,16 @@ void run_cells(dmc_context* ctx, const SweepPlan& P) {
 // ---------------------------------------------------------------------------
 // A halfedge build gives every halfedge its twin and flag, every vertex its
 // out-degree, valence and he_v, and lists the 3-face edges.  The first build
-// pairs through the rows of outgoing (halfedge, destination) pairs the cell
-// stage left (off/adj).  A compaction carries the build over to the mesh it
-// leaves: most groups keep their members, renumbered, and only halfedges at
-// a changed vertex are paired again.  If the device finds the rows or the
-// carry unusable (a quadrilateral with an unresolved neighbour cell, an
-// invalid vertex reference), the build counts generic rows from the
+// comes with the quadrilaterals (k_quads).  A compaction carries the build
+// over to the mesh it leaves: most groups keep their members, renumbered, and
+// only halfedges at a changed vertex are paired again.  If the device finds
+// either unusable (a quadrilateral with an unresolved neighbour cell, an
+// invalid vertex reference), the pass runs again and every build counts
+// generic rows of outgoing (halfedge, destination) pairs from the
 // quadrilaterals and pairs everything.
 
-// Pairing through full rows (on the device only when S->pair_rows): the
-// cell stage's rows, or (generic: launched only in a pass run again for
-// them) rows counted from the quadrilaterals.
-void pair_rows(dmc_context* ctx, bool final_pass, bool generic) {
+// Pairing through generic rows.
+void pair_rows(dmc_context* ctx, bool final_pass) {
     const int64_t vcap = ctx->vcap, qcap = ctx->qcap, hcap = 4 * qcap;
     Sizes* S = dsizes(ctx);
     const int32_t* quads = static_cast<const int32_t*>(ctx->quads[ctx->cur].p);
@@ -847,29 +860,24 @@ void pair_rows(dmc_context* ctx, bool final_pass, bool generic) {
     int32_t* hev = ensure<int32_t>(ctx, ctx->hev, vcap);
     uint32_t* arr = final_pass ? nullptr : ensure<uint32_t>(ctx, ctx->arr, vcap);
     BndRec* recs = ensure<BndRec>(ctx, ctx->bndrec, ctx->reccap);
-    const uint32_t* gen = &S->generic;
-    const uint32_t* rows = &S->pair_rows;
     const DevN nv = dn(&S->nv, vcap);
-    if (generic) {
-        Fills(ctx).u32(deg, nv, 0u, gen).u32(cursor, nv, 0u, gen).run();
-        launch(ctx, "k_he_degree", k_he_degree, dim3(grid_for(ctx, hcap)), dim3(kBlock), quads, (const Sizes*)S,
-               deg, &S->he.bad, gen);
-        scan_to(ctx, ScanCounts{deg}, off, nv, &S->tot, "k_scan", gen, off);
-        launch(ctx, "k_he_scatter", k_he_scatter, dim3(grid_for(ctx, qcap)), dim3(kBlock), quads, (const Sizes*)S,
-               off, cursor, adj, gen);
-    }
     Fills fl(ctx);
-    fl.u32(hev, nv, 0xFFFFFFFFu, rows);
-    if (arr) fl.u32(arr, nv, 0u, rows);
+    fl.u32(deg, nv, 0u).u32(cursor, nv, 0u).u32(hev, nv, 0xFFFFFFFFu);
+    if (arr) fl.u32(arr, nv, 0u);
     unsigned long long* vst = nullptr;
     if (final_pass && ctx->nvol > 1) {
         vst = ensure<unsigned long long>(ctx, ctx->vhe, 3 * (size_t)ctx->nvol);
-        fl.u32(vst, hn(6 * (int64_t)ctx->nvol), 0u, rows);
+        fl.u32(vst, hn(6 * (int64_t)ctx->nvol), 0u);
     }
     fl.run();
+    launch(ctx, "k_he_degree", k_he_degree, dim3(grid_for(ctx, hcap)), dim3(kBlock), quads, (const Sizes*)S, deg,
+           &S->he.bad);
+    scan_to(ctx, ScanCounts{deg}, off, nv, &S->tot, "k_scan", nullptr, off);
+    launch(ctx, "k_he_scatter", k_he_scatter, dim3(grid_for(ctx, qcap)), dim3(kBlock), quads, (const Sizes*)S, off,
+           cursor, adj);
     launch(ctx, "k_he_twins", k_he_twins, dim3(grid_for(ctx, hcap)), dim3(kBlock), quads, (const Sizes*)S, off, adj,
            twin, flag, hev, arr, S->hep, recs, &S->nrec, (uint32_t)ctx->reccap, &S->ovf,
-           static_cast<const int64_t*>(ctx->qbound.p), ctx->nvol, vst, rows);
+           static_cast<const int64_t*>(ctx->qbound.p), ctx->nvol, vst);
     check_launch(ctx, "k_he_twins");
 }
 
@@ -883,8 +891,7 @@ void build_halfedges(dmc_context* ctx, bool final_pass, const StageClears& clear
     launch(ctx, "k_rows_gate", k_rows_gate, dim3(1), dim3(64), S, ready, ctx->commit_pending ? 1 : 0);
     ctx->commit_pending = false;
     ctx->ready = 0;
-    // a carried build pairs nothing here
-    if (ready != 2) pair_rows(ctx, final_pass, ready == 0);
+    if (ready == 0) pair_rows(ctx, final_pass);
     const int gv = grid_for(ctx, vcap);
     if (!final_pass) {
         uint32_t* val = ensure<uint32_t>(ctx, ctx->val, vcap);
@@ -1368,8 +1375,9 @@ void run_tmc(dmc_context* ctx, const std::vector<HostVol>& hv) {
 void enqueue_pass(dmc_context* ctx, const SweepPlan& P, int field_type, uint32_t flags) {
     const int n = ctx->nvol;
     ctx->commit_pending = false;
-    if (field_type == DMC_FIELD_F32) run_cells<float>(ctx, P);
-    else run_cells<double>(ctx, P);
+    const bool final_build = (flags & DMC_SIMPLIFY_ALL) == 0;
+    if (field_type == DMC_FIELD_F32) run_cells<float>(ctx, P, final_build);
+    else run_cells<double>(ctx, P, final_build);
     const bool iso = (flags & DMC_SIMPLIFY_3X3Y_ISOLATED) != 0, p3333 = (flags & DMC_SIMPLIFY_3333) != 0;
     if (flags & DMC_SIMPLIFY_3X3Y_COLOR) {
         mark(ctx, "p3x3y_color");
@@ -1472,10 +1480,10 @@ bool finish_pass(dmc_context* ctx, const std::vector<HostVol>& hv, uint32_t flag
         if (hs.ovf & 8u) ctx->reccap = std::max<int64_t>(ctx->reccap, (int64_t)std::max(hs.nrec, hs.recmax));
         return false;
     }
-    ctx->rows_live = hs.pair_rows != 0u;
-    if (hs.rows != 4 * hs.Q)
-        fail(ctx, DMC_ERR_STATE, "halfedge rows %llu != 4 Q %llu", (unsigned long long)hs.rows,
-             (unsigned long long)(4 * hs.Q));
+    ctx->rows_live = ctx->force_generic;
+    if (hs.open_cells)
+        fail(ctx, DMC_ERR_STATE, "%u cells with a cut edge on no contour (the field is not a number there)",
+             hs.open_cells);
     // getBndVertices: the 3-face records, in key order
     ctx->bnd.clear();
     if (hs.nrec > 0) {
@@ -2115,10 +2123,10 @@ static void ensure_rows(dmc_context* ctx) {
     fill_u32(ctx, deg, nv, 0u);
     fill_u32(ctx, cursor, nv, 0u);
     launch(ctx, "k_he_degree", k_he_degree, dim3(grid_for(ctx, hcap)), dim3(kBlock), quads, (const Sizes*)S, deg,
-           &S->he.pad, (const uint32_t*)nullptr);
+           &S->he.pad);
     scan_to(ctx, ScanCounts{deg}, off, nv, &S->tot, "k_scan", nullptr, off);
     launch(ctx, "k_he_scatter", k_he_scatter, dim3(grid_for(ctx, qcap)), dim3(kBlock), quads, (const Sizes*)S, off,
-           cursor, adj, (const uint32_t*)nullptr);
+           cursor, adj);
     check_launch(ctx, "rows");
     ctx->rows_live = true;
 }

@@ -377,8 +377,7 @@ __device__ __forceinline__ uint32_t contour_spread(uint32_t map, unsigned t) {
 // with at least one interior edge; the others only feed incomplete
 // quadrilaterals and are dropped by removeUnusedVertices
 // (cpp_dmc/DualMarchingCubes.h:685-729).  A vertex's quadrilaterals are
-// those of its contour's interior edges, one each: its degree and, ordered
-// by edge id, its rows in the first halfedge CSR.
+// those of its contour's interior edges, one each: its out-degree.
 __device__ __forceinline__ uint32_t cell_aux(unsigned icase, uint32_t map, int i, int j, int k, const Dims& d) {
     const uint32_t live = c_cut_spread.v[icase] & interior_spread(i, j, k, d);
     uint32_t used = 0;
@@ -387,11 +386,6 @@ __device__ __forceinline__ uint32_t cell_aux(unsigned icase, uint32_t map, int i
         if (contour_spread(map, t) & live) used |= 1u << t;
     return (live & kAllEdgesSpread) | used << 24;
 }
-// interior cut edges of contour t below edge e / in all: a vertex's rows
-__device__ __forceinline__ int contour_rank(uint32_t map, uint32_t aux, unsigned icase, unsigned t, int e) {
-    return __popc(contour_spread(map, t) & aux & c_cut_spread.v[icase] & kAllEdgesSpread & ((1u << (2 * e)) - 1u));
-}
-
 // One active cell, 16 bytes, so that a neighbour lookup is one load.
 struct ActRec {
     uint32_t cell;   // linear cell index in its volume
@@ -474,7 +468,7 @@ __global__ void __launch_bounds__(kBlock) k_cells(VolTable vt, int64_t groups, c
                                                    const uint32_t* __restrict__ segBase, uint4* __restrict__ rec,
                                                    uint32_t* __restrict__ grpV, uint32_t* __restrict__ grpQ,
                                                    VolStat* __restrict__ vstat, unsigned long long* __restrict__ cpart,
-                                                   uint32_t acap) {
+                                                   uint32_t* open_cells, uint32_t acap) {
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t wpb = kBlock / kWave;
     // one volume: its contour count is spread over kContourParts counters
@@ -485,6 +479,7 @@ __global__ void __launch_bounds__(kBlock) k_cells(VolTable vt, int64_t groups, c
                          : &vstat[vol].contours;
     };
     unsigned long long total = 0;
+    uint32_t open = 0;
     int cur = -1;  // volume whose contour count `total` holds (wave-uniform)
     for (int64_t g = (int64_t)blockIdx.x * wpb + __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave); g < groups;
          g += (int64_t)gridDim.x * wpb) {
@@ -523,13 +518,15 @@ __global__ void __launch_bounds__(kBlock) k_cells(VolTable vt, int64_t groups, c
                 const uint32_t map = m & 0xFFFFFFu;
                 total += (unsigned long long)(m >> 24);
                 aux = cell_aux(icase, map, i, j, k, d);
-                nvq = (uint32_t)__popc(aux >> 24) |
-                      ((uint32_t)(edge_cut(icase, 0) && j >= 1 && k >= 1) +
-                       (uint32_t)(edge_cut(icase, 3) && i >= 1 && k >= 1) +
-                       (uint32_t)(edge_cut(icase, 8) && i >= 1 && j >= 1)) << 16;
+                // its own edges 0, 3 and 8 are interior where all four cells
+                // around them exist
+                nvq = (uint32_t)__popc(aux >> 24) | (uint32_t)__popc(aux & 0x10041u) << 16;
                 code = icase | (map << 8);
-                bits = undecided(dec) ? 0x8000u : dec >> 4 << 30;
-                if (!undecided(dec)) aux |= dec << 28;
+                const bool und = undecided(dec);
+                // an interior edge on no contour: its vertex does not exist
+                open += und && (aux >> 24 >> (m >> 24)) != 0u;
+                bits = und ? 0x8000u : dec >> 4 << 30;
+                aux |= und ? 0u : dec << 28;
                 cell = ((uint32_t)k * (uint32_t)(d.ny - 1) + (uint32_t)j) * (uint32_t)d.C + (uint32_t)i;
             }
             const uint32_t inc = wave_inclusive_scan(nvq);
@@ -544,6 +541,7 @@ __global__ void __launch_bounds__(kBlock) k_cells(VolTable vt, int64_t groups, c
             grpQ[g] = cvq >> 16;
         }
     }
+    if (open) atomicAdd(open_cells, open);
     total = wave_sum(total);
     if (lane == 0 && total) atomicAdd(contours(cur), total);
 }
@@ -639,7 +637,8 @@ template <class T>
 __device__ __forceinline__ void store_vertex(const VolDesc& V, int i, int j, int k, const CornerRef& Fc,
                                              const OuterValues<T>& o, const double p[3], uint32_t code, uint32_t aux,
                                              int t, uint32_t out, double* __restrict__ vpos,
-                                             double* __restrict__ vnrm, uint32_t* __restrict__ vdeg) {
+                                             double* __restrict__ vnrm, uint32_t* __restrict__ vdeg,
+                                             uint32_t* __restrict__ varr) {
     const Dims& d = V.d;
     const double u = p[0], v = p[1], ww = p[2];
     const double dx2[3] = {2 * V.geo.dx, 2 * V.geo.dy, 2 * V.geo.dz};
@@ -688,15 +687,16 @@ __device__ __forceinline__ void store_vertex(const VolDesc& V, int i, int j, int
     vn[0] = div_by(n[0], s, rs);
     vn[1] = div_by(n[1], s, rs);
     vn[2] = div_by(n[2], s, rs);
-    vdeg[out] = (uint32_t)contour_rank(code >> 8, aux, code & 0xFFu, (unsigned)t, 12);
+    vdeg[out] = (uint32_t)__popc(contour_spread(code >> 8, (unsigned)t) & aux);
+    if (varr) varr[out] = 0u;   // k_quads counts the boundary halfedges that end here
 }
 
 template <class T, int kUnroll>
 __device__ __forceinline__ void vertices_run(const VolTable& vt, const uint4* __restrict__ rec,
                                              const uint32_t* __restrict__ grpV, DevN dA,
                                              double* __restrict__ vpos, double* __restrict__ vnrm,
-                                             uint32_t* __restrict__ vdeg, uint32_t* __restrict__ slow,
-                                             unsigned long long* qhead) {
+                                             uint32_t* __restrict__ vdeg, uint32_t* __restrict__ varr,
+                                             uint32_t* __restrict__ slow, unsigned long long* qhead) {
     static_assert(kBlock == kBoxStride && kBlock == kCornerStride, "LDS columns are one per thread");
     const int64_t A = dA.get();
     __shared__ float boxes[kBoxFloats * kBoxStride];
@@ -750,7 +750,7 @@ __device__ __forceinline__ void vertices_run(const VolTable& vt, const uint4* __
                     break;
                 }
                 if (!((used >> t) & 1u)) continue;
-                store_vertex<T>(V, i, j, k, Fc, o, p, code, aux, t, out, vpos, vnrm, vdeg);
+                store_vertex<T>(V, i, j, k, Fc, o, p, code, aux, t, out, vpos, vnrm, vdeg, varr);
                 out++;
             }
         }
@@ -775,9 +775,9 @@ template <class T>
 __global__ void __launch_bounds__(kBlock) TMC_VERTICES_ATTR k_vertices(VolTable vt, const uint4* __restrict__ rec,
                                                       const uint32_t* __restrict__ grpV, DevN dA,
                                                       double* __restrict__ vpos, double* __restrict__ vnrm,
-                                                      uint32_t* __restrict__ vdeg, uint32_t* __restrict__ slow,
-                                                      unsigned long long* qhead) {
-    vertices_run<T, 7>(vt, rec, grpV, dA, vpos, vnrm, vdeg, slow, qhead);
+                                                      uint32_t* __restrict__ vdeg, uint32_t* __restrict__ varr,
+                                                      uint32_t* __restrict__ slow, unsigned long long* qhead) {
+    vertices_run<T, 7>(vt, rec, grpV, dA, vpos, vnrm, vdeg, varr, slow, qhead);
 }
 
 // K3 for larger passes: samples one at a time, which fits 3 waves per SIMD
@@ -788,9 +788,10 @@ __global__ void __launch_bounds__(kBlock) TMC_VERTICES_ATTR k_vertices(VolTable 
 template <class T>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 3)))
 k_vertices_wide(VolTable vt, const uint4* __restrict__ rec, const uint32_t* __restrict__ grpV, DevN dA,
-                double* __restrict__ vpos, double* __restrict__ vnrm, uint32_t* __restrict__ vdeg, uint32_t* __restrict__ slow,
+                double* __restrict__ vpos, double* __restrict__ vnrm, uint32_t* __restrict__ vdeg,
+                uint32_t* __restrict__ varr, uint32_t* __restrict__ slow,
                 unsigned long long* qhead) {
-    vertices_run<T, 1>(vt, rec, grpV, dA, vpos, vnrm, vdeg, slow, qhead);
+    vertices_run<T, 1>(vt, rec, grpV, dA, vpos, vnrm, vdeg, varr, slow, qhead);
 }
 
 // General path of K3 for the cells k_vertices deferred: every contour is
@@ -801,7 +802,8 @@ __global__ void __launch_bounds__(kBlock) k_vertices_slow(VolTable vt, const uin
                                                           const uint32_t* __restrict__ grpV,
                                                           const uint32_t* __restrict__ slow,
                                                           double* __restrict__ vpos, double* __restrict__ vnrm,
-                                                          uint32_t* __restrict__ vdeg, VolStat* __restrict__ vstat) {
+                                                          uint32_t* __restrict__ vdeg, uint32_t* __restrict__ varr,
+                                                          VolStat* __restrict__ vstat) {
     __shared__ float boxes[kBoxFloats * kBoxStride];
     __shared__ double corners[8 * kCornerStride];
     const BoxRef B{boxes + threadIdx.x};
@@ -845,7 +847,7 @@ __global__ void __launch_bounds__(kBlock) k_vertices_slow(VolTable vt, const uin
                 }
             }
             if (!((used >> t) & 1u)) continue;
-            store_vertex<T>(V, i, j, k, Fc, o, p, code, aux, t, out, vpos, vnrm, vdeg);
+            store_vertex<T>(V, i, j, k, Fc, o, p, code, aux, t, out, vpos, vnrm, vdeg, varr);
             out++;
         }
     }
@@ -859,9 +861,33 @@ struct SegLists {
     int64_t rsBase;                   // first (row, segment) of the volume
 };
 
-// Position of cell (i, j, k) in the active arrays from its segment's
-// activity words: the active cells before it are those of lower lanes (any
-// word) and of its own lane in lower words.  -1 if the cell is not active.
+// Activity words of a (row, segment) (bit L of word q <-> cell 4L + q) and its
+// first active index.
+struct SegWords {
+    unsigned long long w[4];
+    uint32_t base;
+};
+__device__ __forceinline__ SegWords seg_words(const unsigned long long* __restrict__ mask,
+                                              const uint32_t* __restrict__ base, int64_t rs) {
+    const ulonglong2* m2 = reinterpret_cast<const ulonglong2*>(mask + 4 * rs);
+    const ulonglong2 a = m2[0], b = m2[1];
+    return SegWords{{a.x, a.y, b.x, b.y}, base[rs]};
+}
+// Flat position of the first active cell at or after cell i of the segment's
+// row: the active cells before it are those of lower lanes (any word) and of
+// its own lane in lower words.  The cells before and after cell i in the row,
+// where they are active, are next to it in the flat order, also across
+// segments.
+__device__ __forceinline__ uint32_t active_at(const SegWords& s, int i) {
+    const int il = i % kSeg, ln = il >> 2, q = il & 3;
+    const unsigned long long below = (1ull << ln) - 1ull;
+    uint32_t rank = 0;
+#pragma unroll
+    for (int t = 0; t < 4; t++) rank += (uint32_t)__popcll(s.w[t] & below) + (t < q ? (uint32_t)((s.w[t] >> ln) & 1ull) : 0u);
+    return s.base + rank;
+}
+
+// Position of cell (i, j, k) in the active arrays; -1 if it is not active.
 __device__ __forceinline__ int64_t find_active(const SegLists& L, const Dims& d, int i, int j, int k) {
     const int64_t rs = L.rsBase + ((int64_t)k * (d.ny - 1) + j) * L.S + (i / kSeg);
     const int il = i % kSeg, ln = il >> 2, q = il & 3;
@@ -874,114 +900,6 @@ __device__ __forceinline__ int64_t find_active(const SegLists& L, const Dims& d,
 #pragma unroll
     for (int t = 0; t < 4; t++) rank += __popcll(w[t] & below) + (t < q ? (int)((w[t] >> ln) & 1ull) : 0);
     return (int64_t)L.base[rs] + rank;
-}
-
-// Final id of the vertex of active cell `a` (cell (i, ., .) of cell row r)
-// whose contour contains edge e, and the row of edge e among that contour's
-// interior edges (its slot in the first halfedge CSR).
-__device__ __forceinline__ int32_t vertex_slot_of(const uint4* __restrict__ rec, const uint32_t* __restrict__ grpV,
-                                                  const VolDesc& V, int64_t a, int e, int64_t r, int i, int& slot) {
-    slot = 0;
-    if (a < 0) return -1;
-    const ActRec R = load_rec(rec, a);
-    const uint32_t map = R.code >> 8;
-    const unsigned t = (map >> (2 * e)) & 3u;
-    slot = contour_rank(map, R.aux, R.code & 0xFFu, t, e);
-    return (int32_t)(first_vertex(V, (uint32_t)r, i, R, grpV) + __popc(R.used() & ((1u << t) - 1u)));
-}
-
-// ---------------------------------------------------------------------------
-// K4: quadrilaterals.  Each complete quadrilateral belongs to the grid edge
-// e0 (x), e3 (y) or e8 (z) of the cell at its lower corner; ascending
-// (cell, direction) is the reference's map order
-// (cpp_dmc/DualMarchingCubes.h:215-223, :663-676).  Colour: 3*parity + dir
-// (cpp_dmc/DualMarchingCubes.cpp:180-183).
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(kBlock) k_quads(VolTable vt, const uint4* __restrict__ rec,
-                                                   const uint32_t* __restrict__ grpV,
-                                                   const uint32_t* __restrict__ grpQ, DevN dA,
-                                                   const unsigned long long* __restrict__ segMask,
-                                                   const uint32_t* __restrict__ segBase,
-                                                   int32_t* __restrict__ quads, uint8_t* __restrict__ colors,
-                                                   const uint32_t* __restrict__ off, int2* __restrict__ adj,
-                                                   uint64_t adjcap, uint32_t* unresolved) {
-    const int64_t A = dA.get();
-    for (int64_t a = (int64_t)blockIdx.x * kBlock + threadIdx.x; a < A; a += (int64_t)gridDim.x * kBlock) {
-        const int vol = vol_of(vt.aBase, vt.n, a);
-        const VolDesc& V = vt.desc[vol];
-        const Dims d = V.d;
-        const SegLists L{segMask, segBase, V.S, V.rsBase};
-        const ActRec R = load_rec(rec, a);
-        int i, j, k;
-        uint32_t r;
-        cell_ijk(R.cell, d, i, j, k, r);
-        const unsigned icase = R.code & 0xFFu;
-        const int bit = (icase & 1u) ? 0 : 1;     // field at the edge origin below iso
-        const int parity = (i & 1) | (j & 1) << 1 | (k & 1) << 2;
-        int64_t q = (int64_t)grpQ[cell_group(V, r, i)] + R.qloc();
-        const bool ex = edge_cut(icase, 0) && j >= 1 && k >= 1;
-        const bool ey = edge_cut(icase, 3) && i >= 1 && k >= 1;
-        const bool ez = edge_cut(icase, 8) && i >= 1 && j >= 1;
-        if (!(ex || ey || ez)) continue;
-        int s0, s3, s8;
-        const int32_t own0 = vertex_slot_of(rec, grpV, V, a, 0, r, i, s0);
-        const int32_t own3 = vertex_slot_of(rec, grpV, V, a, 3, r, i, s3);
-        const int32_t own8 = vertex_slot_of(rec, grpV, V, a, 8, r, i, s8);
-        // rows of the cells (., j-1, k) and (., j, k-1)
-        const int64_t rj = (int64_t)r - 1, rk = (int64_t)r - (d.ny - 1);
-        // cells of the previous row (j-1) and plane (k-1) found once
-        const int64_t cjm = (ex || ez) ? find_active(L, d, i, j - 1, k) : -1;
-        const int64_t ckm = (ex || ey) ? find_active(L, d, i, j, k - 1) : -1;
-        int32_t out[4];
-        int sl[4];
-        // quadrilateral q with its vertices in out[]: store it, and each of
-        // its halfedges (4q+p: out[p] -> out[p+1]) in its origin's CSR row
-        auto emit = [&](int c) {
-            if (out[0] < 0 || out[1] < 0 || out[2] < 0 || out[3] < 0) {
-                atomicAdd(unresolved, 1u);
-            } else {
-#pragma unroll
-                for (int p = 0; p < 4; p++) {
-                    // rows total 4 Q (checked by the host); never past the array
-                    const uint64_t at = (uint64_t)off[out[p]] + (uint64_t)sl[p];
-                    if (at < adjcap) adj[at] = make_int2((int32_t)(4 * q + p), out[(p + 1) & 3]);
-                }
-            }
-            reinterpret_cast<int4*>(quads)[q] = make_int4(out[0], out[1], out[2], out[3]);
-            colors[q] = (uint8_t)(3 * parity + c);
-            q++;
-        };
-        // x edge: cells (i,j,k) e0, (i,j-1,k) e2, (i,j,k-1) e4, (i,j-1,k-1) e6
-        if (ex) {
-            const int64_t e = find_active(L, d, i, j - 1, k - 1);
-            out[edge_slot(0, bit)] = own0;
-            sl[edge_slot(0, bit)] = s0;
-            out[edge_slot(2, bit)] = vertex_slot_of(rec, grpV, V, cjm, 2, rj, i, sl[edge_slot(2, bit)]);
-            out[edge_slot(4, bit)] = vertex_slot_of(rec, grpV, V, ckm, 4, rk, i, sl[edge_slot(4, bit)]);
-            out[edge_slot(6, bit)] = vertex_slot_of(rec, grpV, V, e, 6, rk - 1, i, sl[edge_slot(6, bit)]);
-            emit(0);
-        }
-        // y edge: cells (i,j,k) e3, (i-1,j,k) e1, (i,j,k-1) e7, (i-1,j,k-1) e5
-        if (ey) {
-            const int64_t e = ckm > 0 ? ckm - 1 : -1;
-            out[edge_slot(3, bit)] = own3;
-            sl[edge_slot(3, bit)] = s3;
-            out[edge_slot(1, bit)] = vertex_slot_of(rec, grpV, V, a - 1, 1, r, i - 1, sl[edge_slot(1, bit)]);
-            out[edge_slot(7, bit)] = vertex_slot_of(rec, grpV, V, ckm, 7, rk, i, sl[edge_slot(7, bit)]);
-            out[edge_slot(5, bit)] = vertex_slot_of(rec, grpV, V, e, 5, rk, i - 1, sl[edge_slot(5, bit)]);
-            emit(1);
-        }
-        // z edge: cells (i,j,k) e8, (i-1,j,k) e9, (i,j-1,k) e11, (i-1,j-1,k) e10
-        if (ez) {
-            const int64_t e = cjm > 0 ? cjm - 1 : -1;
-            out[edge_slot(8, bit)] = own8;
-            sl[edge_slot(8, bit)] = s8;
-            out[edge_slot(9, bit)] = vertex_slot_of(rec, grpV, V, a - 1, 9, r, i - 1, sl[edge_slot(9, bit)]);
-            out[edge_slot(11, bit)] = vertex_slot_of(rec, grpV, V, cjm, 11, rj, i, sl[edge_slot(11, bit)]);
-            out[edge_slot(10, bit)] = vertex_slot_of(rec, grpV, V, e, 10, rj, i - 1, sl[edge_slot(10, bit)]);
-            emit(2);
-        }
-    }
 }
 
 // ---------------------------------------------------------------------------

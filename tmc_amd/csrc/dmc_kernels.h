@@ -80,7 +80,6 @@ struct Sizes {
     uint64_t acnt;               // active cells the cell kernels process: A, or 0 once a capacity is exceeded
     uint64_t nv, nq;             // the live mesh
     uint64_t nn, qn;             // vertices / quadrilaterals a compaction keeps
-    uint64_t rows;               // first CSR's row total (4 Q)
     uint64_t tot;                // a scan total no one else reads
     uint64_t hq;                 // halfedges of the mesh a compaction leaves (4 qn)
     uint64_t naff;               // halfedges a compaction left to pair again
@@ -89,10 +88,8 @@ struct Sizes {
     uint32_t ovf;                // capacities exceeded: 1 active cells, 2 vertices, 4 quads, 8 3-face records
     uint32_t unresolved;         // quadrilaterals with an unresolved neighbour cell
     uint32_t zero;               // vertices of valence 0 (all valence passes)
-    uint32_t generic;            // this halfedge build counts its rows from the quadrilaterals
+    uint32_t open_cells;         // cells with an interior edge on no contour (NaN deciders)
     uint32_t need_generic;       // a build needed generic rows the pass did not launch: run it again with them
-    uint32_t pair_rows;          // this build pairs halfedges through full rows (cell rows or generic)
-    uint32_t incr;               // this build is the one the last compaction carried over
     uint32_t incr_ok;            // the build before the compaction saw no invalid vertex reference
     uint32_t cbad;               // invalid references the last quadrilateral compaction met
     uint32_t nrec;               // 3-face edge records of the current build

@@ -24,9 +24,7 @@ __device__ __forceinline__ int32_t he_prev(int32_t h) { return (h & ~3) | ((h + 
 __device__ __forceinline__ bool vid_ok(int32_t v, int64_t nv) { return v >= 0 && (int64_t)v < nv; }
 
 __global__ void __launch_bounds__(kBlock) k_he_degree(const int32_t* __restrict__ quads, const Sizes* S,
-                                                       uint32_t* __restrict__ deg, uint32_t* __restrict__ bad,
-                                                       const uint32_t* __restrict__ gate) {
-    if (gated_off(gate)) return;
+                                                       uint32_t* __restrict__ deg, uint32_t* __restrict__ bad) {
     const int64_t nhe = 4 * (int64_t)S->nq, nv = (int64_t)S->nv;
     TMC_GRID_STRIDE(h, nhe) {
         const int32_t v = quads[h];
@@ -39,8 +37,7 @@ __global__ void __launch_bounds__(kBlock) k_he_degree(const int32_t* __restrict_
 // inside a row is arbitrary (the group search sorts what it needs).
 __global__ void __launch_bounds__(kBlock) k_he_scatter(const int32_t* __restrict__ quads, const Sizes* S,
                                                         const uint32_t* __restrict__ off, uint32_t* __restrict__ cursor,
-                                                        int2* __restrict__ adj, const uint32_t* __restrict__ gate) {
-    if (gated_off(gate)) return;
+                                                        int2* __restrict__ adj) {
     const int64_t nq = (int64_t)S->nq, nv = (int64_t)S->nv;
     TMC_GRID_STRIDE(f, nq) {
         const int4 q = reinterpret_cast<const int4*>(quads)[f];
@@ -213,11 +210,14 @@ struct HeCount {
 
 // Per volume of a batch (rare events): [3v] non-manifold halfedges, [3v+1]
 // 3-face halfedges, [3v+2] groups of more than 4.
+__device__ __forceinline__ void vol_count_of(unsigned long long* __restrict__ vst, int vol, uint8_t fl) {
+    if (!vst || (fl != 1 && fl != 2 && fl != kFlagErrFirst)) return;
+    atomicAdd(&vst[3 * vol + (fl == 1 ? 0 : fl == 2 ? 1 : 2)], 1ull);
+}
 __device__ __forceinline__ void vol_count(unsigned long long* __restrict__ vst, const int64_t* __restrict__ qb,
                                           int nvol, int32_t h, uint8_t fl) {
     if (!vst || (fl != 1 && fl != 2 && fl != kFlagErrFirst)) return;
-    const int vol = vol_of(qb, nvol, h >> 2);
-    atomicAdd(&vst[3 * vol + (fl == 1 ? 0 : fl == 2 ? 1 : 2)], 1ull);
+    vol_count_of(vst, vol_of(qb, nvol, h >> 2), fl);
 }
 
 // Twin and flag of every halfedge (cpp_dmc/DualMarchingCubes.cpp:574-669),
@@ -244,10 +244,8 @@ __global__ void __launch_bounds__(kBlock) k_he_twins(const int32_t* __restrict__
                                                       uint32_t* __restrict__ arr, unsigned long long (*hep)[3],
                                                       BndRec* __restrict__ recs, uint32_t* nrec, uint32_t reccap,
                                                       uint32_t* ovf, const int64_t* __restrict__ qb, int nvol,
-                                                      unsigned long long* __restrict__ vst,
-                                                      const uint32_t* __restrict__ gate) {
+                                                      unsigned long long* __restrict__ vst) {
     static_assert(kBlock % 4 == 0, "quads must not straddle blocks");
-    if (gated_off(gate)) return;
     const int64_t nhe = 4 * (int64_t)S->nq, nv = (int64_t)S->nv;
     HeCount cnt;
     TMC_GRID_STRIDE(h64, nhe) {
@@ -1253,34 +1251,28 @@ __global__ void __launch_bounds__(kBlock) k_carry_records(const BndRec* __restri
     }
 }
 
-// Before a halfedge build: which way it pairs.  ready: 0 generic rows
-// (launched only in a pass run again for them), 1 the cell stage's rows, 2
-// the build a compaction carried over.  The cell stage's rows are whole
-// unless a quadrilateral has an unresolved neighbour cell; a carried build
-// stands only if the build before it and the compaction met no invalid
-// vertex reference.  Otherwise the build needs generic rows, which this
-// pass did not launch: it flags the pass to be run again with them.
+// Before a halfedge build: whether what it starts from stands.  ready: 0
+// generic rows (launched only in a pass run again for them), 1 the cell
+// stage's build, 2 the build a compaction carried over.  The cell stage's
+// build is whole unless a quadrilateral has an unresolved neighbour cell; a
+// carried build stands only if the build before it and the compaction met no
+// invalid vertex reference.  Otherwise the build needs generic rows, which
+// this pass did not launch: it flags the pass to be run again with them.
 __global__ void k_rows_gate(Sizes* S, int ready, int commit) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (commit) {   // the compaction before this build: its counts become the live mesh
             S->nv = S->nn;
             S->nq = S->qn;
         }
-        const bool incr = ready == 2 && S->incr_ok != 0u && S->cbad == 0u;
-        const bool need = (ready == 1 && S->unresolved != 0u) || (ready == 2 && !incr);
-        if (need) S->need_generic = 1u;
-        S->incr = incr ? 1u : 0u;
-        S->pair_rows = ready == 0 || (ready == 1 && !need) ? 1u : 0u;
-        S->generic = ready == 0 ? 1u : 0u;
-        if (!incr) {
+        const bool stands = ready == 1 ? S->unresolved == 0u : ready == 2 && S->incr_ok != 0u && S->cbad == 0u;
+        if (ready != 0 && !stands) S->need_generic = 1u;
+        if (!stands) {
             S->recmax = S->nrec > S->recmax ? S->nrec : S->recmax;
             he_clear(S);
             S->nrec = 0;
         }
     }
 }
-
-
 
 // ---------------------------------------------------------------------------
 // Diagnostics of a finished mesh
