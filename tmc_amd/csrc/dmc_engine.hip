@@ -26,6 +26,7 @@
 #include "dmc_extract_kernels.h"
 #include "dmc_mesh_kernels.h"
 #include "dmc_quad_kernels.h"
+#include "dmc_simplify_kernels.h"
 #include "tmc_kernels.h"
 
 using namespace tmc;
@@ -117,20 +118,16 @@ struct dmc_context {
     int pcur = 0;  // which positions/normals buffer holds the vertex data
     int scur = 0;  // which slot map is live ...
     bool slots = false;  // ... once a compaction has run (else slots are the identity)
-    // what the next halfedge build starts from: 1 the cell stage's build, 2 the
-    // build a compaction carried over, 0 nothing
-    int ready = 0;
     bool rows_live = false;   // off/adj hold the rows of the last extraction's final mesh
-    bool force_generic = false;   // this extraction's passes pair every build through generic rows
-    bool commit_pending = false;  // a compaction's counts wait for the next build's gate to commit them
-    bool always_generic = false;  // every extraction pairs through generic rows (TMC_GENERIC_ROWS=1)
+    bool force_generic = false;   // this extraction's passes compact and pair through generic rows per stage
+    bool commit_pending = false;  // a compaction's counts wait for the next build to commit them
+    bool always_generic = false;  // every extraction runs so (TMC_GENERIC_ROWS=1)
     int scan_spin = kScanSpin;    // polls a scan look-back waits before it sums the input (TMC_SCAN_SPIN)
-    // halfedges / simplification scratch.  twin, flag, deg (out-degree), hev
-    // and bndrec are the current build's; the ...2 buffers receive the build
-    // a compaction carries over, and the pairs swap.
-    Buf deg, off, cursor, adj, twin, flag, hev, ovr, bndrec, nbnd, val, p, em, vfirst, vsecond, lastT, lastR,
-        newV, newQ, clist, cnbr, ccnt, tris, stats, off2, adj2, vmap, mlist, slow, twin2, flag2, deg2, hev2, bndrec2, arr,
-        cflag, aflag, bcount, boff, alist;
+    // halfedges / simplification scratch.  twin, flag, hev and bndrec are the
+    // current mesh's; the ...2 buffers receive the compacted mesh's, and the
+    // pairs swap.
+    Buf deg, deg2, off, cursor, adj, arr, twin, flag, hev, twin2, flag2, hev2, ovr, bndrec, bndrec2, val, p, em, vfirst,
+        vsecond, lastT, lastR, newV, newQ, clist, cnbr, ccnt, tris, vmap, mlist, slow, dead, vstate, irr, head, ent, frame;
     // diagnostics of the last mesh
     Buf drep, dnew, dval, dhist, dedges, dqual;
     // topologically correct MC: per active cell vertex / triangle counts and
@@ -157,7 +154,7 @@ struct dmc_context {
         std::string key;
         hipGraphExec_t exec = nullptr;
         uint64_t use = 0;
-        int cur = 0, pcur = 0, scur = 0, ready = 0;
+        int cur = 0, pcur = 0, scur = 0;
         bool slots = false;
         uint32_t swapped = 0;   // which buffer pairs are in the order opposite to their addresses
     };
@@ -195,12 +192,11 @@ struct dmc_context {
 
     dmc_context() {
         Buf* all[] = {&segCount, &segBase, &segMask, &lists, &acell, &acode, &rec, &grpNV, &grpNQ, &grpV, &grpQ,
-                      &field, &grads, &scanPartial, &scanState, &scanTotal, &sizes, &pos[0], &pos[1], &nrm[0], &nrm[1], &vslot[0], &vslot[1],
-                      &quads[0], &quads[1], &colors, &deg, &off, &cursor, &adj, &twin, &flag, &hev, &ovr,
-                      &bndrec, &nbnd, &val, &p, &em, &vfirst, &vsecond, &lastT, &lastR, &newV,
-                      &newQ, &clist, &cnbr, &ccnt, &tris, &stats, &vtab, &vstat, &vbound, &qbound, &vhe,
-                      &off2, &adj2, &vmap, &mlist, &slow, &twin2, &flag2, &deg2, &hev2, &bndrec2, &arr, &cflag,
-                      &aflag, &bcount, &boff, &alist, &drep, &dnew, &dval,
+                      &field, &grads, &scanPartial, &scanState, &scanTotal, &sizes, &pos[0], &pos[1], &nrm[0], &nrm[1],
+                      &vslot[0], &vslot[1], &quads[0], &quads[1], &colors, &deg, &deg2, &off, &cursor, &adj, &arr,
+                      &twin, &flag, &hev, &twin2, &flag2, &hev2, &ovr, &bndrec, &bndrec2, &val, &p, &em, &vfirst,
+                      &vsecond, &lastT, &lastR, &newV, &newQ, &clist, &cnbr, &ccnt, &tris, &vmap, &mlist, &slow,
+                      &dead, &vstate, &irr, &head, &ent, &frame, &vtab, &vstat, &vbound, &qbound, &vhe, &drep, &dnew, &dval,
                       &dhist, &dedges, &dqual, &tcntv, &tcntt, &tvofs, &ttofs, &tamb, &tvb, &tstats, &tpos, &tnrm,
                       &ttris};
         for (Buf* b : all) bufs.push_back(b);
@@ -387,12 +383,11 @@ uint64_t read_u64(dmc_context* ctx, const void* dptr) {
 // Device sizes block of the running pass (allocated with the pass).
 Sizes* dsizes(dmc_context* ctx) { return static_cast<Sizes*>(ctx->sizes.p); }
 
-// The double-buffered halfedge arrays swap at every compaction; a pass
+// The double-buffered halfedge arrays swap at the compaction; a pass
 // starts from one order (lower address current) so that passes of one shape
 // launch on the same pointers.
 Buf dmc_context::* const kPairs[][2] = {{&dmc_context::twin, &dmc_context::twin2},
                                         {&dmc_context::flag, &dmc_context::flag2},
-                                        {&dmc_context::deg, &dmc_context::deg2},
                                         {&dmc_context::hev, &dmc_context::hev2},
                                         {&dmc_context::bndrec, &dmc_context::bndrec2}};
 constexpr int kNumPairs = sizeof(kPairs) / sizeof(kPairs[0]);
@@ -749,10 +744,10 @@ void plan_caps(dmc_context* ctx, const std::vector<HostVol>& hv, int64_t cells) 
     ctx->reccap = std::max<int64_t>(ctx->reccap, 1024);
 }
 
-// final_build: no simplification follows, the cell stage's halfedges are the
-// final mesh's.
+// live: simplifications follow on the live mesh, whose per-vertex and
+// per-face state the cell stage initialises.
 template <class T>
-void run_cells(dmc_context* ctx, const SweepPlan& P, bool final_build) {
+void run_cells(dmc_context* ctx, const SweepPlan& P, bool live) {
     // canonical buffer roles at the start of every pass, so that a pass of
     // the same shape launches on the same pointers (and can be replayed)
     set_pair_order(ctx, 0);
@@ -792,21 +787,26 @@ void run_cells(dmc_context* ctx, const SweepPlan& P, bool final_build) {
     double* nrm = ensure<double>(ctx, ctx->nrm[0], 3 * vcap);
     int32_t* quads = ensure<int32_t>(ctx, ctx->quads[0], 4 * qcap);
     uint8_t* colors = ensure<uint8_t>(ctx, ctx->colors, qcap);
-    // the first halfedge build straight from the cells: out-degree of each
-    // vertex from k_vertices, the rest from k_quads
-    uint32_t* deg = ensure<uint32_t>(ctx, ctx->deg, vcap);
-    uint32_t* arr = final_build ? nullptr : ensure<uint32_t>(ctx, ctx->arr, vcap);
+    // the first halfedge build straight from the cells (k_quads)
+    VertexOut vo{};
     QuadOut qo{};
     qo.quads = quads;
     qo.colors = colors;
     qo.twin = ensure<int32_t>(ctx, ctx->twin, 4 * qcap);
     qo.flag = ensure<uint8_t>(ctx, ctx->flag, 4 * qcap);
     qo.hev = ensure<int32_t>(ctx, ctx->hev, vcap);
-    qo.arr = arr;
     qo.recs = ensure<BndRec>(ctx, ctx->bndrec, ctx->reccap);
     qo.reccap = (uint32_t)ctx->reccap;
     qo.S = S;
-    if (final_build && n > 1) {
+    if (live) {
+        vo.val = ensure<int32_t>(ctx, ctx->val, vcap);
+        vo.claim = ensure<int32_t>(ctx, ctx->lastR, vcap);
+        vo.last = ensure<int32_t>(ctx, ctx->lastT, vcap);
+        vo.vs = ensure<uint8_t>(ctx, ctx->vstate, vcap + 4);
+        qo.val = vo.val;
+        qo.dead = ensure<uint8_t>(ctx, ctx->dead, qcap + 4);
+    }
+    if (n > 1) {
         qo.vst = ensure<unsigned long long>(ctx, ctx->vhe, 3 * (size_t)n);
         fill_u32(ctx, qo.vst, hn(6 * (int64_t)n), 0u);
     }
@@ -817,34 +817,32 @@ void run_cells(dmc_context* ctx, const SweepPlan& P, bool final_build) {
     // threads (F32 fields: the F64 form would spill at 3 waves)
     const dim3 gv(grid_for(ctx, acap, kBlock, kVerticesBlocks));
     if (std::is_same<T, float>::value && acap > kVerticesBlocks * kBlock)
-        launch(ctx, "k_vertices", k_vertices_wide<T>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, deg,
-               arr, slow, &S->qhead);
+        launch(ctx, "k_vertices", k_vertices_wide<T>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, vo, slow,
+               &S->qhead);
     else
-        launch(ctx, "k_vertices", k_vertices<T>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, deg, arr,
-               slow, &S->qhead);
+        launch(ctx, "k_vertices", k_vertices<T>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, vo, slow,
+               &S->qhead);
     check_launch(ctx, "k_vertices");
     launch(ctx, "k_vertices_slow", k_vertices_slow<T>, dim3(grid_for(ctx, acap, kBlock, 1024)), dim3(kBlock), vt,
-           rec, grpV, slow, pos, nrm, deg, arr, sw.vstat);
+           rec, grpV, slow, pos, nrm, vo, sw.vstat);
     check_launch(ctx, "k_vertices_slow");
     mark(ctx, "quads");
     launch(ctx, "k_quads", n > 1 ? k_quads<true> : k_quads<false>, dim3(grid_for(ctx, acap)), dim3(kBlock), vt, rec,
            grpV, grpQ, A, sw.segMask, sw.segBase, qo, &S->unresolved);
     check_launch(ctx, "k_quads");
-    ctx->ready = 1;
 }
 
 // ---------------------------------------------------------------------------
 // halfedges
 // ---------------------------------------------------------------------------
 // A halfedge build gives every halfedge its twin and flag, every vertex its
-// out-degree, valence and he_v, and lists the 3-face edges.  The first build
-// comes with the quadrilaterals (k_quads).  A compaction carries the build
-// over to the mesh it leaves: most groups keep their members, renumbered, and
-// only halfedges at a changed vertex are paired again.  If the device finds
-// either unusable (a quadrilateral with an unresolved neighbour cell, an
-// invalid vertex reference), the pass runs again and every build counts
-// generic rows of outgoing (halfedge, destination) pairs from the
-// quadrilaterals and pairs everything.
+// valence and he_v, and lists the 3-face edges.  It comes with the
+// quadrilaterals (k_quads), and the simplifications keep it up to date on the
+// live mesh (dmc_simplify_kernels.h).  A pass that meets what these cannot
+// express (a quadrilateral with an unresolved neighbour cell, need_generic)
+// runs again stage by stage: each build counts generic rows of outgoing
+// (halfedge, destination) pairs from the quadrilaterals and pairs everything,
+// each simplification compacts the mesh.
 
 // Pairing through generic rows.
 void pair_rows(dmc_context* ctx, bool final_pass) {
@@ -877,41 +875,35 @@ void pair_rows(dmc_context* ctx, bool final_pass) {
            cursor, adj);
     launch(ctx, "k_he_twins", k_he_twins, dim3(grid_for(ctx, hcap)), dim3(kBlock), quads, (const Sizes*)S, off, adj,
            twin, flag, hev, arr, S->hep, recs, &S->nrec, (uint32_t)ctx->reccap, &S->ovf,
-           static_cast<const int64_t*>(ctx->qbound.p), ctx->nvol, vst);
+           static_cast<const int64_t*>(ctx->qbound.p), ctx->nvol, vst, final_pass ? 1 : 0);
     check_launch(ctx, "k_he_twins");
 }
 
-// A halfedge build of the live mesh.  Not final: ends with the valence,
-// which also clears what the next simplification needs cleared.  Final: the
-// 3-face overrides of he_v and the reference's flag values.
+// A halfedge build of a pass run stage by stage.  Not final: ends with the
+// valence, which also clears what the next simplification needs cleared.
 void build_halfedges(dmc_context* ctx, bool final_pass, const StageClears& clears = StageClears{}) {
     Sizes* S = dsizes(ctx);
     const int64_t vcap = ctx->vcap;
-    const int ready = ctx->force_generic ? 0 : ctx->ready;
-    launch(ctx, "k_rows_gate", k_rows_gate, dim3(1), dim3(64), S, ready, ctx->commit_pending ? 1 : 0);
+    launch(ctx, "k_build_begin", k_build_begin, dim3(1), dim3(64), S, ctx->commit_pending ? 1 : 0);
     ctx->commit_pending = false;
-    ctx->ready = 0;
-    if (ready == 0) pair_rows(ctx, final_pass);
-    const int gv = grid_for(ctx, vcap);
-    if (!final_pass) {
-        uint32_t* val = ensure<uint32_t>(ctx, ctx->val, vcap);
-        launch(ctx, "k_valence", k_valence, dim3(gv), dim3(kBlock), static_cast<const uint32_t*>(ctx->deg.p),
-               static_cast<const uint32_t*>(ctx->arr.p), (const Sizes*)S, val, &S->zero, clears);
-        check_launch(ctx, "valence");
-        return;
-    }
-    const int32_t* quads = static_cast<const int32_t*>(ctx->quads[ctx->cur].p);
-    int32_t* hev = static_cast<int32_t*>(ctx->hev.p);
-    const BndRec* recs = static_cast<const BndRec*>(ctx->bndrec.p);
-    unsigned long long* ovr = ensure<unsigned long long>(ctx, ctx->ovr, vcap);
-    fill_u32(ctx, ovr, DevN{nullptr, 2 * vcap}, 0u, &S->nrec);
-    const int gr = grid_for(ctx, ctx->reccap);
-    for (int pass = 0; pass < 2; pass++)
-        launch(ctx, "k_three_apply", k_three_apply, dim3(gr), dim3(kBlock), recs, (const Sizes*)S,
-               (uint32_t)ctx->reccap, quads, ovr, pass, hev);
-    launch(ctx, "k_strip_flags", k_strip_flags, dim3(grid_for(ctx, 4 * ctx->qcap)), dim3(kBlock), (const Sizes*)S,
-           static_cast<uint8_t*>(ctx->flag.p));
-    check_launch(ctx, "final halfedges");
+    pair_rows(ctx, final_pass);
+    if (final_pass) return;
+    uint32_t* val = ensure<uint32_t>(ctx, ctx->val, vcap);
+    launch(ctx, "k_valence", k_valence, dim3(grid_for(ctx, vcap)), dim3(kBlock),
+           static_cast<const uint32_t*>(ctx->deg.p), static_cast<const uint32_t*>(ctx->arr.p), (const Sizes*)S, val,
+           &S->zero, clears);
+    check_launch(ctx, "valence");
+}
+
+// The 3-face overrides of he_v of the finished mesh; compacted: its counts
+// replace the live mesh's.
+void finish_halfedges(dmc_context* ctx, bool compacted) {
+    Sizes* S = dsizes(ctx);
+    unsigned long long* ovr = ensure<unsigned long long>(ctx, ctx->ovr, ctx->vcap);
+    launch(ctx, "k_finish", k_finish, dim3(1), dim3(1024), S, static_cast<const BndRec*>(ctx->bndrec.p),
+           (uint32_t)ctx->reccap, static_cast<const int32_t*>(ctx->quads[ctx->cur].p), ovr,
+           static_cast<int32_t*>(ctx->hev.p), compacted ? 1 : 0);
+    check_launch(ctx, "k_finish");
 }
 
 // Meshes of at most this many faces are coloured by one block.
@@ -1012,17 +1004,16 @@ void remap_bounds(dmc_context* ctx, Buf& bounds, const uint32_t* newidx, const u
 // stay where they are; the slot map follows the vertices (gather_vertices
 // lays them out at the end).
 // The scan of the kept vertices into ctx->newV (S->nn of them), the job that
-// compact_vertices(..., scanned = true) expects to have run.
+// compact_vertices expects to have run.
 ScanJob<ScanKeep> kept_vertices_job(dmc_context* ctx, const uint8_t* removed) {
     Sizes* S = dsizes(ctx);
     return scan_job(ScanKeep{removed}, ensure<uint32_t>(ctx, ctx->newV, ctx->vcap), dn(&S->nv, ctx->vcap), &S->nn);
 }
 
-uint32_t* compact_vertices(dmc_context* ctx, const uint8_t* removed, int32_t* vsecond, bool scanned = false) {
+uint32_t* compact_vertices(dmc_context* ctx, const uint8_t* removed, int32_t* vsecond) {
     const int64_t vcap = ctx->vcap;
     Sizes* S = dsizes(ctx);
     uint32_t* newidx = ensure<uint32_t>(ctx, ctx->newV, vcap);
-    if (!scanned) scan_to(ctx, ScanKeep{removed}, newidx, dn(&S->nv, vcap), &S->nn);
     const uint32_t* slot = ctx->slots ? static_cast<const uint32_t*>(ctx->vslot[ctx->scur].p) : nullptr;
     uint32_t* slot2 = ensure<uint32_t>(ctx, ctx->vslot[1 - ctx->scur], vcap);
     launch(ctx, "k_compact_slots", k_compact_slots, dim3(grid_for(ctx, vcap)), dim3(kBlock), removed, newidx,
@@ -1050,81 +1041,23 @@ void gather_vertices(dmc_context* ctx) {
     ctx->slots = false;
 }
 
-// The carry of a compaction, first half: the face map and the buffers of the
-// carried build (the vertex map kernel then opens the carry's counters,
-// clears its flags and counts -- carry_clears -- and carries the kept
-// vertices' out-degree and he_v).  S->nn and S->qn must be on the device;
-// `last`: the compaction before the final build (a batch counts per volume).
-Carry carry_begin(dmc_context* ctx, const uint32_t* newq, bool last) {
-    const int64_t vcap = ctx->vcap, qcap = ctx->qcap, hcap = 4 * qcap;
+// The quadrilateral compaction that ends a stage of a pass run stage by
+// stage; the next build commits its counts.
+void compact_quads(dmc_context* ctx, const uint32_t* newQ, const int32_t* vmap, const uint8_t* p3333,
+                   const int32_t* vtwin) {
+    const int64_t qcap = ctx->qcap;
     Sizes* S = dsizes(ctx);
-    Carry c{};
-    c.twin = static_cast<const int32_t*>(ctx->twin.p);
-    c.flag = static_cast<const uint8_t*>(ctx->flag.p);
-    c.qmap = reinterpret_cast<const int32_t*>(newq);
-    uint8_t* cflag = ensure<uint8_t>(ctx, ctx->cflag, vcap + 4);
-    c.cflag = cflag;
-    c.twin_n = ensure<int32_t>(ctx, ctx->twin2, hcap);
-    c.flag_n = ensure<uint8_t>(ctx, ctx->flag2, hcap);
-    c.deg_n = ensure<uint32_t>(ctx, ctx->deg2, vcap);
-    c.hev_n = ensure<int32_t>(ctx, ctx->hev2, vcap);
-    c.arr = ensure<uint32_t>(ctx, ctx->arr, vcap);
-    c.aflag = ensure<uint8_t>(ctx, ctx->aflag, hcap);
-    c.cnt = ensure<uint32_t>(ctx, ctx->cursor, vcap);
-    const int64_t turns = qcap / kBlock + 1;
-    c.bcount = ensure<uint32_t>(ctx, ctx->bcount, turns);
-    c.S = S;
-    c.qb = static_cast<const int64_t*>(ctx->qbound.p);
-    c.nvol = ctx->nvol;
-    Fills fl(ctx);
-    if (last && ctx->nvol > 1) {
-        c.vst = ensure<unsigned long long>(ctx, ctx->vhe, 3 * (size_t)ctx->nvol);
-        fl.u32(c.vst, hn(6 * (int64_t)ctx->nvol), 0u);
-    }
-    fl.run();
-    return c;
-}
-
-// What k_vmap* clears for the carry begun by carry_begin.
-CarryClears carry_clears(dmc_context* ctx, const Carry& c) {
-    return CarryClears{reinterpret_cast<uint32_t*>(const_cast<uint8_t*>(c.cflag)), (ctx->vcap + 4) / 4, c.arr, c.cnt,
-                       c.bcount, ctx->qcap / kBlock + 1};
-}
-
-// Second half, after the compaction kernel: the flagged halfedges paired
-// through their rows, the 3-face records carried, the counts committed and
-// the carried build made current.
-void carry_end(dmc_context* ctx, const Carry& c, const int32_t* vmap) {
-    const int64_t vcap = ctx->vcap, hcap = 4 * ctx->qcap;
-    Sizes* S = dsizes(ctx);
-    const DevN nn = dn(&S->nn, vcap);
-    const int32_t* quads2 = static_cast<const int32_t*>(ctx->quads[1 - ctx->cur].p);
-    uint32_t* aoff = ensure<uint32_t>(ctx, ctx->off2, vcap + 1);
-    int2* aadj = ensure<int2>(ctx, ctx->adj2, hcap);
-    BndRec* recs_n = ensure<BndRec>(ctx, ctx->bndrec2, ctx->reccap);
-    const int gh = grid_for(ctx, hcap);
-    const int64_t turns = ctx->qcap / kBlock + 1;
-    uint32_t* boff = ensure<uint32_t>(ctx, ctx->boff, turns);
-    int32_t* alist = ensure<int32_t>(ctx, ctx->alist, hcap);
-    scan_pair(ctx, scan_job(ScanCounts{c.bcount}, boff, hn(turns), &S->naff),
-              scan_job(ScanCounts{c.cnt}, aoff, nn, &S->tot, nullptr, aoff));
-    launch(ctx, "k_aff_scatter", k_aff_scatter, dim3(grid_for(ctx, ctx->qcap)), dim3(kBlock), (const Sizes*)S,
-           c.qmap, (const uint8_t*)c.aflag, (const uint32_t*)c.bcount, (const uint32_t*)boff, quads2,
-           (const uint32_t*)aoff, aadj, alist);
-    launch(ctx, "k_aff_twins", k_aff_twins, dim3(gh), dim3(kBlock), (const int32_t*)alist, (const Sizes*)S, quads2,
-           (const uint32_t*)aoff, (const int2*)aadj, c, recs_n, (uint32_t)ctx->reccap);
-    launch(ctx, "k_carry_records", k_carry_records, dim3(grid_for(ctx, ctx->reccap)), dim3(kBlock),
-           static_cast<const BndRec*>(ctx->bndrec.p), (const Sizes*)S, vmap, c.cflag, c.qmap, recs_n, &S->nrec,
-           (uint32_t)ctx->reccap, &S->ovf);
-    check_launch(ctx, "carry");
-    // the counts are committed by the next build's gate
+    int32_t* q2 = ensure<int32_t>(ctx, ctx->quads[1 - ctx->cur], 4 * qcap);
+    remap_bounds(ctx, ctx->qbound, newQ, &S->nq, &S->qn);
+    launch(ctx, "k_compact_quads", k_compact_quads, dim3(grid_for(ctx, qcap)), dim3(kBlock),
+           static_cast<const int32_t*>(ctx->quads[ctx->cur].p), (const Sizes*)S, p3333, vtwin, vmap,
+           reinterpret_cast<const int32_t*>(newQ), q2);
+    check_launch(ctx, "k_compact_quads");
     ctx->commit_pending = true;
-    swap_pairs(ctx);
     ctx->cur = 1 - ctx->cur;
-    ctx->ready = 2;
 }
 
-void simplify3x3y(dmc_context* ctx, bool colored, bool last) {
+void simplify3x3y(dmc_context* ctx, bool colored) {
     const int64_t vcap = ctx->vcap, qcap = ctx->qcap;
     uint8_t* p = ensure<uint8_t>(ctx, ctx->p, qcap);
     uint8_t* em = ensure<uint8_t>(ctx, ctx->em, qcap);
@@ -1166,24 +1099,14 @@ void simplify3x3y(dmc_context* ctx, bool colored, bool last) {
            static_cast<double*>(ctx->pos[ctx->pcur].p), static_cast<double*>(ctx->nrm[ctx->pcur].p),
            ctx->slots ? static_cast<const uint32_t*>(ctx->vslot[ctx->scur].p) : nullptr, vsecond);
     check_launch(ctx, "k_merge_apply");
-    compact_vertices(ctx, vfirst, vsecond, true);
-    int32_t* q2 = ensure<int32_t>(ctx, ctx->quads[1 - ctx->cur], 4 * qcap);
+    compact_vertices(ctx, vfirst, vsecond);
     int32_t* vmap = ensure<int32_t>(ctx, ctx->vmap, vcap);
-    remap_bounds(ctx, ctx->qbound, newQ, &S->nq, &S->qn);
-    Carry c = carry_begin(ctx, newQ, last);
     launch(ctx, "k_vmap3x3y", k_vmap3x3y, dim3(grid_for(ctx, vcap)), dim3(kBlock), (const uint8_t*)vfirst,
-           (const int32_t*)vsecond, S, vmap, static_cast<const uint32_t*>(ctx->deg.p),
-           static_cast<const int32_t*>(ctx->hev.p), c.qmap, c.deg_n, c.hev_n, carry_clears(ctx, c));
-    launch(ctx, "k_changed3x3y", k_changed3x3y, dim3(gq), dim3(kBlock), quads, (const int32_t*)mlist,
-           (const Sizes*)S, (const uint8_t*)em, (const int32_t*)vmap, static_cast<const int32_t*>(ctx->hev.p),
-           const_cast<uint8_t*>(c.cflag), c.deg_n, c.hev_n);
-    launch(ctx, "k_compact_quads3x3y", k_compact_quads3x3y, dim3(gq), dim3(kBlock), quads, (const Sizes*)S,
-           (const int32_t*)vmap, q2, c);
-    check_launch(ctx, "k_compact_quads3x3y");
-    carry_end(ctx, c, vmap);
+           (const int32_t*)vsecond, (const Sizes*)S, vmap);
+    compact_quads(ctx, newQ, vmap, nullptr, nullptr);
 }
 
-void simplify3333(dmc_context* ctx, bool last) {
+void simplify3333(dmc_context* ctx) {
     const int64_t vcap = ctx->vcap, qcap = ctx->qcap;
     uint8_t* vflag = ensure<uint8_t>(ctx, ctx->vfirst, vcap);
     int32_t* vtwin = ensure<int32_t>(ctx, ctx->vsecond, vcap);
@@ -1202,7 +1125,7 @@ void simplify3333(dmc_context* ctx, bool last) {
     build_halfedges(ctx, false, cl);
     const int32_t* val = static_cast<const int32_t*>(ctx->val.p);
     Sizes* S = dsizes(ctx);
-    const DevN nv = dn(&S->nv, vcap), nq = dn(&S->nq, qcap);
+    const DevN nq = dn(&S->nq, qcap);
     const int32_t* quads = static_cast<int32_t*>(ctx->quads[ctx->cur].p);
     const int32_t* twin = static_cast<int32_t*>(ctx->twin.p);
     const uint8_t* flag = static_cast<uint8_t*>(ctx->flag.p);
@@ -1214,24 +1137,109 @@ void simplify3333(dmc_context* ctx, bool last) {
     check_launch(ctx, "mark3333");
     uint32_t* newQ = ensure<uint32_t>(ctx, ctx->newQ, qcap);
     scan_pair(ctx, scan_job(ScanKeepMap{{rflag}}, newQ, nq, &S->qn), kept_vertices_job(ctx, vflag));
-    uint32_t* newv = compact_vertices(ctx, vflag, nullptr, true);
-    int32_t* q2 = ensure<int32_t>(ctx, ctx->quads[1 - ctx->cur], 4 * qcap);
+    uint32_t* newv = compact_vertices(ctx, vflag, nullptr);
     int32_t* vmap = ensure<int32_t>(ctx, ctx->vmap, vcap);
-    remap_bounds(ctx, ctx->qbound, newQ, &S->nq, &S->qn);
-    // the dropped quadrilaterals, whose corners are the changed vertices
-    int32_t* dlist = ensure<int32_t>(ctx, ctx->mlist, qcap);
-    launch(ctx, "k_list_flagged", k_list_flagged, dim3(gq), dim3(kBlock), (const uint8_t*)rflag,
-           (const int32_t*)newQ, nq, dlist);
-    Carry c = carry_begin(ctx, newQ, last);
     launch(ctx, "k_vmap3333", k_vmap3333, dim3(grid_for(ctx, vcap)), dim3(kBlock), (const uint8_t*)vflag,
-           (const uint32_t*)newv, S, vmap, static_cast<const uint32_t*>(ctx->deg.p),
-           static_cast<const int32_t*>(ctx->hev.p), c.qmap, c.deg_n, c.hev_n, carry_clears(ctx, c));
-    launch(ctx, "k_changed3333", k_changed3333, dim3(gq), dim3(kBlock), quads, (const int32_t*)dlist,
-           (const Sizes*)S, (const int32_t*)vmap, const_cast<uint8_t*>(c.cflag), c.deg_n, c.hev_n);
-    launch(ctx, "k_compact_quads3333", k_compact_quads3333, dim3(gq), dim3(kBlock), quads, (const Sizes*)S,
-           (const uint8_t*)p3333, (const int32_t*)vtwin, (const int32_t*)vmap, q2, c);
-    check_launch(ctx, "k_compact_quads3333");
-    carry_end(ctx, c, vmap);
+           (const uint32_t*)newv, (const Sizes*)S, vmap);
+    compact_quads(ctx, newQ, vmap, p3333, vtwin);
+}
+
+// ---------------------------------------------------------------------------
+// simplifications on the live mesh
+// ---------------------------------------------------------------------------
+Live live_mesh(dmc_context* ctx) {
+    const int64_t vcap = ctx->vcap, qcap = ctx->qcap;
+    Live m{};
+    m.quads = static_cast<int32_t*>(ctx->quads[ctx->cur].p);
+    m.twin = static_cast<int32_t*>(ctx->twin.p);
+    m.flag = static_cast<uint8_t*>(ctx->flag.p);
+    m.hev = static_cast<int32_t*>(ctx->hev.p);
+    m.val = static_cast<int32_t*>(ctx->val.p);
+    m.dead = static_cast<uint8_t*>(ctx->dead.p);
+    m.vs = static_cast<uint8_t*>(ctx->vstate.p);
+    m.claim = static_cast<int32_t*>(ctx->lastR.p);
+    m.last = static_cast<int32_t*>(ctx->lastT.p);
+    m.pos = static_cast<double*>(ctx->pos[ctx->pcur].p);
+    m.nrm = static_cast<double*>(ctx->nrm[ctx->pcur].p);
+    m.p = ensure<uint8_t>(ctx, ctx->p, qcap);
+    m.em = ensure<uint8_t>(ctx, ctx->em, qcap);
+    m.list = ensure<uint32_t>(ctx, ctx->mlist, qcap);
+    m.irr = ensure<uint32_t>(ctx, ctx->irr, qcap);
+    m.head = ensure<int32_t>(ctx, ctx->head, vcap);
+    m.ent = ensure<int4>(ctx, ctx->ent, 4 * qcap);
+    m.frame = ensure<int4>(ctx, ctx->frame, 2 * qcap);
+    m.recs = static_cast<BndRec*>(ctx->bndrec.p);
+    m.reccap = (uint32_t)ctx->reccap;
+    m.S = dsizes(ctx);
+    m.vst = ctx->nvol > 1 ? static_cast<unsigned long long*>(ctx->vhe.p) : nullptr;
+    m.qb = static_cast<const int64_t*>(ctx->qbound.p);
+    m.nvol = ctx->nvol;
+    return m;
+}
+
+// Blocks of the kernels that gather a stage's list (a contiguous share of the
+// faces each): one add on the list's counter per block and 768 entries.
+constexpr int kListBlocks = 4096;
+
+void stage_rest(dmc_context* ctx, const Live& m, bool is3333) {
+    const int64_t qcap = ctx->qcap;
+    launch(ctx, "k_stage_rewrite", k_stage_rewrite, dim3(grid_for(ctx, qcap)), dim3(kBlock), m, is3333 ? 1 : 0);
+    launch(ctx, "k_stage_pair", k_stage_pair, dim3(grid_for(ctx, qcap)), dim3(kBlock), m);
+    check_launch(ctx, "stage");
+}
+
+void stage_3x3y(dmc_context* ctx, Live& m, bool colored) {
+    m.stage++;
+    const int64_t qcap = ctx->qcap;
+    if (colored) color_faces(ctx);
+    // lists of merging faces are sized by the faces (a launch only needs to
+    // cover them)
+    const int gq = grid_for(ctx, qcap), gl = grid_for(ctx, qcap / 4 + 1);
+    launch(ctx, "k_stage_mark", k_stage_mark, dim3(gq), dim3(kBlock), m);
+    launch(ctx, "k_stage_claim", k_stage_claim, dim3(grid_for(ctx, qcap, kBlock, kListBlocks)), dim3(kBlock), m,
+           colored ? static_cast<const uint8_t*>(ctx->colors.p) : nullptr);
+    launch(ctx, "k_stage_sort", k_stage_sort, dim3(gl), dim3(kBlock), m);
+    launch(ctx, "k_stage_merge", k_stage_merge, dim3(gl), dim3(kBlock), m);
+    launch(ctx, "k_stage_irregular", k_stage_irregular, dim3(gl), dim3(kBlock), m);
+    stage_rest(ctx, m, false);
+}
+
+void stage_3333(dmc_context* ctx, Live& m) {
+    m.stage++;
+    const int64_t qcap = ctx->qcap;
+    const int gl = grid_for(ctx, qcap / 4 + 1);
+    launch(ctx, "k_stage_mark3333", k_stage_mark3333, dim3(grid_for(ctx, qcap, kBlock, kListBlocks)), dim3(kBlock), m);
+    launch(ctx, "k_stage_cut3333", k_stage_cut3333, dim3(gl), dim3(kBlock), m);
+    launch(ctx, "k_stage_irregular", k_stage_irregular3333, dim3(gl), dim3(kBlock), m);
+    stage_rest(ctx, m, true);
+}
+
+// The one compaction: maps of the kept vertices and live faces, then both.
+void compact_live(dmc_context* ctx, const Live& m) {
+    const int64_t vcap = ctx->vcap, qcap = ctx->qcap;
+    Sizes* S = dsizes(ctx);
+    uint32_t* vmap = ensure<uint32_t>(ctx, ctx->newV, vcap);
+    uint32_t* qmap = ensure<uint32_t>(ctx, ctx->newQ, qcap);
+    scan_pair(ctx, scan_job(ScanKeepMap{{m.dead}}, qmap, dn(&S->nq, qcap), &S->qn),
+              scan_job(ScanUnclaimed{m.claim}, vmap, dn(&S->nv, vcap), &S->nn));
+    remap_bounds(ctx, ctx->vbound, vmap, &S->nv, &S->nn);
+    remap_bounds(ctx, ctx->qbound, qmap, &S->nq, &S->qn);
+    double* pos2 = ensure<double>(ctx, ctx->pos[1 - ctx->pcur], 3 * vcap);
+    double* nrm2 = ensure<double>(ctx, ctx->nrm[1 - ctx->pcur], 3 * vcap);
+    int32_t* quads2 = ensure<int32_t>(ctx, ctx->quads[1 - ctx->cur], 4 * qcap);
+    int32_t* twin2 = ensure<int32_t>(ctx, ctx->twin2, 4 * qcap);
+    uint8_t* flag2 = ensure<uint8_t>(ctx, ctx->flag2, 4 * qcap);
+    int32_t* hev2 = ensure<int32_t>(ctx, ctx->hev2, vcap);
+    BndRec* recs2 = ensure<BndRec>(ctx, ctx->bndrec2, ctx->reccap);
+    const int32_t *vm = reinterpret_cast<const int32_t*>(vmap), *qm = reinterpret_cast<const int32_t*>(qmap);
+    launch(ctx, "k_final_vertices", k_final_vertices, dim3(grid_for(ctx, vcap)), dim3(kBlock), m, vm, qm, pos2, nrm2,
+           hev2, recs2);
+    launch(ctx, "k_final_faces", k_final_faces, dim3(grid_for(ctx, qcap)), dim3(kBlock), m, vm, qm, quads2, twin2,
+           flag2, hev2);
+    check_launch(ctx, "compaction");
+    swap_pairs(ctx);
+    ctx->cur = 1 - ctx->cur;
+    ctx->pcur = 1 - ctx->pcur;
 }
 
 void clear_timing(dmc_context* ctx) {
@@ -1375,25 +1383,33 @@ void run_tmc(dmc_context* ctx, const std::vector<HostVol>& hv) {
 void enqueue_pass(dmc_context* ctx, const SweepPlan& P, int field_type, uint32_t flags) {
     const int n = ctx->nvol;
     ctx->commit_pending = false;
-    const bool final_build = (flags & DMC_SIMPLIFY_ALL) == 0;
-    if (field_type == DMC_FIELD_F32) run_cells<float>(ctx, P, final_build);
-    else run_cells<double>(ctx, P, final_build);
-    const bool iso = (flags & DMC_SIMPLIFY_3X3Y_ISOLATED) != 0, p3333 = (flags & DMC_SIMPLIFY_3333) != 0;
+    const bool simplify = (flags & DMC_SIMPLIFY_ALL) != 0, live = simplify && !ctx->force_generic;
+    if (field_type == DMC_FIELD_F32) run_cells<float>(ctx, P, live);
+    else run_cells<double>(ctx, P, live);
+    Live m{};
+    if (live) m = live_mesh(ctx);
     if (flags & DMC_SIMPLIFY_3X3Y_COLOR) {
         mark(ctx, "p3x3y_color");
-        simplify3x3y(ctx, true, !iso && !p3333);
+        if (live) stage_3x3y(ctx, m, true);
+        else simplify3x3y(ctx, true);
     }
-    if (iso) {
+    if (flags & DMC_SIMPLIFY_3X3Y_ISOLATED) {
         mark(ctx, "p3x3y_isolated");
-        simplify3x3y(ctx, false, !p3333);
+        if (live) stage_3x3y(ctx, m, false);
+        else simplify3x3y(ctx, false);
     }
-    if (p3333) {
+    if (flags & DMC_SIMPLIFY_3333) {
         mark(ctx, "p3333");
-        simplify3333(ctx, true);
+        if (live) stage_3333(ctx, m);
+        else simplify3333(ctx);
     }
     mark(ctx, "halfedges");
-    build_halfedges(ctx, true);
-    gather_vertices(ctx);
+    if (live) compact_live(ctx, m);
+    if (ctx->force_generic) {
+        build_halfedges(ctx, true);
+        gather_vertices(ctx);
+    }
+    finish_halfedges(ctx, live);
     Sizes* S = dsizes(ctx);
     int32_t* tris = nullptr;
     if (flags & DMC_TRIANGLES) {
@@ -1466,8 +1482,8 @@ bool finish_pass(dmc_context* ctx, const std::vector<HostVol>& hv, uint32_t flag
             ctx->rarea[k] = std::max(ctx->rarea[k], cnt[k] / area_of(c));
         }
     }
-    if (hs.need_generic) {
-        // a build needed generic rows: the same pass again with them
+    if (!ctx->force_generic && (hs.need_generic || hs.unresolved)) {
+        // the live mesh could not express the pass: the same stage by stage
         ctx->force_generic = true;
         if (!hs.ovf) return false;
     }
@@ -1611,7 +1627,6 @@ void save_post(dmc_context* ctx, dmc_context::PassGraph& g) {
     g.pcur = ctx->pcur;
     g.scur = ctx->scur;
     g.slots = ctx->slots;
-    g.ready = ctx->ready;
     g.swapped = pair_order(ctx);
 }
 
@@ -1620,7 +1635,6 @@ void load_post(dmc_context* ctx, const dmc_context::PassGraph& g) {
     ctx->pcur = g.pcur;
     ctx->scur = g.scur;
     ctx->slots = g.slots;
-    ctx->ready = g.ready;
     set_pair_order(ctx, g.swapped);
 }
 
@@ -1643,8 +1657,6 @@ void run_pass(dmc_context* ctx, const SweepPlan& P, int field_type, uint32_t fla
         for (auto& g : ctx->graphs) {
             if (g.key != key) continue;
             upload_vtab(ctx, P);
-            if (ctx->off.p > ctx->off2.p) std::swap(ctx->off, ctx->off2);
-            if (ctx->adj.p > ctx->adj2.p) std::swap(ctx->adj, ctx->adj2);
             HIPC(ctx, hipGraphLaunch(g.exec, ctx->stream));
             load_post(ctx, g);
             g.use = ++ctx->graph_clock;

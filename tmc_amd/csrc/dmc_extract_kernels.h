@@ -627,7 +627,16 @@ __device__ __forceinline__ double div_by(double x, double c, double rc) {
     return r;
 }
 
-// Position, normal and interior-edge count of the vertex at local
+// What the simplifications keep per vertex, initialised with the vertex
+// (val == null: none follow).
+struct VertexOut {
+    int32_t* val;
+    int32_t* claim;
+    int32_t* last;
+    uint8_t* vs;
+};
+
+// Position, normal and out-degree of the vertex at local
 // coordinates p of cell (i, j, k) (cpp_dmc/DualMarchingCubes.cpp:160-171,
 // UniformGrid.h:286-305).  The normal is the trilinear blend of the eight
 // corner gradients, normalised.  Corner gradients are the supplied ones, or
@@ -637,8 +646,7 @@ template <class T>
 __device__ __forceinline__ void store_vertex(const VolDesc& V, int i, int j, int k, const CornerRef& Fc,
                                              const OuterValues<T>& o, const double p[3], uint32_t code, uint32_t aux,
                                              int t, uint32_t out, double* __restrict__ vpos,
-                                             double* __restrict__ vnrm, uint32_t* __restrict__ vdeg,
-                                             uint32_t* __restrict__ varr) {
+                                             double* __restrict__ vnrm, const VertexOut& vo) {
     const Dims& d = V.d;
     const double u = p[0], v = p[1], ww = p[2];
     const double dx2[3] = {2 * V.geo.dx, 2 * V.geo.dy, 2 * V.geo.dz};
@@ -687,15 +695,20 @@ __device__ __forceinline__ void store_vertex(const VolDesc& V, int i, int j, int
     vn[0] = div_by(n[0], s, rs);
     vn[1] = div_by(n[1], s, rs);
     vn[2] = div_by(n[2], s, rs);
-    vdeg[out] = (uint32_t)__popc(contour_spread(code >> 8, (unsigned)t) & aux);
-    if (varr) varr[out] = 0u;   // k_quads counts the boundary halfedges that end here
+    if (vo.val) {
+        // out-degree; k_quads adds the boundary halfedges that end here
+        vo.val[out] = __popc(contour_spread(code >> 8, (unsigned)t) & aux);
+        vo.claim[out] = 0;
+        vo.last[out] = 0;
+        vo.vs[out] = 0;
+    }
 }
 
 template <class T, int kUnroll>
 __device__ __forceinline__ void vertices_run(const VolTable& vt, const uint4* __restrict__ rec,
                                              const uint32_t* __restrict__ grpV, DevN dA,
                                              double* __restrict__ vpos, double* __restrict__ vnrm,
-                                             uint32_t* __restrict__ vdeg, uint32_t* __restrict__ varr,
+                                             VertexOut vo,
                                              uint32_t* __restrict__ slow, unsigned long long* qhead) {
     static_assert(kBlock == kBoxStride && kBlock == kCornerStride, "LDS columns are one per thread");
     const int64_t A = dA.get();
@@ -750,7 +763,7 @@ __device__ __forceinline__ void vertices_run(const VolTable& vt, const uint4* __
                     break;
                 }
                 if (!((used >> t) & 1u)) continue;
-                store_vertex<T>(V, i, j, k, Fc, o, p, code, aux, t, out, vpos, vnrm, vdeg, varr);
+                store_vertex<T>(V, i, j, k, Fc, o, p, code, aux, t, out, vpos, vnrm, vo);
                 out++;
             }
         }
@@ -775,9 +788,9 @@ template <class T>
 __global__ void __launch_bounds__(kBlock) TMC_VERTICES_ATTR k_vertices(VolTable vt, const uint4* __restrict__ rec,
                                                       const uint32_t* __restrict__ grpV, DevN dA,
                                                       double* __restrict__ vpos, double* __restrict__ vnrm,
-                                                      uint32_t* __restrict__ vdeg, uint32_t* __restrict__ varr,
+                                                      VertexOut vo,
                                                       uint32_t* __restrict__ slow, unsigned long long* qhead) {
-    vertices_run<T, 7>(vt, rec, grpV, dA, vpos, vnrm, vdeg, varr, slow, qhead);
+    vertices_run<T, 7>(vt, rec, grpV, dA, vpos, vnrm, vo, slow, qhead);
 }
 
 // K3 for larger passes: samples one at a time, which fits 3 waves per SIMD
@@ -788,10 +801,9 @@ __global__ void __launch_bounds__(kBlock) TMC_VERTICES_ATTR k_vertices(VolTable 
 template <class T>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 3)))
 k_vertices_wide(VolTable vt, const uint4* __restrict__ rec, const uint32_t* __restrict__ grpV, DevN dA,
-                double* __restrict__ vpos, double* __restrict__ vnrm, uint32_t* __restrict__ vdeg,
-                uint32_t* __restrict__ varr, uint32_t* __restrict__ slow,
+                double* __restrict__ vpos, double* __restrict__ vnrm, VertexOut vo, uint32_t* __restrict__ slow,
                 unsigned long long* qhead) {
-    vertices_run<T, 1>(vt, rec, grpV, dA, vpos, vnrm, vdeg, varr, slow, qhead);
+    vertices_run<T, 1>(vt, rec, grpV, dA, vpos, vnrm, vo, slow, qhead);
 }
 
 // General path of K3 for the cells k_vertices deferred: every contour is
@@ -802,7 +814,7 @@ __global__ void __launch_bounds__(kBlock) k_vertices_slow(VolTable vt, const uin
                                                           const uint32_t* __restrict__ grpV,
                                                           const uint32_t* __restrict__ slow,
                                                           double* __restrict__ vpos, double* __restrict__ vnrm,
-                                                          uint32_t* __restrict__ vdeg, uint32_t* __restrict__ varr,
+                                                          VertexOut vo,
                                                           VolStat* __restrict__ vstat) {
     __shared__ float boxes[kBoxFloats * kBoxStride];
     __shared__ double corners[8 * kCornerStride];
@@ -847,7 +859,7 @@ __global__ void __launch_bounds__(kBlock) k_vertices_slow(VolTable vt, const uin
                 }
             }
             if (!((used >> t) & 1u)) continue;
-            store_vertex<T>(V, i, j, k, Fc, o, p, code, aux, t, out, vpos, vnrm, vdeg, varr);
+            store_vertex<T>(V, i, j, k, Fc, o, p, code, aux, t, out, vpos, vnrm, vo);
             out++;
         }
     }
@@ -922,9 +934,11 @@ __global__ void k_cell_guard(Sizes* S, uint64_t acap, uint64_t vcap, uint64_t qc
         slow[0] = 0;   // k_vertices' count of deferred cells
         const uint32_t o = (S->A > acap ? 1u : 0u) | (S->V > vcap ? 2u : 0u) | (S->Q > qcap ? 4u : 0u);
         S->ovf |= o;
-        S->acnt = o ? 0 : S->A;
-        S->nv = o ? 0 : S->V;
-        S->nq = o ? 0 : S->Q;
+        // (a cell on no contour leaves vertices that no one writes)
+        const bool run = !o && !S->open_cells;
+        S->acnt = run ? S->A : 0;
+        S->nv = run ? S->V : 0;
+        S->nq = run ? S->Q : 0;
     }
 }
 

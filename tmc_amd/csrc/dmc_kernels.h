@@ -81,20 +81,17 @@ struct Sizes {
     uint64_t nv, nq;             // the live mesh
     uint64_t nn, qn;             // vertices / quadrilaterals a compaction keeps
     uint64_t tot;                // a scan total no one else reads
-    uint64_t hq;                 // halfedges of the mesh a compaction leaves (4 qn)
-    uint64_t naff;               // halfedges a compaction left to pair again
     unsigned long long qhead;    // work queue of k_vertices: the next chunk of active cells
     HeStats he;                  // the last halfedge build
     uint32_t ovf;                // capacities exceeded: 1 active cells, 2 vertices, 4 quads, 8 3-face records
     uint32_t unresolved;         // quadrilaterals with an unresolved neighbour cell
     uint32_t zero;               // vertices of valence 0 (all valence passes)
     uint32_t open_cells;         // cells with an interior edge on no contour (NaN deciders)
-    uint32_t need_generic;       // a build needed generic rows the pass did not launch: run it again with them
-    uint32_t incr_ok;            // the build before the compaction saw no invalid vertex reference
-    uint32_t cbad;               // invalid references the last quadrilateral compaction met
-    uint32_t nrec;               // 3-face edge records of the current build
-    uint32_t nrec_prev;          // ... of the build before (carried over by a compaction)
+    uint32_t need_generic;       // the pass met what only a compaction and generic rows per stage express: run it so
+    uint32_t nrec;               // 3-face edge records of the current build (dropped ones among them)
+    uint32_t nrec_final;         // ... under the compacted numbers
     uint32_t recmax;             // most 3-face records any build of the pass wrote (capacity planning)
+    uint32_t nlist[4], nirr[4], nent[4];   // per stage: merging faces, irregular ones, halfedges to pair again
     uint32_t colors[48];         // colour classes: counts [0, 24), starts [24, 48)
     unsigned long long cpart[kContourParts];   // a single volume's contour count, in parts
     unsigned long long hep[kHeParts][3];      // the build's flagged halfedges per slot: groups of 4, of 3, error groups
@@ -212,6 +209,24 @@ struct ScanKeep {
 // rank is ~map).  The kept count before item i is map[i] or i - ~map[i].
 struct ScanKeepMap : ScanKeep {
     static constexpr bool kMap = true;
+};
+
+// The same over claims (dmc_simplify_kernels.h): a vertex is kept where its
+// claim is below the first stage's.
+struct ScanUnclaimed {
+    static constexpr bool kMap = true;
+    const int32_t* p;
+    __device__ __forceinline__ uint32_t at(int64_t i) const { return p[i] < (1 << 29) ? 1u : 0u; }
+    __device__ __forceinline__ void vec16(int64_t base, uint32_t v[kScanIPT]) const {
+#pragma unroll
+        for (int q = 0; q < kScanIPT / 4; q++) {
+            const int4 t = reinterpret_cast<const int4*>(p + base)[q];
+            v[4 * q] = t.x < (1 << 29);
+            v[4 * q + 1] = t.y < (1 << 29);
+            v[4 * q + 2] = t.z < (1 << 29);
+            v[4 * q + 3] = t.w < (1 << 29);
+        }
+    }
 };
 
 template <class In>

@@ -244,7 +244,7 @@ __global__ void __launch_bounds__(kBlock) k_he_twins(const int32_t* __restrict__
                                                       uint32_t* __restrict__ arr, unsigned long long (*hep)[3],
                                                       BndRec* __restrict__ recs, uint32_t* nrec, uint32_t reccap,
                                                       uint32_t* ovf, const int64_t* __restrict__ qb, int nvol,
-                                                      unsigned long long* __restrict__ vst) {
+                                                      unsigned long long* __restrict__ vst, int final_pass) {
     static_assert(kBlock % 4 == 0, "quads must not straddle blocks");
     const int64_t nhe = 4 * (int64_t)S->nq, nv = (int64_t)S->nv;
     HeCount cnt;
@@ -343,7 +343,7 @@ __global__ void __launch_bounds__(kBlock) k_he_twins(const int32_t* __restrict__
         uint8_t fl;
         twin_rule(quads, c, g, h, tw, fl);
         twin[h] = tw;
-        flag[h] = fl;
+        flag[h] = final_pass && (fl & kFlagErr) ? 0 : fl;
         // valence: a boundary halfedge adds one to the vertex it ends at
         if (tw == -1 && arr && vid_ok(b, nv)) atomicAdd(&arr[b], 1u);
         cnt.add(fl);
@@ -351,33 +351,6 @@ __global__ void __launch_bounds__(kBlock) k_he_twins(const int32_t* __restrict__
         if (c == 3 && g[0] == h) put_record(recs, nrec, reccap, ovf, three_record(quads, g, h));
     }
     cnt.flush(hep);
-}
-
-// The 3-face overrides of he_v (cpp_dmc/DualMarchingCubes.cpp:603-637) from
-// the final build's records: pass 0 finds each lone vertex's largest key,
-// pass 1 lets that record write.  ovr (2 words per vertex) starts at 0.
-__global__ void __launch_bounds__(kBlock) k_three_apply(const BndRec* __restrict__ recs, const Sizes* S,
-                                                         uint32_t reccap, const int32_t* __restrict__ quads,
-                                                         unsigned long long* __restrict__ ovr, int pass,
-                                                         int32_t* __restrict__ he_v) {
-    const int64_t n = S->nrec < reccap ? S->nrec : reccap, nv = (int64_t)S->nv;
-    TMC_GRID_STRIDE(i, n) {
-        const BndRec r = recs[i];
-        const int32_t vl = quads[r.lone];
-        if (!vid_ok(vl, nv)) continue;
-        if (pass == 0) atomicMax(&ovr[vl], r.key + 1ull);
-        else if (ovr[vl] == r.key + 1ull) he_v[vl] = r.lone;
-    }
-}
-
-// The final mesh's flags as the reference leaves them: the markers of
-// groups of more than 4 faces cleared (only when there are any).
-__global__ void __launch_bounds__(kBlock) k_strip_flags(const Sizes* S, uint8_t* __restrict__ flag) {
-    if (he_errors(S) == 0) return;
-    const int64_t nhe = 4 * (int64_t)S->nq;
-    TMC_GRID_STRIDE(h, nhe) {
-        if (flag[h] & kFlagErr) flag[h] = 0;
-    }
 }
 
 // Arrays the simplification after a halfedge build needs cleared, cleared
@@ -821,456 +794,65 @@ __global__ void __launch_bounds__(kBlock) k_twin3333(const int32_t* __restrict__
     }
 }
 
-// Opens a compaction's carry (thread 0 of the vertex-map kernel, whose other
-// threads do not read these): whether the build it starts from met invalid
-// vertex references, and fresh counters for the carried build.
-__device__ __forceinline__ void open_carry(Sizes* S) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    S->incr_ok = S->he.bad == 0u ? 1u : 0u;
-    he_clear(S);
-    S->nrec_prev = S->nrec;
-    S->recmax = S->nrec > S->recmax ? S->nrec : S->recmax;
-    S->nrec = 0;
-    S->hq = 4 * S->qn;
-    S->cbad = 0;
-}
-
-// A kept vertex x hands its out-degree and he_v (renumbered by the face
-// map) to its new id y; the changed vertices and those that lost a corner
-// are corrected afterwards (k_changed*).
-__device__ __forceinline__ void carry_vertex(int64_t x, int32_t y, int64_t nn, const uint32_t* __restrict__ deg,
-                                             const int32_t* __restrict__ hev, const int32_t* __restrict__ qmap,
-                                             uint32_t* __restrict__ deg_n, int32_t* __restrict__ hev_n) {
-    if (!vid_ok(y, nn)) return;
-    deg_n[y] = deg[x];
-    const int32_t e = hev[x];
-    const int32_t m = e < 0 ? -1 : qmap[e >> 2];
-    hev_n[y] = m < 0 ? -1 : 4 * m + (e & 3);
-}
-
-// The zeroed state of a carry, cleared by the vertex map kernel that starts
-// it (which reads none of it): the changed-vertex marks (whole words, set
-// with word atomics), the new vertices' arrivals and per-origin counts, and
-// the per-turn counts of the compaction.
-struct CarryClears {
-    uint32_t* cflag;
-    int64_t cwords;
-    uint32_t* arr;
-    uint32_t* cnt;
-    uint32_t* bcount;
-    int64_t turns;
-};
-
-__device__ __forceinline__ void carry_clear(const CarryClears& z, int64_t nn) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    for (int64_t i = t0; i < z.cwords; i += stride) z.cflag[i] = 0u;
-    for (int64_t i = t0; i < nn; i += stride) {
-        z.arr[i] = 0u;
-        z.cnt[i] = 0u;
-    }
-    for (int64_t i = t0; i < z.turns; i += stride) z.bcount[i] = 0u;
-}
-
+// The compactions of a pass run stage by stage (generic rows).
 // 3X3Y: vmap[x] = vsecond[x] for a kept x (its new id after the vertex
-// compaction), vsecond[vsecond[x]] for a removed one (its target's); and the
-// kept vertices' carry.
+// compaction), vsecond[vsecond[x]] for a removed one (its target's).
 __global__ void __launch_bounds__(kBlock) k_vmap3x3y(const uint8_t* __restrict__ vfirst,
-                                                      const int32_t* __restrict__ vsecond, Sizes* S,
-                                                      int32_t* __restrict__ vmap, const uint32_t* __restrict__ deg,
-                                                      const int32_t* __restrict__ hev,
-                                                      const int32_t* __restrict__ qmap, uint32_t* __restrict__ deg_n,
-                                                      int32_t* __restrict__ hev_n, CarryClears z) {
-    const int64_t nv = (int64_t)S->nv, nn = (int64_t)S->nn;
-    open_carry(S);
-    carry_clear(z, nn);
+                                                      const int32_t* __restrict__ vsecond, const Sizes* S,
+                                                      int32_t* __restrict__ vmap) {
+    const int64_t nv = (int64_t)S->nv;
     TMC_GRID_STRIDE(x, nv) {
         int32_t y = vsecond[x];
-        const bool removed = vfirst[x] != 0;
-        if (removed) y = vid_ok(y, nv) ? vsecond[y] : -1;
+        if (vfirst[x] != 0) y = vid_ok(y, nv) ? vsecond[y] : -1;
         vmap[x] = y;
-        if (!removed) carry_vertex(x, y, nn, deg, hev, qmap, deg_n, hev_n);
     }
 }
 
-// 3333: vmap[x] = new id of a kept x, -1 for a removed one; and the kept
-// vertices' carry.
+// 3333: vmap[x] = new id of a kept x, -1 for a removed one.
 __global__ void __launch_bounds__(kBlock) k_vmap3333(const uint8_t* __restrict__ vflag,
-                                                      const uint32_t* __restrict__ newv, Sizes* S,
-                                                      int32_t* __restrict__ vmap, const uint32_t* __restrict__ deg,
-                                                      const int32_t* __restrict__ hev,
-                                                      const int32_t* __restrict__ qmap, uint32_t* __restrict__ deg_n,
-                                                      int32_t* __restrict__ hev_n, CarryClears z) {
-    const int64_t nv = (int64_t)S->nv, nn = (int64_t)S->nn;
-    open_carry(S);
-    carry_clear(z, nn);
-    TMC_GRID_STRIDE(x, nv) {
-        const bool removed = vflag[x] != 0;
-        const int32_t y = removed ? -1 : (int32_t)newv[x];
-        vmap[x] = y;
-        if (!removed) carry_vertex(x, y, nn, deg, hev, qmap, deg_n, hev_n);
-    }
+                                                      const uint32_t* __restrict__ newv, const Sizes* S,
+                                                      int32_t* __restrict__ vmap) {
+    const int64_t nv = (int64_t)S->nv;
+    TMC_GRID_STRIDE(x, nv) vmap[x] = vflag[x] != 0 ? -1 : (int32_t)newv[x];
 }
 
-// ---------------------------------------------------------------------------
-// The halfedges of a compacted mesh, carried over from the build before it.
-//
-// A compaction keeps face f as face newq[f] (unless dropped) with corner k
-// in place, each vertex renamed to its new id.  Call a new vertex changed
-// (cflag bit 1) if a removed vertex maps to it, or if it is the image of a
-// corner of a dropped face that the compaction moved or merged (3X3Y: the
-// two valence-3 corners of a merging face; 3333: every kept corner of a
-// dropped face, which covers the pattern face's new corners too).  For a
-// new edge {a, b} with neither end changed, a and b each have exactly one
-// preimage x, y (kept vertices), every halfedge on {x, y} sits in a
-// surviving face that is not a pattern face, and every halfedge on {a, b}
-// comes from one of them: the edge's group is the old group renumbered by
-// newq, which keeps its order, so its twins (renumbered) and flags carry
-// over, and so does its 3-face record.  Halfedges with a changed end are
-// paired again through rows of those halfedges only (keyed by origin): a
-// group with a changed end has all its members there.
-//
-// Out-degree and he_v (the largest halfedge leaving the vertex) carry over
-// for a vertex with no corner in a dropped face.  A changed vertex has all
-// its out-halfedges in its row.  A vertex that only lost corners (the
-// valence >= 5 corners of a merging face) loses one out-halfedge per
-// corner, and takes he_v again (with atomics over its surviving
-// out-halfedges) only if its largest one was dropped (cflag bit 4).
-// ---------------------------------------------------------------------------
-struct Carry {
-    const int32_t* twin;          // the build before the compaction
-    const uint8_t* flag;
-    const int32_t* qmap;          // new index of each face; negative if dropped (ScanKeepMap)
-    const uint8_t* cflag;         // changed new vertices (bit 1), vertices whose he_v is taken again (bit 4)
-    int32_t* twin_n;              // the carried build
-    uint8_t* flag_n;
-    uint32_t* deg_n;
-    int32_t* hev_n;
-    uint32_t* arr;                // boundary arrivals per new vertex (valence)
-    uint8_t* aflag;               // new halfedges to pair again: 1 + rank in the origin's row, 0 if carried
-    uint32_t* cnt;                // ... per origin
-    uint32_t* bcount;             // ... per 256 old faces (a block's turn of the compaction loop)
-    Sizes* S;
-    unsigned long long* vst;      // per-volume counts (last compaction of a batch)
-    const int64_t* qb;            // first new face of each volume
-    int nvol;
-};
-
-// Mark a new vertex (bits of cflag, one byte per vertex, updated as words).
-__device__ __forceinline__ void mark_vertex(uint8_t* cflag, int32_t y, uint32_t bits) {
-    atomicOr(reinterpret_cast<uint32_t*>(cflag) + (y >> 2), bits << (8 * (y & 3)));
-}
-
-
-// A changed vertex: paired again, its out-degree and he_v from its row.
-__device__ __forceinline__ void mark_changed(uint8_t* cflag, uint32_t* deg_n, int32_t* hev_n, int32_t y) {
-    mark_vertex(cflag, y, 1u);
-    deg_n[y] = 0;
-    hev_n[y] = -1;
-}
-
-// 3X3Y: the merging faces (mlist, S->nq - S->qn of them).  The moved and
-// the dropped corner are changed.  The other two (valence >= 5, never moved)
-// each lose the halfedge they start in the face; if that was their largest,
-// their he_v is taken again over what survives (cflag bit 4).
-__global__ void __launch_bounds__(kBlock) k_changed3x3y(const int32_t* __restrict__ quads,
-                                                         const int32_t* __restrict__ mlist, const Sizes* S,
-                                                         const uint8_t* __restrict__ em,
-                                                         const int32_t* __restrict__ vmap,
-                                                         const int32_t* __restrict__ hev, uint8_t* __restrict__ cflag,
-                                                         uint32_t* __restrict__ deg_n, int32_t* __restrict__ hev_n) {
-    const int64_t n = (int64_t)(S->nq - S->qn), nv = (int64_t)S->nv, nn = (int64_t)S->nn;
-    TMC_GRID_STRIDE(i, n) {
-        const int32_t f = mlist[i];
-        const int4 q = reinterpret_cast<const int4*>(quads)[f];
-        const bool first = em[f] == 1;
-        const int32_t x[4] = {first ? q.x : q.y, first ? q.z : q.w, first ? q.y : q.x, first ? q.w : q.z};
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            if (!vid_ok(x[k], nv)) continue;
-            const int32_t y = vmap[x[k]];
-            if (!vid_ok(y, nn)) continue;
-            if (k < 2) {
-                mark_changed(cflag, deg_n, hev_n, y);
-            } else {
-                atomicSub(&deg_n[y], 1u);
-                if ((hev[x[k]] >> 2) == f) {
-                    mark_vertex(cflag, y, 4u);
-                    hev_n[y] = -1;
-                }
-            }
-        }
-    }
-}
-
-// 3333: the dropped faces (dlist, S->nq - S->qn of them); every kept corner
-// is changed.
-__global__ void __launch_bounds__(kBlock) k_changed3333(const int32_t* __restrict__ quads,
-                                                         const int32_t* __restrict__ dlist, const Sizes* S,
-                                                         const int32_t* __restrict__ vmap, uint8_t* __restrict__ cflag,
-                                                         uint32_t* __restrict__ deg_n, int32_t* __restrict__ hev_n) {
-    const int64_t n = (int64_t)(S->nq - S->qn), nv = (int64_t)S->nv, nn = (int64_t)S->nn;
-    TMC_GRID_STRIDE(i, n) {
-        const int4 q = reinterpret_cast<const int4*>(quads)[dlist[i]];
-        const int32_t x[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            if (!vid_ok(x[k], nv)) continue;
-            const int32_t y = vmap[x[k]];
-            if (vid_ok(y, nn)) mark_changed(cflag, deg_n, hev_n, y);
-        }
-    }
-}
-
-// The carry of surviving face f (new index nf, new corners r): every
-// halfedge either keeps its group (twin renumbered, flag, arrival) or is
-// flagged for pairing, with its rank in its origin's row (a rank past 253,
-// never met in practice, sends the next build to the generic rows).
-// Returns the number flagged.
-__device__ __forceinline__ uint32_t carry_face(const Carry& c, bool act, int64_t f, uint32_t nf, const int32_t r[4],
-                                               int64_t nn, HeCount& cnt) {
-    int32_t tw[4] = {-1, -1, -1, -1};
-    uint32_t fl = 0, af = 0, naff = 0;
-    if (act) {
-        const int4 t4 = reinterpret_cast<const int4*>(c.twin)[f];
-        const uint32_t f4 = reinterpret_cast<const uint32_t*>(c.flag)[f];
-        const int32_t t[4] = {t4.x, t4.y, t4.z, t4.w};
-        uint8_t cf[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) cf[k] = vid_ok(r[k], nn) ? c.cflag[r[k]] : 0;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int32_t a = r[k], b = r[(k + 1) & 3];
-            const int32_t h = (int32_t)(4 * nf) + k;
-            if (!vid_ok(a, nn) || !vid_ok(b, nn)) continue;   // invalid ids: the next build starts over
-            const uint8_t ca = cf[k], cb = cf[(k + 1) & 3];
-            if (ca & 4u) atomicMax(&c.hev_n[a], h);   // its largest halfedge was dropped
-            if ((ca | cb) & 1u) {
-                const uint32_t rk = atomicAdd(&c.cnt[a], 1u);
-                if (rk >= 254u) atomicOr(&c.S->cbad, 0x80000000u);
-                af |= (rk < 254u ? rk + 1u : 255u) << (8 * k);
-                naff++;
-                continue;
-            }
-            const int32_t nq = t[k] >= 0 ? c.qmap[t[k] >> 2] : -1;
-            tw[k] = nq < 0 ? -1 : 4 * nq + (t[k] & 3);
-            const uint8_t x = (uint8_t)(f4 >> (8 * k));
-            fl |= (uint32_t)x << (8 * k);
-            if (tw[k] < 0) atomicAdd(&c.arr[b], 1u);
-            cnt.add(x);
-            vol_count(c.vst, c.qb, c.nvol, h, x);
-        }
-        reinterpret_cast<int4*>(c.twin_n)[nf] = make_int4(tw[0], tw[1], tw[2], tw[3]);
-        reinterpret_cast<uint32_t*>(c.flag_n)[nf] = fl;
-        reinterpret_cast<uint32_t*>(c.aflag)[nf] = af;
-    }
-    return naff;
-}
-
-// The block's count of flagged halfedges for its turn j of the compaction
-// loop (every thread of the block calls this).
-__device__ __forceinline__ void block_count(uint32_t* __restrict__ bcount, int64_t j, uint32_t k) {
-    __shared__ uint32_t sm[kBlock / kWave];
-    const uint32_t w = wave_sum(k);
-    if ((threadIdx.x & (kWave - 1)) == 0) sm[threadIdx.x / kWave] = w;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t t = 0;
-        for (int i = 0; i < kBlock / kWave; i++) t += sm[i];
-        bcount[j] = t;
-    }
-    __syncthreads();
-}
-
-// removeQuadrilaterals3X3Y (cpp_dmc/DualMarchingCubes.cpp:1114-1137), with
-// the carry of the halfedges.  The vertex ids come from vmap (k_vmap3x3y):
+// removeQuadrilaterals3X3Y (cpp_dmc/DualMarchingCubes.cpp:1114-1137) and
+// removeQuadrilaterals3333 (:1320-1360, p3333 set): face f becomes face
+// qmap[f] (negative: dropped).  The vertex ids come from vmap, for 3X3Y
 // vm[vm[x]]-style lookups of a removed vertex x, exactly as the reference
-// composes them.  Blocks stride over the faces in whole turns of 256, each
-// turn writing its count of flagged halfedges.
-__global__ void __launch_bounds__(kBlock) k_compact_quads3x3y(const int32_t* __restrict__ quads, const Sizes* S,
-                                                               const int32_t* __restrict__ vmap,
-                                                               int32_t* __restrict__ quads2, Carry c) {
-    const int64_t nq = (int64_t)S->nq, nv = (int64_t)S->nv, nn = (int64_t)S->nn;
-    HeCount cnt;
-    for (int64_t f0 = (int64_t)blockIdx.x * kBlock; f0 < nq; f0 += (int64_t)gridDim.x * kBlock) {
-        const int64_t f = f0 + threadIdx.x;
-        const int32_t m = f < nq ? c.qmap[f] : -1;
-        const bool act = m >= 0;
-        int32_t r[4] = {-1, -1, -1, -1};
-        const uint32_t nf = act ? (uint32_t)m : 0u;
-        if (act) {
-            const int4 q = reinterpret_cast<const int4*>(quads)[f];
-            const int32_t x[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-            for (int k = 0; k < 4; k++) r[k] = vid_ok(x[k], nv) ? vmap[x[k]] : -1;
-#pragma unroll
-            for (int k = 0; k < 4; k++)
-                if (r[k] < 0) atomicAdd(&c.S->cbad, 1u);
-            reinterpret_cast<int4*>(quads2)[nf] = make_int4(r[0], r[1], r[2], r[3]);
-        }
-        block_count(c.bcount, f0 / kBlock, carry_face(c, act, f, nf, r, nn, cnt));
-    }
-    cnt.flush(c.S->hep);
-}
-
-// removeQuadrilaterals3333 (cpp_dmc/DualMarchingCubes.cpp:1320-1360), with
-// the carry of the halfedges (a pattern face's halfedges all end at
-// changed vertices, so none of them is carried).
-__global__ void __launch_bounds__(kBlock) k_compact_quads3333(const int32_t* __restrict__ quads, const Sizes* S,
-                                                               const uint8_t* __restrict__ p3333,
-                                                               const int32_t* __restrict__ vtwin,
-                                                               const int32_t* __restrict__ vmap,
-                                                               int32_t* __restrict__ quads2, Carry c) {
-    const int64_t nq = (int64_t)S->nq, nv = (int64_t)S->nv, nn = (int64_t)S->nn;
-    HeCount cnt;
-    for (int64_t f0 = (int64_t)blockIdx.x * kBlock; f0 < nq; f0 += (int64_t)gridDim.x * kBlock) {
-        const int64_t f = f0 + threadIdx.x;
-        const int32_t m = f < nq ? c.qmap[f] : -1;
-        const bool act = m >= 0;
-        int32_t r[4] = {-1, -1, -1, -1};
-        const uint32_t nf = act ? (uint32_t)m : 0u;
-        if (act) {
-            const int4 q = reinterpret_cast<const int4*>(quads)[f];
-            int32_t x[4] = {q.x, q.y, q.z, q.w};
-            if (p3333[f]) {
-#pragma unroll
-                for (int k = 0; k < 4; k++)
-                    if (vid_ok(x[k], nv)) x[k] = vtwin[x[k]];
-            }
-            // vmap[x] = new id of a kept x, -1 for a removed one (k_vmap3333)
-#pragma unroll
-            for (int k = 0; k < 4; k++) r[k] = vid_ok(x[k], nv) ? vmap[x[k]] : -1;
-#pragma unroll
-            for (int k = 0; k < 4; k++)
-                if (r[k] < 0) atomicAdd(&c.S->cbad, 1u);
-            reinterpret_cast<int4*>(quads2)[nf] = make_int4(r[0], r[1], r[2], r[3]);
-        }
-        block_count(c.bcount, f0 / kBlock, carry_face(c, act, f, nf, r, nn, cnt));
-    }
-    cnt.flush(c.S->hep);
-}
-
-// The flagged halfedges as a dense list, and their rows by origin.  Walks
-// the old faces in the compaction's turns of 256: boff = exclusive scan of
-// the turns' counts, ranks inside a turn from a block scan.  aoff =
-// exclusive scan of the rows' counts; a halfedge's place in its row is the
-// rank its flag holds.
-__global__ void __launch_bounds__(kBlock) k_aff_scatter(const Sizes* S, const int32_t* __restrict__ qmap,
-                                                         const uint8_t* __restrict__ aflag,
-                                                         const uint32_t* __restrict__ bcount,
-                                                         const uint32_t* __restrict__ boff,
-                                                         const int32_t* __restrict__ quads,
-                                                         const uint32_t* __restrict__ aoff,
-                                                         int2* __restrict__ aadj, int32_t* __restrict__ alist) {
-    __shared__ uint32_t sm[kBlock / kWave + 1];
-    const int64_t nq = (int64_t)S->nq;
-    for (int64_t f0 = (int64_t)blockIdx.x * kBlock; f0 < nq; f0 += (int64_t)gridDim.x * kBlock) {
-        if (bcount[f0 / kBlock] == 0u) continue;   // a turn with nothing flagged (block-uniform)
-        const int64_t f = f0 + threadIdx.x;
-        const int32_t m = f < nq ? qmap[f] : -1;
-        const uint32_t af = m >= 0 ? reinterpret_cast<const uint32_t*>(aflag)[m] : 0u;
-        uint32_t k4 = 0;
-#pragma unroll
-        for (int k = 0; k < 4; k++) k4 += ((af >> (8 * k)) & 0xFFu) != 0u;
-        uint32_t tot;
-        uint32_t p = boff[f0 / kBlock] + block_exclusive_scan<uint32_t, kBlock>(k4, sm, tot);
+// composes them; a pattern face's corners go through vtwin first.
+__global__ void __launch_bounds__(kBlock) k_compact_quads(const int32_t* __restrict__ quads, const Sizes* S,
+                                                           const uint8_t* __restrict__ p3333,
+                                                           const int32_t* __restrict__ vtwin,
+                                                           const int32_t* __restrict__ vmap,
+                                                           const int32_t* __restrict__ qmap,
+                                                           int32_t* __restrict__ quads2) {
+    const int64_t nq = (int64_t)S->nq, nv = (int64_t)S->nv;
+    TMC_GRID_STRIDE(f, nq) {
+        const int32_t m = qmap[f];
+        if (m < 0) continue;
+        const int4 q = reinterpret_cast<const int4*>(quads)[f];
+        int32_t x[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            const uint32_t code = (af >> (8 * k)) & 0xFFu;
-            if (!code) continue;
-            const int32_t h = 4 * m + k;
-            alist[p++] = h;
-            if (code == 255u) continue;   // rank unknown: this build is redone from generic rows
-            const int32_t a = quads[h], b = he_dest(quads, h);
-            aadj[aoff[a] + code - 1u] = make_int2(h, b);
+            if (p3333 && p3333[f] && vid_ok(x[k], nv)) x[k] = vtwin[x[k]];
+            x[k] = vid_ok(x[k], nv) ? vmap[x[k]] : -1;
         }
+        reinterpret_cast<int4*>(quads2)[m] = make_int4(x[0], x[1], x[2], x[3]);
     }
 }
 
-// Pair the flagged halfedges (cpp_dmc/DualMarchingCubes.cpp:574-669) through
-// their rows; a changed origin also takes its out-degree and he_v from its
-// row, which holds all its out-halfedges.
-__global__ void __launch_bounds__(kBlock) k_aff_twins(const int32_t* __restrict__ alist, const Sizes* S,
-                                                       const int32_t* __restrict__ quads,
-                                                       const uint32_t* __restrict__ aoff,
-                                                       const int2* __restrict__ aadj, Carry c, BndRec* __restrict__ recs,
-                                                       uint32_t reccap) {
-    // rows incomplete (a rank past 253): the next build starts over
-    if (S->cbad & 0x80000000u) return;
-    const int64_t n = (int64_t)S->naff, nn = (int64_t)S->nn;
-    HeCount cnt;
-    TMC_GRID_STRIDE(i, n) {
-        const int32_t h = alist[i];
-        const int32_t a = quads[h], b = he_dest(quads, h);
-        int32_t g[5];
-        const int k = he_group(quads, aoff, aadj, h, nn, g);
-        int32_t tw;
-        uint8_t fl;
-        twin_rule(quads, k, g, h, tw, fl);
-        c.twin_n[h] = tw;
-        c.flag_n[h] = fl;
-        if (tw == -1) atomicAdd(&c.arr[b], 1u);
-        cnt.add(fl);
-        vol_count(c.vst, c.qb, c.nvol, h, fl);
-        if (k == 3 && g[0] == h) put_record(recs, &c.S->nrec, reccap, &c.S->ovf, three_record(quads, g, h));
-        if (c.cflag[a] & 1u) {
-            const uint32_t s = aoff[a], e = aoff[a + 1];
-            int32_t hmax = -1;
-            for_row(aadj, s, e, [&](int2 x) { hmax = max(hmax, x.x); });
-            c.deg_n[a] = e - s;
-            if (h == hmax) c.hev_n[a] = h;
-        }
-    }
-    cnt.flush(c.S->hep);
-}
-
-// 3-face records of groups the compaction left alone, renumbered.
-__global__ void __launch_bounds__(kBlock) k_carry_records(const BndRec* __restrict__ recs, const Sizes* S,
-                                                           const int32_t* __restrict__ vmap,
-                                                           const uint8_t* __restrict__ cflag,
-                                                           const int32_t* __restrict__ qmap,
-                                                           BndRec* __restrict__ recs_n, uint32_t* nrec,
-                                                           uint32_t reccap, uint32_t* ovf) {
-    const int64_t n = S->nrec_prev < reccap ? S->nrec_prev : reccap;
-    const int64_t nv = (int64_t)S->nv, nn = (int64_t)S->nn;
-    TMC_GRID_STRIDE(i, n) {
-        const BndRec r = recs[i];
-        const int32_t v0 = (int32_t)(r.key >> 32), v1 = (int32_t)(r.key & 0xFFFFFFFFull);
-        if (!vid_ok(v0, nv) || !vid_ok(v1, nv) || !vid_ok(r.a, nv) || !vid_ok(r.b, nv)) continue;
-        const int32_t y0 = vmap[v0], y1 = vmap[v1];
-        if (!vid_ok(y0, nn) || !vid_ok(y1, nn) || ((cflag[y0] | cflag[y1]) & 1u)) continue;
-        BndRec o;
-        o.key = he_key(y0, y1);
-        o.a = vmap[r.a];
-        o.b = vmap[r.b];
-        const int32_t m = qmap[r.lone >> 2];
-        if (m < 0) continue;
-        o.lone = 4 * m + (r.lone & 3);
-        o.pad = 0;
-        put_record(recs_n, nrec, reccap, ovf, o);
-    }
-}
-
-// Before a halfedge build: whether what it starts from stands.  ready: 0
-// generic rows (launched only in a pass run again for them), 1 the cell
-// stage's build, 2 the build a compaction carried over.  The cell stage's
-// build is whole unless a quadrilateral has an unresolved neighbour cell; a
-// carried build stands only if the build before it and the compaction met no
-// invalid vertex reference.  Otherwise the build needs generic rows, which
-// this pass did not launch: it flags the pass to be run again with them.
-__global__ void k_rows_gate(Sizes* S, int ready, int commit) {
+// Before a halfedge build of a pass run stage by stage: the counts the
+// compaction before it kept become the mesh's, and the statistics start over.
+__global__ void k_build_begin(Sizes* S, int commit) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        if (commit) {   // the compaction before this build: its counts become the live mesh
+        if (commit) {
             S->nv = S->nn;
             S->nq = S->qn;
         }
-        const bool stands = ready == 1 ? S->unresolved == 0u : ready == 2 && S->incr_ok != 0u && S->cbad == 0u;
-        if (ready != 0 && !stands) S->need_generic = 1u;
-        if (!stands) {
-            S->recmax = S->nrec > S->recmax ? S->nrec : S->recmax;
-            he_clear(S);
-            S->nrec = 0;
-        }
+        S->recmax = S->nrec > S->recmax ? S->nrec : S->recmax;
+        he_clear(S);
+        S->nrec = 0;
     }
 }
 

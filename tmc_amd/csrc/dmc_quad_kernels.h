@@ -51,7 +51,8 @@ struct QuadOut {
     int32_t* twin;
     uint8_t* flag;
     int32_t* hev;
-    uint32_t* arr;   // boundary arrivals per vertex (null: not wanted)
+    int32_t* val;    // valence per vertex, out-degrees so far (null: not wanted)
+    uint8_t* dead;   // face marks of the simplifications, cleared (with val)
     BndRec* recs;
     uint32_t reccap;
     Sizes* S;
@@ -342,11 +343,12 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 
             reinterpret_cast<uint32_t*>(o.flag)[q] = cf << (8 * s0) | (s0 ? cf >> (32 - 8 * s0) : 0u);
             o.colors[q] = (uint8_t)(3 * (entry >> 10) + (uint32_t)t);
             // valence: a boundary halfedge adds one to the vertex it ends at
-            if (o.arr) {
-                if (h0 < 0) atomicAdd(&o.arr[c1], 1u);
-                if (h1 < 0) atomicAdd(&o.arr[UW.v], 1u);
-                if (h2 < 0) atomicAdd(&o.arr[c3], 1u);
-                if (h3 < 0) atomicAdd(&o.arr[O.v], 1u);
+            if (o.val) {
+                if (h0 < 0) atomicAdd(&o.val[c1], 1);
+                if (h1 < 0) atomicAdd(&o.val[UW.v], 1);
+                if (h2 < 0) atomicAdd(&o.val[c3], 1);
+                if (h3 < 0) atomicAdd(&o.val[O.v], 1);
+                o.dead[q] = 0;
             }
             // he_v: the edge is the last interior one of the vertex's contour
             constexpr uint32_t l0 = later_edges(0), l3 = later_edges(3), l8 = later_edges(8), l2 = later_edges(2),
