@@ -1183,7 +1183,8 @@ constexpr int kListBlocks = 4096;
 
 void stage_rest(dmc_context* ctx, const Live& m, bool is3333) {
     const int64_t qcap = ctx->qcap;
-    launch(ctx, "k_stage_rewrite", k_stage_rewrite, dim3(grid_for(ctx, qcap)), dim3(kBlock), m, is3333 ? 1 : 0);
+    launch(ctx, "k_stage_rewrite", k_stage_rewrite, dim3(grid_for(ctx, qcap, kBlock, kListBlocks)), dim3(kBlock), m,
+           is3333 ? 1 : 0);
     launch(ctx, "k_stage_pair", k_stage_pair, dim3(grid_for(ctx, qcap)), dim3(kBlock), m);
     check_launch(ctx, "stage");
 }
@@ -1194,9 +1195,9 @@ void stage_3x3y(dmc_context* ctx, Live& m, bool colored) {
     if (colored) color_faces(ctx);
     // lists of merging faces are sized by the faces (a launch only needs to
     // cover them)
-    const int gq = grid_for(ctx, qcap), gl = grid_for(ctx, qcap / 4 + 1);
-    launch(ctx, "k_stage_mark", k_stage_mark, dim3(gq), dim3(kBlock), m);
-    launch(ctx, "k_stage_claim", k_stage_claim, dim3(grid_for(ctx, qcap, kBlock, kListBlocks)), dim3(kBlock), m,
+    const int gb = grid_for(ctx, qcap, kBlock, kListBlocks), gl = grid_for(ctx, qcap / 4 + 1);
+    launch(ctx, "k_stage_mark", k_stage_mark<false>, dim3(gb), dim3(kBlock), m);
+    launch(ctx, "k_stage_claim", k_stage_claim, dim3(gb), dim3(kBlock), m,
            colored ? static_cast<const uint8_t*>(ctx->colors.p) : nullptr);
     launch(ctx, "k_stage_sort", k_stage_sort, dim3(gl), dim3(kBlock), m);
     launch(ctx, "k_stage_merge", k_stage_merge, dim3(gl), dim3(kBlock), m);
@@ -1207,8 +1208,9 @@ void stage_3x3y(dmc_context* ctx, Live& m, bool colored) {
 void stage_3333(dmc_context* ctx, Live& m) {
     m.stage++;
     const int64_t qcap = ctx->qcap;
-    const int gl = grid_for(ctx, qcap / 4 + 1);
-    launch(ctx, "k_stage_mark3333", k_stage_mark3333, dim3(grid_for(ctx, qcap, kBlock, kListBlocks)), dim3(kBlock), m);
+    const int gb = grid_for(ctx, qcap, kBlock, kListBlocks), gl = grid_for(ctx, qcap / 4 + 1);
+    launch(ctx, "k_stage_mark", k_stage_mark<true>, dim3(gb), dim3(kBlock), m);
+    launch(ctx, "k_stage_claim", k_stage_claim3333, dim3(gb), dim3(kBlock), m);
     launch(ctx, "k_stage_cut3333", k_stage_cut3333, dim3(gl), dim3(kBlock), m);
     launch(ctx, "k_stage_irregular", k_stage_irregular3333, dim3(gl), dim3(kBlock), m);
     stage_rest(ctx, m, true);

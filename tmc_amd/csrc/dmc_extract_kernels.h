@@ -971,6 +971,14 @@ __global__ void k_vol_remap(int64_t* __restrict__ b, int n1, const uint32_t* __r
     }
 }
 
+// Volume of item x of a wave's consecutive items, the first of them `first`
+// (wave-uniform): one search per wave, then the few volumes a wave spans.
+__device__ __forceinline__ int vol_from(const int64_t* __restrict__ base, int n, int64_t first, int64_t x) {
+    int v = vol_of(base, n, first);
+    while (v + 1 < n && base[v + 1] <= x) v++;
+    return v;
+}
+
 __global__ void __launch_bounds__(kBlock) k_rebase(const int64_t* __restrict__ vb, const int64_t* __restrict__ qb,
                                                     int n, int32_t* __restrict__ quads, int32_t* __restrict__ twin,
                                                     int32_t* __restrict__ tris, const Sizes* S,
@@ -978,21 +986,30 @@ __global__ void __launch_bounds__(kBlock) k_rebase(const int64_t* __restrict__ v
     const int64_t nq = (int64_t)S->nq, nv = (int64_t)S->nv;
     const int64_t m = nq > nv ? nq : nv;
     for (int64_t x = (int64_t)blockIdx.x * kBlock + threadIdx.x; x < m; x += (int64_t)gridDim.x * kBlock) {
+        // the wave's first item (lane 0 is always in range with any lane)
+        const int64_t x0 = x - (int)(threadIdx.x & (kWave - 1));
+        const int64_t first = ((int64_t)__builtin_amdgcn_readfirstlane((int)(x0 >> 32)) << 32) |
+                              (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x0);
         if (x < nq) {
-            const int vol = vol_of(qb, n, x);
+            const int vol = vol_from(qb, n, first, x);
             const int32_t v0 = (int32_t)vb[vol], h0 = (int32_t)(4 * qb[vol]);
+            int4 q = reinterpret_cast<const int4*>(quads)[x], t = reinterpret_cast<const int4*>(twin)[x];
+            q = make_int4(q.x - v0, q.y - v0, q.z - v0, q.w - v0);
+            t = make_int4(t.x >= 0 ? t.x - h0 : t.x, t.y >= 0 ? t.y - h0 : t.y, t.z >= 0 ? t.z - h0 : t.z,
+                          t.w >= 0 ? t.w - h0 : t.w);
+            reinterpret_cast<int4*>(quads)[x] = q;
+            reinterpret_cast<int4*>(twin)[x] = t;
+            if (tris) {
+                int2* tr = reinterpret_cast<int2*>(tris + 6 * x);
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                quads[4 * x + k] -= v0;
-                const int32_t t = twin[4 * x + k];
-                if (t >= 0) twin[4 * x + k] = t - h0;
+                for (int k = 0; k < 3; k++) {
+                    const int2 e = tr[k];
+                    tr[k] = make_int2(e.x - v0, e.y - v0);
+                }
             }
-            if (tris)
-#pragma unroll
-                for (int k = 0; k < 6; k++) tris[6 * x + k] -= v0;
         }
         if (x < nv) {
-            const int vol = vol_of(vb, n, x);
+            const int vol = vol_from(vb, n, first, x);
             const int32_t e = hev[x];
             if (e >= 0) hev[x] = e - (int32_t)(4 * qb[vol]);
         }

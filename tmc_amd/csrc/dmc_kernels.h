@@ -91,7 +91,8 @@ struct Sizes {
     uint32_t nrec;               // 3-face edge records of the current build (dropped ones among them)
     uint32_t nrec_final;         // ... under the compacted numbers
     uint32_t recmax;             // most 3-face records any build of the pass wrote (capacity planning)
-    uint32_t nlist[4], nirr[4], nent[4];   // per stage: merging faces, irregular ones, halfedges to pair again
+    // per stage: candidate faces, merging ones, irregular ones, rewritten faces with halfedges to pair
+    uint32_t ncand[4], nlist[4], nirr[4], nent[4];
     uint32_t colors[48];         // colour classes: counts [0, 24), starts [24, 48)
     unsigned long long cpart[kContourParts];   // a single volume's contour count, in parts
     unsigned long long hep[kHeParts][3];      // the build's flagged halfedges per slot: groups of 4, of 3, error groups

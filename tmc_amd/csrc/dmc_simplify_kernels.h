@@ -6,8 +6,8 @@
 // or vertices sees the order it would see after a compaction per stage).  A
 // stage changes what lies around its merging faces and nothing else:
 //
-//   k_stage_mark, k_stage_claim   which faces merge; the last face to remove a
-//                    vertex claims it (the reference's sequential loop,
+//   k_stage_mark, k_stage_claim   the candidates and which of them merge; the
+//                    last face to remove a vertex claims it (the reference's sequential loop,
 //                    cpp_dmc/DualMarchingCubes.cpp:916-1094);
 //   k_stage_sort     the regular ones: both merging vertices closed fans of
 //                    three faces, all edges around in groups of two, the
@@ -21,7 +21,7 @@
 //                    changed corner is rewritten, and the halfedges on a
 //                    changed vertex are paired again by vertex pair.
 //
-// 3333 is built the same way (k_stage_mark3333, k_stage_cut3333, ...).  A pass
+// 3333 is built the same way (k_stage_claim3333, k_stage_cut3333, ...).  A pass
 // that meets what the in-place form does not express (a vertex merged into a
 // removed one, whose result depends on the compacted numbering; a face left
 // with a removed corner) sets need_generic and is run again with a compaction
@@ -55,13 +55,13 @@ struct Live {
     int32_t* last;     // 3X3Y: last irregular face to move each vertex; 3333: the vertex that takes its place
     double* pos;
     double* nrm;
-    uint8_t* p;        // faces of the pattern (3333: 2 irregular)
-    uint8_t* em;       // merging faces: which pair of vertices merges (1 / 2)
-    uint32_t* list;    // merging / pattern faces of the stage
-    int4* frame;       // their frames, two words of four (MergeFrame)
-    uint32_t* irr;     // the irregular ones
+    uint8_t* p;        // 3X3Y: faces of the pattern; 3333: 2 irregular pattern faces
+    uint8_t* em;       // merging faces: which pair of vertices merges (1 / 2); rewritten ones: halfedges to pair
+    uint32_t* list;    // merging / pattern faces of the stage, then the rewritten ones
+    int4* frame;       // the merging faces' frames, two words of four (MergeFrame)
+    uint32_t* irr;     // candidates, then the irregular ones of the list
     int32_t* head;     // changed vertices: their halfedges to pair, a list through ...
-    int4* ent;         // ... (halfedge, next entry, origin, destination)
+    int4* ent;         // ... entry h of halfedge h (next, origin, destination, changed vertex)
     BndRec* recs;
     uint32_t reccap;
     Sizes* S;
@@ -112,28 +112,33 @@ __device__ __forceinline__ void vs_or(uint8_t* vs, int32_t v, uint32_t bits) {
 // The face lists of a stage.  A block walks a contiguous range of faces and
 // gathers its entries in LDS, so that the list's counter takes few adds and
 // the list keeps neighbouring faces together.
-constexpr int kListBuf = 1024;
+constexpr int kListBuf = 2048;
+constexpr int kListIlp = 4;   // faces a thread looks at per turn: their gathers are in flight together
+constexpr int kListTurn = kListIlp * kBlock;
 struct ListBuf {
-    uint32_t* buf;
+    uint32_t* buf;    // LDS, kListBuf entries
     uint32_t* n;      // LDS: entries held, then the base of a flush
     uint32_t* out;
     uint32_t* count;
-    // every thread of the block calls this, once per turn of kBlock faces
-    __device__ __forceinline__ void turn(bool has, uint32_t x) const {
+    // at most kListIlp adds per thread and turn
+    __device__ __forceinline__ void add(bool has, uint32_t x) const {
         const uint64_t m = __ballot(has);
-        if (m) {
-            uint32_t base = 0;
-            const int leader = __ffsll((unsigned long long)m) - 1;
-            if ((int)__lane_id() == leader) base = atomicAdd(&n[0], (uint32_t)__popcll(m));
-            base = (uint32_t)__shfl((int)base, leader, kWave);
-            if (has) buf[base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = x;
-        }
+        if (!m) return;
+        uint32_t base = 0;
+        const int leader = __ffsll((unsigned long long)m) - 1;
+        if ((int)__lane_id() == leader) base = atomicAdd(&n[0], (uint32_t)__popcll(m));
+        base = (uint32_t)__shfl((int)base, leader, kWave);
+        if (has) buf[base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = x;
+    }
+    // every thread of the block calls these, once per turn / at the end
+    __device__ __forceinline__ void end_turn() const {
         __syncthreads();
         const uint32_t held = n[0];
         __syncthreads();   // the next turn adds
-        if (held > kListBuf - kBlock) flush();
+        if (held > kListBuf - kListTurn) flush();
     }
     __device__ __forceinline__ void flush() const {
+        __syncthreads();
         const uint32_t k = n[0];
         if (threadIdx.x == 0) n[1] = k ? atomicAdd(count, k) : 0u;
         __syncthreads();
@@ -144,9 +149,21 @@ struct ListBuf {
         __syncthreads();
     }
 };
-// a block's share of n faces, a multiple of kBlock
+// a block's share of n items: whole turns where there are many
 __device__ __forceinline__ int64_t block_share(int64_t n) {
-    return (n + (int64_t)gridDim.x * kBlock - 1) / ((int64_t)gridDim.x * kBlock) * kBlock;
+    const int64_t each = (n + (int64_t)gridDim.x - 1) / (int64_t)gridDim.x;
+    const int64_t unit = each > kListTurn ? kListTurn : kBlock;
+    return (each + unit - 1) / unit * unit;
+}
+// Calls fn(f, in range) for the block's share of n faces, kListIlp faces per
+// thread and turn, consecutive threads on consecutive faces; then end().
+template <class F, class E>
+__device__ __forceinline__ void for_share(int64_t n, F&& fn, E&& end_turn) {
+    const int64_t share = block_share(n), begin = (int64_t)blockIdx.x * share, end = min(n, begin + share);
+    for (int64_t f0 = begin; f0 < end; f0 += kListTurn) {
+        fn(f0 + threadIdx.x, end);
+        end_turn();
+    }
 }
 
 // Kept vertices of valence 0, counted at each stage's start.
@@ -158,40 +175,66 @@ __device__ __forceinline__ void count_zero(const Live& m) {
     if ((threadIdx.x & (kWave - 1)) == 0 && z) atomicAdd(&m.S->zero, z);
 }
 
-// 3X3Y pattern (cpp_dmc/DualMarchingCubes.cpp:889-913) of the live faces.
+// Candidates of the stage among the live faces, listed in m.irr: 3X3Y the
+// pattern (cpp_dmc/DualMarchingCubes.cpp:889-913), also kept per face for its
+// neighbours; 3333 the faces of four valence-3 corners (:1190-1301 asks more).
+// Bound by the valence gathers: four faces per thread keep sixteen in flight.
+template <bool k3333>
 __global__ void __launch_bounds__(kBlock) k_stage_mark(Live m) {
-    const int64_t nq = (int64_t)m.S->nq;
-    TMC_GRID_STRIDE(f, nq) {
-        uint8_t r = 0;
-        if (!m.dead[f]) {
-            const int4 q = reinterpret_cast<const int4*>(m.quads)[f];
-            const int a = m.val[q.x], b = m.val[q.y], c = m.val[q.z], d = m.val[q.w];
-            r = (a == 3 && b >= 5 && c == 3 && d >= 5) || (a >= 5 && b == 3 && c >= 5 && d == 3);
+    __shared__ uint32_t buf[kListBuf], n[2];
+    if (threadIdx.x == 0) n[0] = 0;
+    __syncthreads();
+    const ListBuf L{buf, n, m.irr, &m.S->ncand[m.stage]};
+    for_share((int64_t)m.S->nq, [&](int64_t f0, int64_t end) {
+        bool r[kListIlp];
+        int4 q[kListIlp];
+        uint8_t dead[kListIlp];
+#pragma unroll
+        for (int u = 0; u < kListIlp; u++) {
+            const int64_t f = f0 + u * kBlock;
+            const bool in = f < end;
+            q[u] = in ? reinterpret_cast<const int4*>(m.quads)[f] : make_int4(0, 0, 0, 0);
+            dead[u] = in ? m.dead[f] : 1;
         }
-        m.p[f] = r;
-    }
+#pragma unroll
+        for (int u = 0; u < kListIlp; u++) {
+            const int a = m.val[q[u].x], b = m.val[q[u].y], c = m.val[q[u].z], d = m.val[q[u].w];
+            r[u] = k3333 ? a == 3 && b == 3 && c == 3 && d == 3
+                         : (a == 3 && b >= 5 && c == 3 && d >= 5) || (a >= 5 && b == 3 && c >= 5 && d == 3);
+            r[u] = r[u] && !dead[u];
+        }
+#pragma unroll
+        for (int u = 0; u < kListIlp; u++) {
+            const int64_t f = f0 + u * kBlock;
+            if (f < end) m.p[f] = !k3333 && r[u];
+            L.add(r[u], (uint32_t)f);
+        }
+    }, [&] { L.end_turn(); });
+    L.flush();
     // every vertex of the cell stage has a face
     if (m.stage > 1) count_zero(m);
 }
 
-// The merging faces: each claims the vertex it removes.
+// The merging faces among the candidates: each claims the vertex it removes.
 __global__ void __launch_bounds__(kBlock) k_stage_claim(Live m, const uint8_t* __restrict__ colors) {
     __shared__ uint32_t buf[kListBuf], n[2];
     if (threadIdx.x == 0) n[0] = 0;
     __syncthreads();
     const ListBuf L{buf, n, m.list, &m.S->nlist[m.stage]};
-    const int64_t nq = (int64_t)m.S->nq, nv = (int64_t)m.S->nv, share = block_share(nq);
-    const int64_t end = min(nq, ((int64_t)blockIdx.x + 1) * share);
-    for (int64_t f0 = (int64_t)blockIdx.x * share; f0 < end; f0 += kBlock) {
-        const int64_t f = f0 + threadIdx.x;
-        const int d = f < end ? merge_decision(f, m.quads, m.val, m.p, colors, m.twin, m.flag, nv) : 0;
-        if (d) {
-            const int4 q = reinterpret_cast<const int4*>(m.quads)[f];
-            m.em[f] = (uint8_t)d;
-            atomicMax(&m.claim[d == 1 ? q.z : q.w], m.tag(f));
+    const int64_t nv = (int64_t)m.S->nv;
+    for_share((int64_t)m.S->ncand[m.stage], [&](int64_t i0, int64_t end) {
+        for (int u = 0; u < kListIlp; u++) {
+            const int64_t i = i0 + u * kBlock;
+            const int64_t f = i < end ? (int64_t)m.irr[i] : 0;
+            const int d = i < end ? merge_decision(f, m.quads, m.val, m.p, colors, m.twin, m.flag, nv) : 0;
+            if (d) {
+                const int4 q = reinterpret_cast<const int4*>(m.quads)[f];
+                m.em[f] = (uint8_t)d;
+                atomicMax(&m.claim[d == 1 ? q.z : q.w], m.tag(f));
+            }
+            L.add(d != 0, (uint32_t)f | (uint32_t)(d == 2) << 31);
         }
-        L.turn(d != 0, (uint32_t)f | (uint32_t)(d == 2) << 31);
-    }
+    }, [&] { L.end_turn(); });
     L.flush();
 }
 
@@ -388,78 +431,91 @@ __global__ void __launch_bounds__(kBlock) k_stage_irregular(Live m) {
 
 // Every live face with a corner that was removed or changed irregularly: the
 // corners' new names (3333: a pattern face's corners are replaced), and its
-// halfedges on a changed vertex listed with that vertex.  3-face records with
-// such an end are dropped.
+// halfedges on a changed vertex linked into that vertex's list (entry h is
+// halfedge h's); such faces are listed in m.list, which the merges are done
+// with, their halfedges in m.em.  3-face records with such an end are dropped.
+__device__ __forceinline__ uint32_t rewrite_face(const Live& m, int64_t f, const int4& q, const uint8_t (&s)[4],
+                                                 bool is3333, HeDelta& cnt) {
+    const uint8_t ch = m.changed();
+    const bool pattern = is3333 && m.p[f] == 2;
+    const int32_t x[4] = {q.x, q.y, q.z, q.w};
+    int32_t r[4];
+    uint8_t sr[4];
+    bool lost = false;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        r[k] = x[k];
+        if (pattern) r[k] = m.last[x[k]];
+        else if (s[k] & kVsGone) r[k] = is3333 ? -1 : renamed(m, x[k]);
+        if (r[k] < 0) {
+            lost = true;
+            r[k] = x[k];
+        }
+        sr[k] = r[k] == x[k] ? s[k] : m.vs[r[k]];
+    }
+    if (lost) m.S->need_generic = 1u;   // a removed corner without a new name
+    reinterpret_cast<int4*>(m.quads)[f] = make_int4(r[0], r[1], r[2], r[3]);
+    const int4 t4 = reinterpret_cast<const int4*>(m.twin)[f];
+    const int32_t tw[4] = {t4.x, t4.y, t4.z, t4.w};
+    const uint32_t fl = reinterpret_cast<const uint32_t*>(m.flag)[f];
+    uint32_t aff = 0;   // halfedges to pair again
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int b = (k + 1) & 3;
+        if (!((sr[k] | sr[b]) & ch)) continue;
+        aff |= 1u << k;
+        const int32_t h = (int32_t)(4 * f) + k;
+        const uint8_t o = (uint8_t)(fl >> (8 * k));
+        cnt.add(o, -1);
+        vol_delta(m, h, o, -1);
+        // a boundary halfedge leaves a vertex that is counted on
+        if (tw[k] < 0 && !(s[b] & (ch | kVsGone))) atomicSub(&m.val[x[b]], 1);
+        if (sr[k] & ch) {
+            atomicAdd(&m.val[r[k]], 1);
+            atomicMax(&m.hev[r[k]], h);
+        }
+        const int32_t w = (sr[k] & sr[b] & ch) ? min(r[k], r[b]) : (sr[k] & ch) ? r[k] : r[b];
+        m.ent[h] = make_int4(atomicExch(&m.head[w], h), r[k], r[b], w);
+    }
+    if (aff) m.em[f] = (uint8_t)aff;
+    return aff;
+}
+
 __global__ void __launch_bounds__(kBlock) k_stage_rewrite(Live m, int is3333) {
-    __shared__ uint32_t sm[kBlock / kWave + 1], s_base;
+    __shared__ uint32_t buf[kListBuf], n[2];
     if (m.S->nirr[m.stage] == 0u) return;
-    const int64_t nq = (int64_t)m.S->nq;
+    if (threadIdx.x == 0) n[0] = 0;
+    __syncthreads();
+    const ListBuf L{buf, n, m.list, &m.S->nent[m.stage]};
     const uint8_t ch = m.changed();
     HeDelta cnt;
-    for (int64_t f0 = (int64_t)blockIdx.x * kBlock; f0 < nq; f0 += (int64_t)gridDim.x * kBlock) {
-        const int64_t f = f0 + threadIdx.x;
-        uint32_t aff = 0;   // halfedges to pair again
-        int32_t r[4] = {0, 0, 0, 0};
-        uint8_t sr[4] = {0, 0, 0, 0};
-        if (f < nq && !m.dead[f]) {
-            const int4 q = reinterpret_cast<const int4*>(m.quads)[f];
-            const int32_t x[4] = {q.x, q.y, q.z, q.w};
-            uint8_t s[4];
+    for_share((int64_t)m.S->nq, [&](int64_t f0, int64_t end) {
+        int4 q[kListIlp];
+        uint8_t s[kListIlp][4];
+        bool hit[kListIlp];
 #pragma unroll
-            for (int k = 0; k < 4; k++) s[k] = m.vs[x[k]];
-            const bool pattern = is3333 && m.p[f] == 2;
-            if (pattern || ((s[0] | s[1] | s[2] | s[3]) & (ch | kVsGone))) {
-                bool lost = false;
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    r[k] = x[k];
-                    if (pattern) r[k] = m.last[x[k]];
-                    else if (s[k] & kVsGone) r[k] = is3333 ? -1 : renamed(m, x[k]);
-                    if (r[k] < 0) {
-                        lost = true;
-                        r[k] = x[k];
-                    }
-                    sr[k] = r[k] == x[k] ? s[k] : m.vs[r[k]];
-                }
-                if (lost) m.S->need_generic = 1u;   // a removed corner without a new name
-                reinterpret_cast<int4*>(m.quads)[f] = make_int4(r[0], r[1], r[2], r[3]);
-                const int4 t4 = reinterpret_cast<const int4*>(m.twin)[f];
-                const int32_t tw[4] = {t4.x, t4.y, t4.z, t4.w};
-                const uint32_t fl = reinterpret_cast<const uint32_t*>(m.flag)[f];
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const int b = (k + 1) & 3;
-                    if (!((sr[k] | sr[b]) & ch)) continue;
-                    aff |= 1u << k;
-                    const int32_t h = (int32_t)(4 * f) + k;
-                    const uint8_t o = (uint8_t)(fl >> (8 * k));
-                    cnt.add(o, -1);
-                    vol_delta(m, h, o, -1);
-                    // a boundary halfedge leaves a vertex that is counted on
-                    if (tw[k] < 0 && !(s[b] & (ch | kVsGone))) atomicSub(&m.val[x[b]], 1);
-                    if (sr[k] & ch) {
-                        atomicAdd(&m.val[r[k]], 1);
-                        atomicMax(&m.hev[r[k]], h);
-                    }
-                }
-            }
+        for (int u = 0; u < kListIlp; u++) {
+            const int64_t f = f0 + u * kBlock;
+            hit[u] = f < end && !m.dead[f];
+            q[u] = f < end ? reinterpret_cast<const int4*>(m.quads)[f] : make_int4(0, 0, 0, 0);
         }
-        uint32_t tot;
-        uint32_t at = block_exclusive_scan<uint32_t, kBlock>((uint32_t)__popc(aff), sm, tot);
-        if (tot == 0u) continue;   // block-uniform
-        if (threadIdx.x == 0) s_base = atomicAdd(&m.S->nent[m.stage], tot);
-        __syncthreads();
-        at += s_base;
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            if (!((aff >> k) & 1u)) continue;
-            const int b = (k + 1) & 3;
-            const int32_t w = (sr[k] & sr[b] & ch) ? min(r[k], r[b]) : (sr[k] & ch) ? r[k] : r[b];
-            m.ent[at] = make_int4((int32_t)(4 * f) + k, atomicExch(&m.head[w], (int32_t)at), r[k], r[b]);
-            at++;
+        for (int u = 0; u < kListIlp; u++) {
+            s[u][0] = m.vs[q[u].x];
+            s[u][1] = m.vs[q[u].y];
+            s[u][2] = m.vs[q[u].z];
+            s[u][3] = m.vs[q[u].w];
+            const bool pattern = is3333 && hit[u] && m.p[f0 + u * kBlock] == 2;
+            hit[u] = hit[u] && (pattern || ((s[u][0] | s[u][1] | s[u][2] | s[u][3]) & (ch | kVsGone)));
         }
-        __syncthreads();
-    }
+#pragma unroll
+        for (int u = 0; u < kListIlp; u++) {
+            const int64_t f = f0 + u * kBlock;
+            const uint32_t aff = hit[u] ? rewrite_face(m, f, q[u], s[u], is3333 != 0, cnt) : 0u;
+            L.add(aff != 0u, (uint32_t)f);
+        }
+    }, [&] { L.end_turn(); });
+    L.flush();
     const int64_t nr = min((int64_t)m.S->nrec, (int64_t)m.reccap);
     TMC_GRID_STRIDE(i, nr) {
         const BndRec r = m.recs[i];
@@ -470,30 +526,30 @@ __global__ void __launch_bounds__(kBlock) k_stage_rewrite(Live m, int is3333) {
     cnt.flush(m.S->hep);
 }
 
-// The listed halfedges, paired by vertex pair (cpp_dmc/DualMarchingCubes.cpp:
-// 574-669): all halfedges on a pair with a changed vertex are in that
-// vertex's list (both changed: the smaller one's).
+// The listed faces' linked halfedges, paired by vertex pair
+// (cpp_dmc/DualMarchingCubes.cpp:574-669): all halfedges on a pair with a
+// changed vertex are in that vertex's list (both changed: the smaller one's).
 __global__ void __launch_bounds__(kBlock) k_stage_pair(Live m) {
-    const int64_t n = (int64_t)m.S->nent[m.stage];
+    const int64_t n = 4 * (int64_t)m.S->nent[m.stage];
     if (n == 0) return;
-    const uint8_t ch = m.changed();
     HeDelta cnt;
     TMC_GRID_STRIDE(i, n) {
-        const int4 own = m.ent[i];
-        const int32_t h = own.x, a = own.z, b = own.w;
-        const uint8_t sa = m.vs[a], sb = m.vs[b];
-        const int32_t w = (sa & sb & ch) ? min(a, b) : (sa & ch) ? a : b;
+        const uint32_t f = m.list[i >> 2];
+        if (!((m.em[f] >> (i & 3)) & 1u)) continue;
+        const int32_t h = (int32_t)(4u * f) + (int32_t)(i & 3);
+        const int4 own = m.ent[h];
+        const int32_t a = own.y, b = own.z;
         int32_t g[5];
 #pragma unroll
         for (int k = 0; k < 5; k++) g[k] = 0x7FFFFFFF;
         int c = 0;
-        for (int32_t e = m.head[w]; e >= 0;) {
+        for (int32_t e = m.head[own.w]; e >= 0;) {
             const int4 x = m.ent[e];
-            if ((x.z == a && x.w == b) || (x.z == b && x.w == a)) {
-                group_insert(g, x.x);
+            if ((x.y == a && x.z == b) || (x.y == b && x.z == a)) {
+                group_insert(g, e);
                 c++;
             }
-            e = x.y;
+            e = x.x;
         }
         int32_t tw;
         uint8_t fl;
@@ -508,22 +564,20 @@ __global__ void __launch_bounds__(kBlock) k_stage_pair(Live m) {
     cnt.flush(m.S->hep);
 }
 
-// 3333 patterns (cpp_dmc/DualMarchingCubes.cpp:1190-1301): the four corners
-// are claimed, the four faces around dropped.
-__global__ void __launch_bounds__(kBlock) k_stage_mark3333(Live m) {
+// The 3333 patterns among the candidates (cpp_dmc/DualMarchingCubes.cpp:
+// 1190-1301): the four corners are claimed, the four faces around dropped.
+__global__ void __launch_bounds__(kBlock) k_stage_claim3333(Live m) {
     __shared__ uint32_t buf[kListBuf], n[2];
     if (threadIdx.x == 0) n[0] = 0;
     __syncthreads();
     const ListBuf L{buf, n, m.list, &m.S->nlist[m.stage]};
-    const int64_t nq = (int64_t)m.S->nq, nv = (int64_t)m.S->nv, share = block_share(nq);
-    const int64_t end = min(nq, ((int64_t)blockIdx.x + 1) * share);
-    for (int64_t f0 = (int64_t)blockIdx.x * share; f0 < end; f0 += kBlock) {
-        const int64_t f = f0 + threadIdx.x;
-        bool has = false;
-        if (f < end) {
+    const int64_t nv = (int64_t)m.S->nv;
+    for_share((int64_t)m.S->ncand[m.stage], [&](int64_t i0, int64_t end) {
+        for (int u = 0; u < kListIlp; u++) {
+            const int64_t i = i0 + u * kBlock;
+            const int64_t f = i < end ? (int64_t)m.irr[i] : 0;
             int32_t vq[4], vo[4], fn[4];
-            has = !(m.dead[f] & 1u) && pattern3333(f, m.quads, m.twin, m.flag, m.val, nv, vq, vo, fn);
-            m.p[f] = has;
+            const bool has = i < end && pattern3333(f, m.quads, m.twin, m.flag, m.val, nv, vq, vo, fn);
             if (has) {
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
@@ -531,11 +585,10 @@ __global__ void __launch_bounds__(kBlock) k_stage_mark3333(Live m) {
                     m.dead[fn[k]] = 2;
                 }
             }
+            L.add(has, (uint32_t)f);
         }
-        L.turn(has, (uint32_t)f);
-    }
+    }, [&] { L.end_turn(); });
     L.flush();
-    if (m.stage > 1) count_zero(m);
 }
 
 // The regular patterns: the corners' fans close over the four dropped faces,
