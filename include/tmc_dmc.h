@@ -350,8 +350,9 @@ dmc_status tmc_download(dmc_context* ctx, double* positions, double* normals, in
  *   grid_cap     blocks (256 threads) of every grid-stride kernel, which
  *                loops over its items: 64 .. 2^24, default 32768 (env
  *                TMC_GRID_CAP);
- *   sweep_waves  waves the field sweep aims for, one 256-cell x 16-row tile
- *                of K planes each; sets K (never below 8): 256 .. 2^24,
+ *   sweep_waves  waves the field sweep aims for, one 256-cell x 4-row tile
+ *                (8 rows from 2^28 points on) of K planes each; sets K:
+ *                256 .. 2^24,
  *                default 32768 (env TMC_SWEEP_WAVES).
  * There is no hash-table load factor to choose: vertex and quadrilateral
  * ids come from prefix sums over the cells, not from hash tables.

@@ -591,7 +591,8 @@ struct Swept {
 // by upload_vtab) and the sweep's tiling.
 struct SweepPlan {
     int64_t W, RS, groups, cells;
-    bool vec;
+    int J;          // cell rows per wave of the sweep
+    int rows;       // kVectorRows, kLongRows or kShortRows: what every volume's rows allow
     size_t tab_bytes;
 };
 
@@ -603,6 +604,13 @@ struct SweepPlan {
 // 511.
 int group_shift(int64_t rs) { return rs >= (1 << 16) ? 4 : rs >= (1 << 13) ? 2 : 0; }
 
+template <class T, int J>
+auto sweep_kernel(int rows) {
+    return rows == kVectorRows ? k_sweep<T, kVectorRows, J>
+           : rows == kLongRows ? k_sweep<T, kLongRows, J>
+                               : k_sweep<T, kShortRows, J>;
+}
+
 template <class T>
 SweepPlan plan_sweep(dmc_context* ctx, const std::vector<HostVol>& hv) {
     const int n = (int)hv.size();
@@ -610,7 +618,9 @@ SweepPlan plan_sweep(dmc_context* ctx, const std::vector<HostVol>& hv) {
     // sweep tiling: J rows per wave; one plane count K for the whole
     // extraction, chosen so that about ctx->sweep_waves waves fill the chip
     std::vector<VolDesc> desc(n);
-    int64_t units = 0, cells = 0;
+    int64_t units = 0, cells = 0, points = 0;
+    for (int v = 0; v < n; v++) points += (int64_t)hv[v].g.nx * hv[v].g.ny * hv[v].g.nz;
+    const int J = points < kSweepManyPoints ? kSweepRowsFew : kSweepRowsMany;
     for (int v = 0; v < n; v++) {
         const dmc_grid& g = hv[v].g;
         VolDesc& D = desc[v];
@@ -628,19 +638,19 @@ SweepPlan plan_sweep(dmc_context* ctx, const std::vector<HostVol>& hv) {
         D.iso = hv[v].iso;
         D.iso_t = sizeof(T) == 4 ? (double)smallest_float_not_below(hv[v].iso) : hv[v].iso;
         D.S = (int)((D.d.C + kSeg - 1) / kSeg);
-        D.ntj = (g.ny - 1 + kSweepRows - 1) / kSweepRows;
+        D.ntj = (g.ny - 1 + J - 1) / J;
         units += (int64_t)(g.nz - 1) * D.S * D.ntj;
         cells += D.d.C * D.d.R;
     }
-    // (at least 2 planes per wave, so that the shared boundary plane costs at
-    // most half again; small volumes get short marches and many waves)
-    const int Kg = (int)std::max<int64_t>(2, (units + ctx->sweep_waves - 1) / ctx->sweep_waves);
+    // (volumes that cannot fill the chip get one plane a wave: 32^3 5.4 us
+    // against 7.9 with two, 128^3 8.7 against 9.9)
+    const int Kg = (int)std::max<int64_t>(1, (units + ctx->sweep_waves - 1) / ctx->sweep_waves);
     const size_t tab_bytes = (size_t)n * sizeof(VolDesc) + 3 * (size_t)(n + 1) * sizeof(int64_t);
     ctx->vtab_host.assign(tab_bytes, 0);
     int64_t* waveBase = reinterpret_cast<int64_t*>(ctx->vtab_host.data() + (size_t)n * sizeof(VolDesc));
     int64_t* grpBase = waveBase + (n + 1);
     int64_t W = 0, RS = 0;
-    bool vec = true;
+    int rows = kVectorRows;
     int64_t rs_all = 0;
     for (int v = 0; v < n; v++) rs_all += desc[v].d.R * desc[v].S;
     const int gsh = group_shift(rs_all);
@@ -654,13 +664,14 @@ SweepPlan plan_sweep(dmc_context* ctx, const std::vector<HostVol>& hv) {
         grpBase[v] = RS >> gsh;
         W += (int64_t)D.S * D.ntj * D.ntk;
         RS += (D.d.R * D.S + kGroup - 1) / kGroup * kGroup;
-        vec = vec && (D.d.nx % 4 == 0) && ((uintptr_t)D.field % (4 * sizeof(T)) == 0);
+        const bool whole = D.d.nx % 4 == 0 && (uintptr_t)D.field % (4 * sizeof(T)) == 0;
+        rows = std::min<int>(rows, whole ? kVectorRows : D.d.nx >= 4 ? kLongRows : kShortRows);
     }
     waveBase[n] = W;
     grpBase[n] = RS >> gsh;
     memcpy(ctx->vtab_host.data(), desc.data(), (size_t)n * sizeof(VolDesc));
     ensure<uint8_t>(ctx, ctx->vtab, tab_bytes);
-    return SweepPlan{W, RS, RS >> gsh, cells, vec, tab_bytes};
+    return SweepPlan{W, RS, RS >> gsh, cells, J, rows, tab_bytes};
 }
 
 // The volume table to the device (before the pass's launches; a replayed
@@ -690,10 +701,9 @@ Swept sweep_cells(dmc_context* ctx, const SweepPlan& P) {
     mark(ctx, "sweep");
     const int64_t sblocks = (W + kBlock / kWave - 1) / (kBlock / kWave);
     const dim3 sgrid((unsigned)((sblocks + kXcds - 1) / kXcds * kXcds));
-    if (P.vec)
-        launch(ctx, "k_sweep", (k_sweep<T, true>), sgrid, dim3(kBlock), vt, W, lists, segCount, segMask);
-    else
-        launch(ctx, "k_sweep", (k_sweep<T, false>), sgrid, dim3(kBlock), vt, W, lists, segCount, segMask);
+    const auto sweep = P.J == kSweepRowsFew ? sweep_kernel<T, kSweepRowsFew>(P.rows)
+                                            : sweep_kernel<T, kSweepRowsMany>(P.rows);
+    launch(ctx, "k_sweep", sweep, sgrid, dim3(kBlock), vt, W, lists, segCount, segMask);
     check_launch(ctx, "k_sweep");
     mark(ctx, "rows");
     scan_to(ctx, ScanCounts{segCount}, segBase, hn(RS), &S->A, "k_scan_cells");
@@ -1610,7 +1620,8 @@ std::string pass_key(dmc_context* ctx, const std::vector<HostVol>& hv, const Swe
     auto put = [&](int64_t x) { k.append(reinterpret_cast<const char*>(&x), sizeof(x)); };
     put(field_type);
     put(flags & (DMC_SIMPLIFY_ALL | DMC_TRIANGLES));
-    put(P.vec);
+    put(P.J);
+    put(P.rows);
     put(ctx->grid_cap);
     put(ctx->sweep_waves);
     put(ctx->acap);

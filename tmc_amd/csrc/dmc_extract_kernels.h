@@ -81,12 +81,16 @@ struct VolTable {
 // fields (double)f >= iso is evaluated as f >= iso_up, iso_up the smallest
 // float not below iso: the same predicate.
 // ---------------------------------------------------------------------------
+// Cell rows per wave (J).  More rows read fewer halo rows again, fewer rows
+// leave registers for more waves a SIMD and give small volumes more of them.
+// us with 16 / 8 / 4 rows: 32^3 16.4 / 11.7 / 7.9, 128^3 20.0 / 13.8 / 9.9,
+// 129^3 doubles 21 / 14.7 / 11.4, 301^3 43 / 36.7 / 35.8, 512^3 150 / 143 / 142,
+// 1024^3 1095 / 1105 / 1118 (2 rows: 301^3 38, 16 blobs of 300^3 381 against
+// 339 with 4).
+constexpr int kSweepRowsFew = 4, kSweepRowsMany = 8;
+constexpr int64_t kSweepManyPoints = (int64_t)1 << 28;   // points of a pass from which a wave takes many
 constexpr int kSeg = 256;           // cells per segment (one wave) and list slots per (row, segment)
 constexpr int kGroup = 16;          // most (row, segment)s per wave of k_cells; a volume is padded to whole ones
-#ifndef TMC_SWEEP_ROWS
-#define TMC_SWEEP_ROWS 16
-#endif
-constexpr int kSweepRows = TMC_SWEEP_ROWS;  // J
 #ifndef TMC_VERTICES_ATTR
 #define TMC_VERTICES_ATTR
 #endif
@@ -99,12 +103,23 @@ constexpr int kVerticesChunk = TMC_VERTICES_CHUNK;
 // Loads of the 4 points i0..i0+3 of a row.  Rows read by one wave only are
 // streamed (non-temporal, so they do not evict reused lines); rows that a
 // neighbouring wave also reads (KEEP) are loaded through L2.
-template <class T, bool VEC, bool KEEP>
+//
+// ROWS says what a launch's rows allow:
+//   kVectorRows  whole vectors, aligned: one vector load, lanes past the end
+//                read the last 4 points
+//   kLongRows    at least 4 points: one vector load at the element's alignment;
+//                the lanes at the row's end read its last 4 points and shift
+//                their bits back.  With 16 cell rows a wave, against four
+//                clamped loads a lane: 301^3 floats 43 us (72), 16 blobs of
+//                300^3 408 (669), 385^3 doubles 114 (128)
+//   kShortRows   fewer than 4 points: clamped loads
+enum { kShortRows = 0, kLongRows = 1, kVectorRows = 2 };
+template <class T, int ROWS, bool KEEP>
 __device__ __forceinline__ void row_load(const T* __restrict__ row, int i0, int nx, T v[4]) {
-    if constexpr (VEC) {
-        const int ic = min(i0, nx - 4);  // nx % 4 == 0: lanes past the end read the last 4 points
+    if constexpr (ROWS != kShortRows) {
         typedef T vec4 __attribute__((ext_vector_type(4)));
-        const vec4* src = reinterpret_cast<const vec4*>(row + ic);
+        typedef vec4 load4 __attribute__((aligned(ROWS == kVectorRows ? sizeof(vec4) : sizeof(T))));
+        const load4* src = reinterpret_cast<const load4*>(row + min(i0, nx - 4));
         const vec4 t = KEEP ? *src : __builtin_nontemporal_load(src);
         v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
     } else {
@@ -115,10 +130,11 @@ __device__ __forceinline__ void row_load(const T* __restrict__ row, int i0, int 
 
 // bits 0..3: points i0..i0+3 at or above iso; bit 4: point i0+4 (next
 // lane; `edge` is point x0+256 for lane 63)
-template <class T>
-__device__ __forceinline__ uint32_t row_bits(const T v[4], T edge, T iso_t, int lane) {
-    const uint32_t b = (uint32_t)(v[0] >= iso_t) | (uint32_t)(v[1] >= iso_t) << 1 | (uint32_t)(v[2] >= iso_t) << 2 |
-                       (uint32_t)(v[3] >= iso_t) << 3;
+template <class T, int ROWS>
+__device__ __forceinline__ uint32_t row_bits(const T v[4], T edge, T iso_t, int lane, int i0, int nx) {
+    uint32_t b = (uint32_t)(v[0] >= iso_t) | (uint32_t)(v[1] >= iso_t) << 1 | (uint32_t)(v[2] >= iso_t) << 2 |
+                 (uint32_t)(v[3] >= iso_t) << 3;
+    if constexpr (ROWS == kLongRows) b >>= min(i0, nx - 1) - min(i0, nx - 4);
     // DPP wave_shl:1: lane L receives lane L+1's value
     uint32_t nb = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(b & 1u), 0x130, 0xF, 0xF, false);
     nb = lane == kWave - 1 ? (uint32_t)(edge >= iso_t) : nb;
@@ -130,20 +146,19 @@ __device__ __forceinline__ uint32_t row_bits(const T v[4], T edge, T iso_t, int 
 // past the last one are clamped to it and their bits feed no cell.  The
 // first and last rows are shared with the neighbouring row tiles; a whole
 // plane is shared when KEEP.
-template <class T, bool VEC, bool KEEP>
+template <class T, int ROWS, bool KEEP, int J>
 __device__ __forceinline__ void plane_bits(const T* __restrict__ pl, const Dims& d, int j0, int i0, int ie,
-                                           T iso_t, int lane, uint32_t bits[kSweepRows + 1]) {
-    constexpr int J = kSweepRows;
+                                           T iso_t, int lane, uint32_t bits[J + 1]) {
     T v[J + 1][4], e[J + 1];
 #pragma unroll
     for (int jr = 0; jr <= J; jr++) {
         const T* row = pl + (int64_t)min(j0 + jr, d.ny - 1) * d.nx;
-        if (KEEP || jr == 0 || jr == J) row_load<T, VEC, true>(row, i0, d.nx, v[jr]);
-        else row_load<T, VEC, false>(row, i0, d.nx, v[jr]);
+        if (KEEP || jr == 0 || jr == J) row_load<T, ROWS, true>(row, i0, d.nx, v[jr]);
+        else row_load<T, ROWS, false>(row, i0, d.nx, v[jr]);
         e[jr] = row[ie];
     }
 #pragma unroll
-    for (int jr = 0; jr <= J; jr++) bits[jr] = row_bits<T>(v[jr], e[jr], iso_t, lane);
+    for (int jr = 0; jr <= J; jr++) bits[jr] = row_bits<T, ROWS>(v[jr], e[jr], iso_t, lane, i0, d.nx);
 }
 
 // v_writelane_b32 through its LLVM intrinsic, so that the compiler sees the
@@ -164,9 +179,9 @@ struct PlaneCells {
     uint32_t* lists;      // list of the tile's first (row, segment)
     int S, i0, nj;
     uint32_t valid;
-    // lane l of stage[h]: dword (l & 7) of the activity words of row
-    // 8h + (l >> 3); lane jr of counts: active cells of row jr
-    uint32_t stage[2];
+    // lane l of stage: dword (l & 7) of the activity words of row l >> 3;
+    // lane jr of counts: active cells of row jr
+    uint32_t stage;
     uint32_t counts;
 };
 
@@ -181,8 +196,8 @@ __device__ __forceinline__ void cell_row(PlaneCells& c) {
     uint32_t act = any_in & ~all_in & (JR < c.nj ? c.valid : 0u);
     const uint64_t b0 = __ballot(act & 1u), b1 = __ballot(act & 2u), b2 = __ballot(act & 4u), b3 = __ballot(act & 8u);
     const uint32_t total = (uint32_t)(__popcll(b0) + __popcll(b1) + __popcll(b2) + __popcll(b3));
-    uint32_t& st = c.stage[JR >> 3];
-    constexpr int l0 = 8 * (JR & 7);
+    uint32_t& st = c.stage;
+    constexpr int l0 = 8 * JR;
     write_lane<l0 + 0>(st, (uint32_t)b0);
     write_lane<l0 + 1>(st, (uint32_t)(b0 >> 32));
     write_lane<l0 + 2>(st, (uint32_t)b1);
@@ -220,22 +235,20 @@ __device__ __forceinline__ void cell_rows(PlaneCells& c, std::index_sequence<JR.
 // The cells of plane k of the wave's tile from the bits of point planes k
 // (lo) and k+1 (hi); the activity words and active counts of the rows below
 // nj are stored once per plane from their lanes.
-__device__ __forceinline__ void plane_cells(const uint32_t lo[kSweepRows + 1], const uint32_t hi[kSweepRows + 1],
+template <int J>
+__device__ __forceinline__ void plane_cells(const uint32_t lo[J + 1], const uint32_t hi[J + 1],
                                             int64_t k, const Dims& d, int j0, int nj, int S, int s, int i0,
                                             uint32_t valid, int lane, uint32_t* __restrict__ lists,
                                             uint32_t* __restrict__ segCount,
                                             unsigned long long* __restrict__ segMask) {
-    static_assert(kSweepRows <= 16, "activity words of the rows are staged in two VGPRs");
+    static_assert(J <= 8, "activity words of the rows are staged in one VGPR");
     const int64_t rs0 = (k * (d.ny - 1) + j0) * S + s;  // (row, segment) of the tile's first row
-    PlaneCells c{lo, hi, lists + rs0 * kSeg, S, i0, nj, valid, {0u, 0u}, 0u};
-    cell_rows(c, std::make_index_sequence<kSweepRows>{});
+    PlaneCells c{lo, hi, lists + rs0 * kSeg, S, i0, nj, valid, 0u, 0u};
+    cell_rows(c, std::make_index_sequence<J>{});
     // activity of the segment: bit L of word q <-> cell x0 + 4L + q
     uint32_t* mask32 = reinterpret_cast<uint32_t*>(segMask);
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int row = 8 * h + (lane >> 3);
-        if (row < nj && row < kSweepRows) mask32[8 * (rs0 + (int64_t)row * S) + (lane & 7)] = c.stage[h];
-    }
+    const int row = lane >> 3;
+    if (row < nj && row < J) mask32[8 * (rs0 + (int64_t)row * S) + (lane & 7)] = c.stage;
     if (lane < nj) segCount[rs0 + (int64_t)lane * S] = c.counts;
 }
 
@@ -243,34 +256,32 @@ __device__ __forceinline__ void plane_cells(const uint32_t lo[kSweepRows + 1], c
 // downwards.  Plane tiles alternate direction, so two neighbouring tiles
 // read their shared boundary plane both first or both last, at about the
 // same time: the second read is served by L2.
-template <class T, bool VEC, bool DOWN>
+template <class T, int ROWS, bool DOWN, int J>
 __device__ __forceinline__ void sweep_march(const T* __restrict__ field, const Dims& d, int k0, int k1, int j0,
                                             int nj, int S, int s, int i0, int ie, uint32_t valid,
                                             T iso_t, int lane, uint32_t* __restrict__ lists,
                                             uint32_t* __restrict__ segCount,
                                             unsigned long long* __restrict__ segMask) {
-    constexpr int J = kSweepRows;
     const int64_t plane = (int64_t)d.nx * d.ny;
     uint32_t prev[J + 1], cur[J + 1];
     int kp = DOWN ? k1 : k0;
-    plane_bits<T, VEC, true>(field + (int64_t)kp * plane, d, j0, i0, ie, iso_t, lane, prev);
+    plane_bits<T, ROWS, true, J>(field + (int64_t)kp * plane, d, j0, i0, ie, iso_t, lane, prev);
     for (int n = k1 - k0; n > 0; n--) {
         const int kn = DOWN ? kp - 1 : kp + 1;
-        if (n == 1) plane_bits<T, VEC, true>(field + (int64_t)kn * plane, d, j0, i0, ie, iso_t, lane, cur);
-        else plane_bits<T, VEC, false>(field + (int64_t)kn * plane, d, j0, i0, ie, iso_t, lane, cur);
-        if (DOWN) plane_cells(cur, prev, kn, d, j0, nj, S, s, i0, valid, lane, lists, segCount, segMask);
-        else plane_cells(prev, cur, kp, d, j0, nj, S, s, i0, valid, lane, lists, segCount, segMask);
+        if (n == 1) plane_bits<T, ROWS, true, J>(field + (int64_t)kn * plane, d, j0, i0, ie, iso_t, lane, cur);
+        else plane_bits<T, ROWS, false, J>(field + (int64_t)kn * plane, d, j0, i0, ie, iso_t, lane, cur);
+        if (DOWN) plane_cells<J>(cur, prev, kn, d, j0, nj, S, s, i0, valid, lane, lists, segCount, segMask);
+        else plane_cells<J>(prev, cur, kp, d, j0, nj, S, s, i0, valid, lane, lists, segCount, segMask);
 #pragma unroll
         for (int jr = 0; jr <= J; jr++) prev[jr] = cur[jr];
         kp = kn;
     }
 }
 
-template <class T, bool VEC>
+template <class T, int ROWS, int J>
 __global__ void __launch_bounds__(kBlock) k_sweep(VolTable vt, int64_t waves, uint32_t* __restrict__ lists,
                                                    uint32_t* __restrict__ segCount,
                                                    unsigned long long* __restrict__ segMask) {
-    constexpr int J = kSweepRows;
     const int lane = threadIdx.x & (kWave - 1);
     // wave-uniform from here on (kept in scalar registers)
     const int64_t gwave =
@@ -298,10 +309,10 @@ __global__ void __launch_bounds__(kBlock) k_sweep(VolTable vt, int64_t waves, ui
     const int ncell = d.nx - 1 - i0;
     const uint32_t valid = ncell >= 4 ? 0xFu : ncell > 0 ? (1u << ncell) - 1u : 0u;
     if (tk & 1)
-        sweep_march<T, VEC, true>(field, d, k0, k1, j0, nj, S, s, i0, ie, valid, iso_t, lane, lists, segCount,
+        sweep_march<T, ROWS, true, J>(field, d, k0, k1, j0, nj, S, s, i0, ie, valid, iso_t, lane, lists, segCount,
                                   segMask);
     else
-        sweep_march<T, VEC, false>(field, d, k0, k1, j0, nj, S, s, i0, ie, valid, iso_t, lane, lists, segCount,
+        sweep_march<T, ROWS, false, J>(field, d, k0, k1, j0, nj, S, s, i0, ie, valid, iso_t, lane, lists, segCount,
                                    segMask);
     // the volume's last wave empties the padding of its last group
     if (wave == vt.waveBase[v + 1] - vt.waveBase[v] - 1) {
