@@ -132,7 +132,7 @@ struct dmc_context {
     Buf drep, dnew, dval, dhist, dedges, dqual;
     // topologically correct MC: per active cell vertex / triangle counts and
     // offsets, the ambiguous-cell list, owner words; stats; the mesh
-    Buf tcntv, tcntt, tvofs, ttofs, tamb, tvb, tstats, tpos, tnrm, ttris;
+    Buf tvofs, ttofs, tamb, tstats, tpos, tnrm, ttris;
     tmc_mesh tmesh{};
     bool have_tmesh = false;
     // pinned host staging of device-to-host reads (counts, totals, tables)
@@ -197,7 +197,7 @@ struct dmc_context {
                       &twin, &flag, &hev, &twin2, &flag2, &hev2, &ovr, &bndrec, &bndrec2, &val, &p, &em, &vfirst,
                       &vsecond, &lastT, &lastR, &newV, &newQ, &clist, &cnbr, &ccnt, &tris, &vmap, &mlist, &slow,
                       &dead, &vstate, &irr, &head, &ent, &frame, &vtab, &vstat, &vbound, &qbound, &vhe, &drep, &dnew, &dval,
-                      &dhist, &dedges, &dqual, &tcntv, &tcntt, &tvofs, &ttofs, &tamb, &tvb, &tstats, &tpos, &tnrm,
+                      &dhist, &dedges, &dqual, &tvofs, &ttofs, &tamb, &tstats, &tpos, &tnrm,
                       &ttris};
         for (Buf* b : all) bufs.push_back(b);
     }
@@ -1321,25 +1321,22 @@ void run_tmc(dmc_context* ctx, const std::vector<HostVol>& hv) {
     const int64_t G = sw.groups;
     uint32_t* acell = ensure<uint32_t>(ctx, ctx->acell, A);
     uint32_t* acode = ensure<uint32_t>(ctx, ctx->acode, A);
-    uint32_t* cnt_v = ensure<uint32_t>(ctx, ctx->tcntv, A);
-    uint32_t* cnt_t = ensure<uint32_t>(ctx, ctx->tcntt, A);
     uint32_t* vofs = ensure<uint32_t>(ctx, ctx->tvofs, A);
     uint32_t* tofs = ensure<uint32_t>(ctx, ctx->ttofs, A);
-    unsigned long long* st = ensure<unsigned long long>(ctx, ctx->tstats, 3);
+    unsigned long long* st = ensure<unsigned long long>(ctx, ctx->tstats, 2);
     uint32_t* amb = ensure<uint32_t>(ctx, ctx->tamb, A + 1);
-    fill_u32(ctx, st, hn(6), 0u);
-    fill_u32(ctx, amb, hn(1), 0u);
-    launch(ctx, "k_tmc_cells", k_tmc_cells, dim3(grid_for(ctx, G, kBlock / kWave)), dim3(kBlock), sw.vt, G, sw.lists,
-           sw.segCount, sw.segBase, acell, acode, cnt_v, cnt_t, amb, st);
+    Fills(ctx).u32(st, hn(4), 0u).u32(amb, hn(1), 0u).run();
+    launch(ctx, "k_tmc_cells", k_tmc_cells, dim3(grid_for(ctx, G, kBlock / kWave, kTmcCellsBlocks)), dim3(kBlock), sw.vt, G,
+           sw.lists, sw.segCount, sw.segBase, acell, acode, amb);
     check_launch(ctx, "k_tmc_cells");
     if (A > 0) {
         launch(ctx, "k_tmc_amb_count", k_tmc_amb_count<T>, dim3(grid_for(ctx, A, kBlock, 1024)), dim3(kBlock), sw.vt,
-               amb, acell, acode, cnt_v, cnt_t, st);
+               amb, acell, acode, st);
         check_launch(ctx, "k_tmc_amb_count");
     }
     uint64_t* tot = ensure<uint64_t>(ctx, ctx->scanTotal, 2);
-    scan_pair(ctx, scan_job(ScanCounts{cnt_v}, vofs, hn((int64_t)A), tot),
-              scan_job(ScanCounts{cnt_t}, tofs, hn((int64_t)A), tot + 1));
+    scan_pair(ctx, scan_job(ScanTmc<false>{acode}, vofs, hn((int64_t)A), tot),
+              scan_job(ScanTmc<true>{acode}, tofs, hn((int64_t)A), tot + 1));
     uint64_t VT[2] = {0, 0};
     {
         HostReads rd(ctx);
@@ -1353,28 +1350,27 @@ void run_tmc(dmc_context* ctx, const std::vector<HostVol>& hv) {
     double* pos = ensure<double>(ctx, ctx->tpos, 3 * V);
     double* nrm = ensure<double>(ctx, ctx->tnrm, 3 * V);
     int32_t* tris = ensure<int32_t>(ctx, ctx->ttris, 3 * Tn);
-    uint2* avb = ensure<uint2>(ctx, ctx->tvb, A);
     mark(ctx, "emit");
     if (A > 0) {
-        launch(ctx, "k_tmc_vbase", k_tmc_vbase, dim3(grid_for(ctx, A)), dim3(kBlock), sw.vt, acell, acode, vofs,
-               (int64_t)A, avb);
-        check_launch(ctx, "k_tmc_vbase");
-        launch(ctx, "k_tmc_emit", k_tmc_emit<T>, dim3(grid_for(ctx, A)), dim3(kBlock), sw.vt, acell, acode, avb, tofs,
-               sw.segMask, sw.segBase, (int64_t)A, pos, nrm, tris, st + 2);
+        launch(ctx, "k_tmc_emit", k_tmc_emit<T>, dim3(grid_for(ctx, A)), dim3(kBlock), sw.vt, acell, acode, vofs, tofs,
+               sw.segMask, sw.segBase, (int64_t)A, pos, nrm, tris, st + 1);
         check_launch(ctx, "k_tmc_emit");
         launch(ctx, "k_tmc_emit_amb", k_tmc_emit_amb<T>, dim3(grid_for(ctx, A, kBlock, 1024)), dim3(kBlock), sw.vt,
-               amb, acell, acode, avb, tofs, sw.segMask, sw.segBase, pos, nrm, tris, st + 2);
+               amb, acell, acode, vofs, tofs, sw.segMask, sw.segBase, (int64_t)A, pos, nrm, tris, st + 1);
         check_launch(ctx, "k_tmc_emit_amb");
     }
     mark(ctx, "end");
-    unsigned long long hs[3];
+    unsigned long long hs[2];
+    uint32_t namb = 0;
     {
         HostReads rd(ctx);
         rd.add(hs, st, sizeof(hs));
+        rd.add(&namb, amb, sizeof(namb));
         rd.wait();
     }
     finish_timing(ctx);
-    if (hs[2] != 0) fail(ctx, DMC_ERR_STATE, "%llu cut edges without an active owner cell", hs[2]);
+    if (hs[1] != 0)
+        fail(ctx, DMC_ERR_STATE, "%llu cells with a cut edge without an active owner cell", hs[1]);
     tmc_mesh& m = ctx->tmesh;
     m = tmc_mesh{};
     m.nv = (int64_t)V;
@@ -1383,8 +1379,8 @@ void run_tmc(dmc_context* ctx, const std::vector<HostVol>& hv) {
     m.d_normals = nrm;
     m.d_tris = tris;
     m.active_cells = (int64_t)A;
-    m.ambiguous_cells = (int64_t)hs[0];
-    m.face_failures = (int64_t)hs[1];
+    m.ambiguous_cells = namb;
+    m.face_failures = (int64_t)hs[0];
     ctx->have_tmesh = true;
 }
 

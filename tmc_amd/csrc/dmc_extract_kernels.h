@@ -910,21 +910,6 @@ __device__ __forceinline__ uint32_t active_at(const SegWords& s, int i) {
     return s.base + rank;
 }
 
-// Position of cell (i, j, k) in the active arrays; -1 if it is not active.
-__device__ __forceinline__ int64_t find_active(const SegLists& L, const Dims& d, int i, int j, int k) {
-    const int64_t rs = L.rsBase + ((int64_t)k * (d.ny - 1) + j) * L.S + (i / kSeg);
-    const int il = i % kSeg, ln = il >> 2, q = il & 3;
-    const ulonglong2* m2 = reinterpret_cast<const ulonglong2*>(L.mask + 4 * rs);
-    const ulonglong2 w01 = m2[0], w23 = m2[1];
-    const unsigned long long w[4] = {w01.x, w01.y, w23.x, w23.y};
-    if (!((w[q] >> ln) & 1ull)) return -1;
-    const unsigned long long below = (1ull << ln) - 1ull;
-    int rank = 0;
-#pragma unroll
-    for (int t = 0; t < 4; t++) rank += __popcll(w[t] & below) + (t < q ? (int)((w[t] >> ln) & 1ull) : 0);
-    return (int64_t)L.base[rs] + rank;
-}
-
 // ---------------------------------------------------------------------------
 // Per-volume bookkeeping of a batch: first active cell, vertex and
 // quadrilateral of each volume (n+1 entries, the last one the total), kept

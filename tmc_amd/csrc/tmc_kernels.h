@@ -5,19 +5,17 @@
 // The active cells come from the DMC sweep (same classification, f >= iso,
 // same per-(row, segment) lists, whose flat order is the reference's
 // (k, j, i) cell order).  Then:
-//   k_tmc_cells      each active cell's case, new vertices
-//                    (the cut edges it owns) and table triangles; the
-//                    ambiguous cells listed;
+//   k_tmc_cells      each active cell's word: case, the cut edges it owns,
+//                    table triangles; the ambiguous cells listed;
 //   k_tmc_amb_count  the listed cells' inner vertices and triangles from the
 //                    decider slicing (kept out of the cell walk, where one
 //                    ambiguous lane would hold up its wave);
 //   scans            over the active cells: each cell's first vertex and
 //                    triangle -- the reference's numbering, first sight in
 //                    cell order;
-//   k_tmc_emit       one thread per non-ambiguous active cell, and
-//   k_tmc_emit_amb   one per listed cell: positions and normals of the cell's
-//                    new vertices, and its triangles with the vertex ids of
-//                    cut edges owned by earlier cells.
+//   k_tmc_emit       positions and normals of the cells' edge vertices, and
+//                    the table triangles of the non-ambiguous cells;
+//   k_tmc_emit_amb   inner vertices and triangles of the listed cells.
 // A grid edge is owned by the first cell containing it in (k, j, i) order;
 // that cell is active because the edge is cut, so its active index is found
 // from the sweep's activity words.
@@ -33,81 +31,60 @@ namespace tmc {
 __device__ __constant__ uint64_t c_tmc_tri[256] = TMC_CASE_TRIANGLES_INIT;
 __device__ __constant__ uint64_t c_tmc_amb[4] = TMC_AMBIGUOUS_MASK_INIT;
 
-// Edge e: end corners (corner c = i + 2 j + 4 k) packed as v0 | v1 << 4;
-// its first grid point relative to the cell (bits 0..2: x, y, z) and axis
-// (bits 3..4), the reference's key layout (mc/MarchingCubes.cpp:153-159).
+// Edge e: end corners (corner c = i + 2 j + 4 k) packed as v0 | v1 << 4, the
+// lower one first (mc/MarchingCubes.cpp:153-159).
 __device__ __constant__ uint8_t c_tmc_ev[12] = {0x10, 0x31, 0x32, 0x20, 0x54, 0x75, 0x76, 0x64, 0x40, 0x51, 0x73, 0x62};
-__device__ __constant__ uint8_t c_tmc_ekey[12] = {0, 1 | 8, 2, 8, 4, 1 | 4 | 8, 2 | 4, 4 | 8, 16, 1 | 16, 1 | 2 | 16, 2 | 16};
 // faces seen from outside: corners and edges in oriented order
 // (mc/MarchingCubes.h:84-107), one nibble each
 __device__ __constant__ uint16_t c_tmc_fv[6] = {0x3120, 0x6475, 0x1504, 0x7362, 0x2064, 0x7531};
 __device__ __constant__ uint16_t c_tmc_fe[6] = {0x0123, 0x4765, 0x4908, 0x2A6B, 0x83B7, 0x95A1};
-// edge of each axis (x, y, z) by the offset of its first point from a cell
-// (bits: x, y, z of the offset)
-__device__ __constant__ int8_t c_tmc_edge_at[3][8] = {{0, -1, 2, -1, 4, -1, 6, -1},
-                                                      {3, 1, -1, -1, 7, 5, -1, -1},
-                                                      {8, 9, 11, 10, -1, -1, -1, -1}};
 // local coordinates of the edge points per axis: 2 bits per edge, 3 = along
 // the edge (mc/MarchingCubes.cpp:896-903)
 constexpr unsigned kTmcLCoord[3] = {1324855u, 5299420u, 16733440u};
 
 __device__ __forceinline__ bool tmc_ambiguous(unsigned icase) { return (c_tmc_amb[icase >> 6] >> (icase & 63)) & 1ull; }
 
+// Cut edges of a case: x-edges 0 2 4 6 join corners that differ in bit 0,
+// y-edges 3 1 7 5 in bit 1, z-edges 8 9 11 10 in bit 2.
 __device__ __forceinline__ unsigned tmc_cut_mask(unsigned icase) {
-    unsigned m = 0;
-#pragma unroll
-    for (int e = 0; e < 12; e++) {
-        const unsigned a = c_tmc_ev[e] & 0xF, b = c_tmc_ev[e] >> 4;
-        m |= (((icase >> a) ^ (icase >> b)) & 1u) << e;
-    }
-    return m;
+    const unsigned x = icase ^ (icase >> 1), y = icase ^ (icase >> 2), z = icase ^ (icase >> 4);
+    return (x & 0x55u) | (y & 2u) | (y & 1u) << 3 | (y & 0x20u) | (y & 0x10u) << 3 | (z & 3u) << 8 | (z & 8u) << 7 |
+           (z & 4u) << 9;
 }
 
-__device__ __forceinline__ bool cell_exists(int x, int y, int z, const Dims& d) {
-    return x >= 0 && y >= 0 && z >= 0 && x <= d.nx - 2 && y <= d.ny - 2 && z <= d.nz - 2;
+// Edges of cell (i, j, k) that it owns (it is their first cell): the three
+// that meet the far corner, and those that the grid's lower sides leave
+// without an earlier cell.
+__device__ __forceinline__ unsigned tmc_owned_mask(int i, int j, int k) {
+    const unsigned i0 = i == 0, j0 = j == 0, k0 = k == 0;
+    return (1u << 5 | 1u << 6 | 1u << 10) | k0 * (1u << 1 | 1u << 2) | j0 * (1u << 4 | 1u << 9) |
+           i0 * (1u << 7 | 1u << 11) | (j0 & k0) | (i0 & k0) << 3 | (i0 & j0) << 8;
 }
 
-// The first cell in (k, j, i) order that contains edge e of cell (i, j, k),
-// and the edge's id in that cell.  The candidates are the four cells around
-// the edge, earliest first.
-__device__ __forceinline__ void tmc_edge_owner(int i, int j, int k, int e, const Dims& d, int& oi, int& oj, int& ok,
-                                               int& oe) {
-    const unsigned key = c_tmc_ekey[e];
-    const int gx = i + (key & 1), gy = j + ((key >> 1) & 1), gz = k + ((key >> 2) & 1);
-    const int axis = key >> 3;
-    // offsets (s, t) of the candidates along the two other axes, earliest first
-    const int sa[4] = {1, 0, 1, 0}, ta[4] = {1, 1, 0, 0};
+// An active cell's word: case (bits 0-7), "no triangles" (bit 8, a singular
+// face), inner vertices (9-11), owned cut edges (12-23), triangles (24-31).
+__device__ __forceinline__ unsigned tmc_own(uint32_t code) { return (code >> 12) & 0xFFFu; }
+__device__ __forceinline__ unsigned tmc_new_vertices(uint32_t code) {
+    return (unsigned)__popc(code & 0xFFF000u) + ((code >> 9) & 7u);
+}
+// Their scans: new vertices, triangles.
+template <bool TRIS>
+struct ScanTmc {
+    static constexpr bool kMap = false;
+    const uint32_t* p;
+    __device__ __forceinline__ static uint32_t of(uint32_t w) { return TRIS ? w >> 24 : tmc_new_vertices(w); }
+    __device__ __forceinline__ uint32_t at(int64_t i) const { return of(p[i]); }
+    __device__ __forceinline__ void vec16(int64_t base, uint32_t v[kScanIPT]) const {
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-        int cx = gx, cy = gy, cz = gz;
-        if (axis == 0) { cy -= sa[c]; cz -= ta[c]; }
-        else if (axis == 1) { cx -= sa[c]; cz -= ta[c]; }
-        else { cx -= sa[c]; cy -= ta[c]; }
-        if (cell_exists(cx, cy, cz, d)) {
-            oi = cx;
-            oj = cy;
-            ok = cz;
-            oe = c_tmc_edge_at[axis][(gx - cx) | (gy - cy) << 1 | (gz - cz) << 2];
-            return;
+        for (int q = 0; q < kScanIPT / 4; q++) {
+            const uint4 t = reinterpret_cast<const uint4*>(p + base)[q];
+            v[4 * q] = of(t.x);
+            v[4 * q + 1] = of(t.y);
+            v[4 * q + 2] = of(t.z);
+            v[4 * q + 3] = of(t.w);
         }
     }
-    oi = i;
-    oj = j;
-    ok = k;
-    oe = e;
-}
-
-// Edges of cell (i, j, k) that it owns (it is their first cell).
-__device__ __forceinline__ unsigned tmc_owned_mask(int i, int j, int k, const Dims& d) {
-    if (i >= 1 && j >= 1 && k >= 1) return (1u << 5) | (1u << 6) | (1u << 10);
-    unsigned m = 0;
-    for (int e = 0; e < 12; e++) {
-        int oi, oj, ok, oe;
-        tmc_edge_owner(i, j, k, e, d, oi, oj, ok, oe);
-        if (oi == i && oj == j && ok == k) m |= 1u << e;
-    }
-    return m;
-}
+};
 
 __device__ __forceinline__ double tmc_decider(double f0, double f1, double f2, double f3) {
     return (f0 * f3 - f1 * f2) / (f0 + f3 - f1 - f2);
@@ -440,25 +417,27 @@ __device__ __forceinline__ void tmc_corners(const T* __restrict__ field, const D
 }
 
 // K_T1: one wave per group of (row, segment)s as in k_cells, cells in the
-// flat active order: per active cell its cell word, case (acode), new
-// vertices (cnt_v: the cut edges it owns) and triangles (cnt_t: the case
-// table's); the ambiguous cells are listed (amb[0] = count, from amb[1]) for
-// k_tmc_amb_count, which adds their inner vertices and sets their triangles.
-// stats[0] counts them.
+// flat active order: per active cell its cell index and its word.  Ambiguous
+// cells are listed (amb[0] = count, from amb[1]): a wave gathers them in LDS
+// and a block adds them to the list at its end (an add per wave and turn made
+// the counter's queue half of this kernel: 625 us at 1024^3, now 307).
+constexpr int kTmcAmb = 256;             // ambiguous cells a wave holds
+constexpr int kTmcCellsBlocks = 4096;    // at most: the blocks' adds to the counter
 __global__ void __launch_bounds__(kBlock) k_tmc_cells(VolTable vt, int64_t groups, const uint32_t* __restrict__ lists,
                                                        const uint32_t* __restrict__ segCount,
                                                        const uint32_t* __restrict__ segBase,
                                                        uint32_t* __restrict__ acell, uint32_t* __restrict__ acode,
-                                                       uint32_t* __restrict__ cnt_v, uint32_t* __restrict__ cnt_t,
-                                                       uint32_t* __restrict__ amb,
-                                                       unsigned long long* __restrict__ stats) {
-    const int lane = threadIdx.x & (kWave - 1);
+                                                       uint32_t* __restrict__ amb) {
+    __shared__ uint32_t s_amb[kBlock / kWave][kTmcAmb];
+    __shared__ uint32_t s_n[kBlock / kWave], s_base;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int64_t wpb = kBlock / kWave;
-    unsigned long long namb = 0;
-    for (int64_t g = (int64_t)blockIdx.x * wpb + __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave); g < groups;
+    uint32_t* held = s_amb[wave];
+    uint32_t nheld = 0;   // wave-uniform
+    const VolDesc V = vt.desc[0];   // a copy: the list's stores could otherwise change it
+    const Dims d = V.d;
+    for (int64_t g = (int64_t)blockIdx.x * wpb + __builtin_amdgcn_readfirstlane(wave); g < groups;
          g += (int64_t)gridDim.x * wpb) {
-        const VolDesc& V = vt.desc[vol_of(vt.grpBase, vt.n, g)];
-        const Dims d = V.d;
         const GroupLanes L = load_group(V, g, lane, segCount, segBase);
         for (uint32_t x0 = 0; x0 < L.total; x0 += kWave) {
             const uint32_t x = x0 + lane, a = L.first + x;
@@ -471,58 +450,66 @@ __global__ void __launch_bounds__(kBlock) k_tmc_cells(VolTable vt, int64_t group
                 const int i = (int)(e & 0xFFFFFFu);
                 const unsigned icase = e >> 24;
                 isamb = tmc_ambiguous(icase);
-                namb += isamb;
+                const uint32_t nt = isamb ? 0u : (uint32_t)(c_tmc_tri[icase] >> 60);
                 acell[a] = ((uint32_t)k * (uint32_t)(d.ny - 1) + (uint32_t)j) * (uint32_t)d.C + (uint32_t)i;
-                acode[a] = icase;
-                cnt_v[a] = (uint32_t)__popc(tmc_cut_mask(icase) & tmc_owned_mask(i, j, k, d));
-                cnt_t[a] = isamb ? 0u : (uint32_t)(c_tmc_tri[icase] >> 60);
+                acode[a] = icase | (tmc_cut_mask(icase) & tmc_owned_mask(i, j, k)) << 12 | nt << 24;
             }
-            // ambiguous cells go to the list k_tmc_amb_count and k_tmc_emit_amb
-            // work through
             const uint64_t m = __ballot(isamb);
             if (m) {
-                const int leader = __ffsll((unsigned long long)m) - 1;
-                uint32_t base = 0;
-                if (lane == leader) base = atomicAdd(amb, (uint32_t)__popcll(m));
-                base = (uint32_t)__shfl((int)base, leader, kWave);
-                const uint32_t below =
-                    __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-                if (isamb) amb[1 + base + below] = a;
+                if (isamb)
+                    held[nheld + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = a;
+                nheld += (uint32_t)__popcll(m);
+                if (nheld > kTmcAmb - kWave) {   // no room for another turn
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    uint32_t base = 0;
+                    if (lane == 0) base = atomicAdd(amb, nheld);
+                    base = (uint32_t)__shfl((int)base, 0, kWave);
+                    for (uint32_t y = lane; y < nheld; y += kWave) amb[1 + base + y] = held[y];
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    nheld = 0;
+                }
             }
         }
     }
-    namb = wave_sum(namb);
-    if (lane == 0 && namb) atomicAdd(&stats[0], namb);
+    if (lane == 0) s_n[wave] = nheld;
+    __syncthreads();
+    uint32_t at = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < kBlock / kWave; w++) {
+        if (w < wave) at += s_n[w];
+        all += s_n[w];
+    }
+    if (all == 0) return;
+    if (threadIdx.x == 0) s_base = atomicAdd(amb, all);
+    __syncthreads();
+    for (uint32_t y = lane; y < nheld; y += kWave) amb[1 + s_base + at + y] = held[y];
 }
 
-// K_T2: the listed ambiguous cells' inner vertices (added to cnt_v) and
-// triangles (cnt_t) from the decider slicing; acode bit 8 marks a cell
-// whose singular face could not be triangulated (no triangles), counted in
-// stats[1].
+// K_T2: the listed ambiguous cells' inner vertices and triangles from the
+// decider slicing, into the cell's word; bit 8 marks one whose singular face
+// could not be triangulated (no triangles), counted in stats[0].
 template <class T>
 __global__ void __launch_bounds__(kBlock) k_tmc_amb_count(VolTable vt, const uint32_t* __restrict__ amb,
                                                            const uint32_t* __restrict__ acell,
-                                                           uint32_t* __restrict__ acode, uint32_t* __restrict__ cnt_v,
-                                                           uint32_t* __restrict__ cnt_t,
+                                                           uint32_t* __restrict__ acode,
                                                            unsigned long long* __restrict__ stats) {
     const uint32_t n = amb[0];
+    const VolDesc& V = vt.desc[0];
     for (uint32_t s = blockIdx.x * kBlock + threadIdx.x; s < n; s += gridDim.x * kBlock) {
         const uint32_t a = amb[1 + s];
-        const int vol = vol_of(vt.aBase, vt.n, a);
-        const VolDesc& V = vt.desc[vol];
         int i, j, k;
         uint32_t r;
         cell_ijk(acell[a], V.d, i, j, k, r);
-        const unsigned icase = acode[a] & 0xFFu;
+        const uint32_t code = acode[a];
         double F[8];
         tmc_corners(static_cast<const T*>(V.field), V.d, i, j, k, F);
         TmcCount c;
-        if (tmc_slice(F, icase, V.iso, c)) {
-            cnt_v[a] += (uint32_t)c.ninner;
-            cnt_t[a] = (uint32_t)c.nt;
+        if (tmc_slice(F, code & 0xFFu, V.iso, c)) {
+            acode[a] = code | (uint32_t)c.ninner << 9 | (uint32_t)c.nt << 24;
         } else {
-            acode[a] = icase | 0x100u;
-            atomicAdd(&stats[1], 1ull);
+            acode[a] = code | 0x100u;
+            atomicAdd(&stats[0], 1ull);
         }
     }
 }
@@ -550,22 +537,71 @@ __device__ __forceinline__ void tmc_corner_gradient(const T* __restrict__ field,
     else n[2] = (cz ? (double)p[sz] - F[c & ~4] : F[c | 4] - (double)p[-sz]) / (2 * geo.dz);
 }
 
-// After the scans: per active cell its owned cut edges (x) and first vertex
-// id (y, the exclusive scan of cnt_v), one 8-byte word for the owner
-// lookups of k_tmc_emit.
-__global__ void __launch_bounds__(kBlock) k_tmc_vbase(VolTable vt, const uint32_t* __restrict__ acell,
-                                                       const uint32_t* __restrict__ acode,
-                                                       const uint32_t* __restrict__ vofs, int64_t A,
-                                                       uint2* __restrict__ avb) {
-    for (int64_t a = (int64_t)blockIdx.x * kBlock + threadIdx.x; a < A; a += (int64_t)gridDim.x * kBlock) {
-        const int vol = vol_of(vt.aBase, vt.n, a);
-        const VolDesc& V = vt.desc[vol];
-        int i, j, k;
-        uint32_t r;
-        cell_ijk(acell[a], V.d, i, j, k, r);
-        const unsigned own = tmc_cut_mask(acode[a] & 0xFFu) & tmc_owned_mask(i, j, k, V.d);
-        avb[a] = make_uint2(own, vofs[a]);
+// The vertex ids of a cell's cut edges, from the words and first vertices of
+// the cells that own them.  Owners are at most one row, one plane and one cell
+// back: three rows are looked up (the position of cell i there; cell i - 1 is
+// the one before), and only where a cut edge needs them.  At a lower side of
+// the grid the row before falls together with this one.  false: an owner does
+// not list the edge (never, as long as all cells see the same corner signs).
+struct TmcRef {
+    uint32_t code, first;
+};
+__device__ __forceinline__ bool tmc_edge_ids(const SegLists& L, const Dims& d, int64_t A, int64_t a, int i, int j,
+                                             int k, uint32_t code, uint32_t first, const uint32_t* __restrict__ acode,
+                                             const uint32_t* __restrict__ vofs, int32_t ev[12]) {
+    const unsigned cut = tmc_cut_mask(code & 0xFFu);
+    const bool di = i > 0, dj = j > 0, dk = k > 0;
+    const int64_t rs = L.rsBase + ((int64_t)k * (d.ny - 1) + j) * L.S + i / kSeg;
+    const int64_t up = L.S, upk = (int64_t)(d.ny - 1) * L.S;
+    // position of cell i of a row (where it is active; cell i - 1 is before it)
+    auto rank = [&](int64_t row) { return active_at(seg_words(L.mask, L.base, row), i); };
+    const bool wantK = dk && (cut & 0x00Eu || (cut & 1u && !dj));    // edges 1, 2, 3; 0
+    const bool wantJ = dj && (cut & 0x310u || (cut & 1u && !dk));    // edges 4, 8, 9; 0
+    const bool wantJK = dj && dk && (cut & 1u);
+    uint32_t atK = 0, atJ = 0, atJK = 0;
+    if (wantK) atK = rank(rs - upk);
+    if (wantJ) atJ = rank(rs - up);
+    if (wantJK) atJK = rank(rs - upk - up);
+    const TmcRef self{code, first};
+    const uint32_t last = (uint32_t)(A - 1);
+    auto ref = [&](uint32_t at) {
+        const uint32_t x = min(at, last);
+        return TmcRef{acode[x], vofs[x]};
+    };
+    TmcRef Sm = self, K0 = self, Km = self, J0 = self, Jm = self, JK0 = self;
+    if (di && cut & 0x988u) Sm = ref((uint32_t)a - 1u);   // edges 7, 11; 3 at k = 0, 8 at j = 0
+    if (wantK) K0 = ref(atK);
+    if (wantJ) J0 = ref(atJ);
+    if (wantJK) JK0 = ref(atJK);
+    Km = K0;
+    Jm = J0;
+    if (di) {
+        if (!dk) Km = Sm;
+        else if (cut & 0x008u) Km = ref(atK - 1u);
+        if (!dj) Jm = Sm;
+        else if (cut & 0x100u) Jm = ref(atJ - 1u);
     }
+    if (!(dj && dk)) JK0 = dj ? J0 : K0;
+    bool ok = true;
+    // edge e of this cell is edge oe of its owner
+    auto id = [&](int e, const TmcRef& o, int oe) {
+        const unsigned own = tmc_own(o.code);
+        ok = ok && (!((cut >> e) & 1u) || ((own >> oe) & 1u));
+        ev[e] = (int32_t)(o.first + (uint32_t)__popc(own & ((1u << oe) - 1u)));
+    };
+    id(0, JK0, (dj ? 2 : 0) + (dk ? 4 : 0));
+    id(1, K0, dk ? 5 : 1);
+    id(2, K0, dk ? 6 : 2);
+    id(3, Km, (dk ? 4 : 0) + (di ? 1 : 3));
+    id(4, J0, dj ? 6 : 4);
+    id(5, self, 5);
+    id(6, self, 6);
+    id(7, Sm, di ? 5 : 7);
+    id(8, Jm, dj ? (di ? 10 : 11) : (di ? 9 : 8));
+    id(9, J0, dj ? 10 : 9);
+    id(10, self, 10);
+    id(11, Sm, di ? 10 : 11);
+    return ok;
 }
 
 // Writing emitter: triangles with global vertex ids (edge refs through ev,
@@ -607,148 +643,196 @@ struct TmcWrite {
     }
 };
 
-// Vertices and triangles of active cell a.  AMB: the cell is ambiguous
-// (sliced with the decider, inner vertices); else the case table.  Owned
-// edge vertices take the gradients of their two corners only.
-template <class T, bool AMB>
-__device__ __forceinline__ void tmc_emit_cell(const VolTable& vt, int64_t a, const uint32_t* __restrict__ acell,
-                                              const uint32_t* __restrict__ acode,
-                                              const uint2* __restrict__ avb,
-                                              const uint32_t* __restrict__ tofs,
-                                              const unsigned long long* __restrict__ segMask,
-                                              const uint32_t* __restrict__ segBase, double* __restrict__ vpos,
-                                              double* __restrict__ vnrm, int32_t* __restrict__ tris,
-                                              unsigned long long* __restrict__ unresolved) {
-    const int vol = vol_of(vt.aBase, vt.n, a);
-    const VolDesc& V = vt.desc[vol];
-    const Dims d = V.d;
-    const GridGeom geo = V.geo;
-    const T* __restrict__ field = static_cast<const T*>(V.field);
-    const SegLists L{segMask, segBase, V.S, V.rsBase};
-    int i, j, k;
-    uint32_t r;
-    cell_ijk(acell[a], d, i, j, k, r);
-    const uint32_t code = acode[a];
-    const unsigned icase = code & 0xFFu;
-    const unsigned cut = tmc_cut_mask(icase);
-    const uint2 self = avb[a];
-    const unsigned own = self.x;
-    const double i0 = V.iso;
-    const int32_t vbase = (int32_t)self.y;
-    double F[8];
-    tmc_corners(field, d, i, j, k, F);
-    auto corner_pos = [&](int c, double p[3]) {
-        p[0] = geo.x0 + (i + (c & 1)) * geo.dx;
-        p[1] = geo.y0 + (j + ((c >> 1) & 1)) * geo.dy;
-        p[2] = geo.z0 + (k + (c >> 2)) * geo.dz;
-    };
-    int32_t ev[12];
-    int nown = 0;
-    // active index of each owner cell met, by its offset (i - oi) | (j - oj)
-    // << 1 | (k - ok) << 2 (-1: not looked up yet); the cell before in the
-    // row is the previous active cell
-    int64_t oidx[8];
-#pragma unroll
-    for (int x = 0; x < 8; x++) oidx[x] = -1;
-    oidx[1] = a - 1;
-    for (int e = 0; e < 12; e++) {
-        ev[e] = -1;
-        if (!((cut >> e) & 1u)) continue;
-        if ((own >> e) & 1u) {
-            ev[e] = vbase + nown++;
-            const int v0 = c_tmc_ev[e] & 0xF, v1 = c_tmc_ev[e] >> 4;
-            const double l = (i0 - F[v0]) / (F[v1] - F[v0]);
-            double P0[3], P1[3], N0[3], N1[3];
-            corner_pos(v0, P0);
-            corner_pos(v1, P1);
-            tmc_corner_gradient(field, d, geo, F, i, j, k, v0, N0);
-            tmc_corner_gradient(field, d, geo, F, i, j, k, v1, N1);
-            double* p = vpos + 3 * (int64_t)ev[e];
-            double* n = vnrm + 3 * (int64_t)ev[e];
-            double q[3];
-#pragma unroll
-            for (int x = 0; x < 3; x++) p[x] = (1 - l) * P0[x] + l * P1[x];
-#pragma unroll
-            for (int x = 0; x < 3; x++) q[x] = (1 - l) * N0[x] + l * N1[x];
-            const double s = sqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2]);
-            n[0] = q[0] / s;
-            n[1] = q[1] / s;
-            n[2] = q[2] / s;
-            continue;
-        }
-        int oi, oj, ok, oe;
-        tmc_edge_owner(i, j, k, e, d, oi, oj, ok, oe);
-        const int off = (i - oi) | (j - oj) << 1 | (k - ok) << 2;
-        int64_t ao = oidx[off];
-        if (ao < 0) {
-            ao = find_active(L, d, oi, oj, ok);
-            oidx[off] = ao;
-        }
-        if (ao < 0) {
-            atomicAdd(unresolved, 1ull);
-            continue;
-        }
-        const uint2 ob = avb[ao];
-        ev[e] = (int32_t)(ob.y + (uint32_t)__popc(ob.x & ((1u << oe) - 1u)));
-    }
-    const int64_t tbase = tofs[a];
-    if constexpr (AMB) {
-        if (code & 0x100u) return;   // singular face: no triangles
-        double P[8][3], N[8][3];
-        for (int c = 0; c < 8; c++) {
-            corner_pos(c, P[c]);
-            tmc_corner_gradient(field, d, geo, F, i, j, k, c, N[c]);
-        }
-        TmcWrite w{P, N, ev, vbase + nown, vpos, vnrm, tris, tbase};
-        tmc_slice(F, icase, i0, w);
-    } else {
-        const uint64_t wd = c_tmc_tri[icase];
-        const int nt = (int)(wd >> 60);
-        for (int t = 0; t < nt; t++) {
-            const int e0 = (int)((wd >> (12 * t)) & 0xF), e1 = (int)((wd >> (12 * t + 4)) & 0xF),
-                      e2 = (int)((wd >> (12 * t + 8)) & 0xF);
-            int32_t* o = tris + 3 * (tbase + t);
-            o[0] = ev[e2];   // reversed: positive corners outside
-            o[1] = ev[e1];
-            o[2] = ev[e0];
-        }
-    }
+// One component of the gradient at a grid point: central inside the grid,
+// one-sided at its border (mc/MarchingCubes.cpp:1450-1512); p at the point,
+// x its coordinate of n, s the stride.
+template <class T>
+__device__ __forceinline__ void tmc_around(const T* __restrict__ p, int x, int n, int64_t s, T& lo, T& hi) {
+    lo = p[x > 0 ? -s : 0];
+    hi = p[x < n - 1 ? s : 0];
+}
+template <class T>
+__device__ __forceinline__ double tmc_slope(T lo, T hi, int x, int n, double h, double rh2) {
+    const double e = (double)hi - (double)lo;
+    double g = div_by(e, 2 * h, rh2);
+    if (__builtin_expect(x == 0 || x == n - 1, 0)) g = e / h;
+    return g;
 }
 
-// K_T3: one thread per active cell that is not ambiguous (the case table).
+// K_T3: edge vertices of all active cells, table triangles of those that are
+// not ambiguous.  A block takes kBlock cells; their new vertices have
+// consecutive ids and so have their triangles, so both are listed in LDS and
+// given a thread each: consecutive threads write consecutive vertices, and a
+// vertex's 14 field values are in flight together.
+//
+// Bound by memory: at 1024^3 3.9 GB read (nearly the whole field again, in
+// lines of which a surface needs a few points) and 2.3 GB written, 3.0 TB/s.
+// (12 loads a vertex instead of 14, rows read as vectors, or stores staged
+// through LDS changed nothing.)  One thread
+// per cell that walked its twelve edges in turn ran vertices and lookups
+// divergently and scattered its writes: 4.35 + 0.20 ms at 1024^3 (a pass that
+// packed the owners' words included), now 2.09; 129^3 doubles 26 + 6 us, now 11.
 template <class T>
 __global__ void __launch_bounds__(kBlock) k_tmc_emit(VolTable vt, const uint32_t* __restrict__ acell,
                                                       const uint32_t* __restrict__ acode,
-                                                      const uint2* __restrict__ avb,
+                                                      const uint32_t* __restrict__ vofs,
                                                       const uint32_t* __restrict__ tofs,
                                                       const unsigned long long* __restrict__ segMask,
                                                       const uint32_t* __restrict__ segBase, int64_t A,
                                                       double* __restrict__ vpos, double* __restrict__ vnrm,
                                                       int32_t* __restrict__ tris,
                                                       unsigned long long* __restrict__ unresolved) {
-    for (int64_t a = (int64_t)blockIdx.x * kBlock + threadIdx.x; a < A; a += (int64_t)gridDim.x * kBlock) {
-        if (tmc_ambiguous(acode[a] & 0xFFu)) continue;
-        tmc_emit_cell<T, false>(vt, a, acell, acode, avb, tofs, segMask, segBase, vpos, vnrm, tris, unresolved);
+    __shared__ int32_t s_ev[12][kBlock];
+    __shared__ int s_i[kBlock], s_j[kBlock], s_k[kBlock];
+    __shared__ uint32_t s_code[kBlock], s_first[kBlock], s_tri[kBlock];
+    __shared__ uint16_t s_vert[12 * kBlock];   // cell of the block | edge << 8
+    __shared__ uint16_t s_tris[5 * kBlock];    // cell of the block | triangle << 8
+    __shared__ uint32_t s_sum[kBlock / kWave];
+    const VolDesc& V = vt.desc[0];
+    const Dims d = V.d;
+    const T* __restrict__ field = static_cast<const T*>(V.field);
+    const SegLists L{segMask, segBase, V.S, V.rsBase};
+    const int tid = threadIdx.x, wave = tid / kWave;
+    const int64_t sy = d.nx, sz = (int64_t)d.nx * d.ny;
+    for (int64_t a0 = (int64_t)blockIdx.x * kBlock; a0 < A; a0 += (int64_t)gridDim.x * kBlock) {
+        const int64_t a = a0 + tid;
+        uint32_t code = 0, nt = 0;
+        unsigned own = 0;
+        if (a < A) {
+            code = acode[a];
+            const uint32_t first = vofs[a], tri = tofs[a];
+            int i, j, k;
+            uint32_t r;
+            cell_ijk(acell[a], d, i, j, k, r);
+            own = tmc_own(code);
+            s_i[tid] = i;
+            s_j[tid] = j;
+            s_k[tid] = k;
+            s_code[tid] = code;
+            s_first[tid] = first;
+            s_tri[tid] = tri;
+            if (!tmc_ambiguous(code & 0xFFu)) {
+                nt = code >> 24;
+                int32_t ev[12];
+                if (!tmc_edge_ids(L, d, A, a, i, j, k, code, first, acode, vofs, ev)) atomicAdd(unresolved, 1ull);
+#pragma unroll
+                for (int e = 0; e < 12; e++) s_ev[e][tid] = ev[e];
+            }
+        }
+        // places in the two lists: prefix sums over the block, vertices in the
+        // low half (at most 12 * 256), triangles in the high one
+        const uint32_t mine = (uint32_t)__popc(own) | nt << 16;
+        uint32_t upto = mine;
+#pragma unroll
+        for (int w = 1; w < kWave; w *= 2) {
+            const uint32_t t = (uint32_t)__shfl_up((int)upto, w, kWave);
+            if ((tid & (kWave - 1)) >= w) upto += t;
+        }
+        if ((tid & (kWave - 1)) == kWave - 1) s_sum[wave] = upto;
+        __syncthreads();
+        uint32_t at = upto - mine, all = 0;
+#pragma unroll
+        for (int w = 0; w < kBlock / kWave; w++) {
+            if (w < wave) at += s_sum[w];
+            all += s_sum[w];
+        }
+        {
+            uint32_t p = at & 0xFFFFu;
+            for (unsigned m = own; m; m &= m - 1u) s_vert[p++] = (uint16_t)(tid | (__ffs(m) - 1) << 8);
+            p = at >> 16;
+            for (uint32_t t = 0; t < nt; t++) s_tris[p++] = (uint16_t)(tid | t << 8);
+        }
+        __syncthreads();
+        const uint32_t nv = all & 0xFFFFu, ntri = all >> 16;
+        for (uint32_t p = tid; p < nv; p += kBlock) {
+            const int c = s_vert[p] & 0xFF, e = s_vert[p] >> 8;
+            const uint32_t id = s_first[c] + (uint32_t)__popc(tmc_own(s_code[c]) & ((1u << e) - 1u));
+            // first point of the edge, axis
+            const int ax = e >= 8 ? 2 : e & 1;
+            const int x = s_i[c] + (int)(0x622u >> e & 1u), y = s_j[c] + (int)(0xC44u >> e & 1u),
+                      z = s_k[c] + (int)(0x0F0u >> e & 1u);
+            const int x1 = x + (ax == 0), y1 = y + (ax == 1), z1 = z + (ax == 2);
+            const T* p0 = field + (int64_t)z * sz + (int64_t)y * sy + x;
+            const T* p1 = p0 + (ax == 0 ? 1 : ax == 1 ? sy : sz);
+            T lo0[3], hi0[3], lo1[3], hi1[3];
+            const T f0 = *p0, f1 = *p1;
+            tmc_around(p0, x, d.nx, (int64_t)1, lo0[0], hi0[0]);
+            tmc_around(p0, y, d.ny, sy, lo0[1], hi0[1]);
+            tmc_around(p0, z, d.nz, sz, lo0[2], hi0[2]);
+            tmc_around(p1, x1, d.nx, (int64_t)1, lo1[0], hi1[0]);
+            tmc_around(p1, y1, d.ny, sy, lo1[1], hi1[1]);
+            tmc_around(p1, z1, d.nz, sz, lo1[2], hi1[2]);
+            const double F0 = (double)f0, l = (V.iso - F0) / ((double)f1 - F0);
+            const GridGeom geo = V.geo;
+            double q[3];
+            q[0] = (1 - l) * tmc_slope(lo0[0], hi0[0], x, d.nx, geo.dx, V.rdx2[0]) +
+                   l * tmc_slope(lo1[0], hi1[0], x1, d.nx, geo.dx, V.rdx2[0]);
+            q[1] = (1 - l) * tmc_slope(lo0[1], hi0[1], y, d.ny, geo.dy, V.rdx2[1]) +
+                   l * tmc_slope(lo1[1], hi1[1], y1, d.ny, geo.dy, V.rdx2[1]);
+            q[2] = (1 - l) * tmc_slope(lo0[2], hi0[2], z, d.nz, geo.dz, V.rdx2[2]) +
+                   l * tmc_slope(lo1[2], hi1[2], z1, d.nz, geo.dz, V.rdx2[2]);
+            const double s = sqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2]);
+            const double rs = 1.0 / s;
+            double* o = vpos + 3 * (int64_t)id;
+            o[0] = (1 - l) * (geo.x0 + x * geo.dx) + l * (geo.x0 + x1 * geo.dx);
+            o[1] = (1 - l) * (geo.y0 + y * geo.dy) + l * (geo.y0 + y1 * geo.dy);
+            o[2] = (1 - l) * (geo.z0 + z * geo.dz) + l * (geo.z0 + z1 * geo.dz);
+            double* n = vnrm + 3 * (int64_t)id;
+            n[0] = div_by(q[0], s, rs);
+            n[1] = div_by(q[1], s, rs);
+            n[2] = div_by(q[2], s, rs);
+        }
+        for (uint32_t p = tid; p < ntri; p += kBlock) {
+            const int c = s_tris[p] & 0xFF, t = s_tris[p] >> 8;
+            const uint32_t wd = (uint32_t)(c_tmc_tri[s_code[c] & 0xFFu] >> (12 * t));
+            int32_t* o = tris + 3 * ((int64_t)s_tri[c] + t);
+            o[0] = s_ev[wd >> 8 & 0xFu][c];   // reversed: positive corners outside
+            o[1] = s_ev[wd >> 4 & 0xFu][c];
+            o[2] = s_ev[wd & 0xFu][c];
+        }
+        __syncthreads();   // before the next cells
     }
 }
 
 // K_T4: the ambiguous cells k_tmc_cells listed (amb[0] = count, cells from
-// amb[1]): sliced with the asymptotic decider.
+// amb[1]): inner vertices and triangles, sliced with the asymptotic decider.
 template <class T>
 __global__ void __launch_bounds__(kBlock) k_tmc_emit_amb(VolTable vt, const uint32_t* __restrict__ amb,
                                                           const uint32_t* __restrict__ acell,
                                                           const uint32_t* __restrict__ acode,
-                                                          const uint2* __restrict__ avb,
+                                                          const uint32_t* __restrict__ vofs,
                                                           const uint32_t* __restrict__ tofs,
                                                           const unsigned long long* __restrict__ segMask,
-                                                          const uint32_t* __restrict__ segBase,
+                                                          const uint32_t* __restrict__ segBase, int64_t A,
                                                           double* __restrict__ vpos, double* __restrict__ vnrm,
                                                           int32_t* __restrict__ tris,
                                                           unsigned long long* __restrict__ unresolved) {
-    const uint32_t n = amb[0];
-    for (uint32_t s = blockIdx.x * kBlock + threadIdx.x; s < n; s += gridDim.x * kBlock)
-        tmc_emit_cell<T, true>(vt, (int64_t)amb[1 + s], acell, acode, avb, tofs, segMask, segBase, vpos, vnrm, tris,
-                               unresolved);
+    const uint32_t cells = amb[0];
+    const VolDesc& V = vt.desc[0];
+    const Dims d = V.d;
+    const GridGeom geo = V.geo;
+    const T* __restrict__ field = static_cast<const T*>(V.field);
+    const SegLists L{segMask, segBase, V.S, V.rsBase};
+    for (uint32_t s = blockIdx.x * kBlock + threadIdx.x; s < cells; s += gridDim.x * kBlock) {
+        const uint32_t a = amb[1 + s], code = acode[a];
+        if (code & 0x100u) continue;   // singular face: no triangles
+        int i, j, k;
+        uint32_t r;
+        cell_ijk(acell[a], d, i, j, k, r);
+        const uint32_t first = vofs[a];
+        int32_t ev[12];
+        if (!tmc_edge_ids(L, d, A, a, i, j, k, code, first, acode, vofs, ev)) atomicAdd(unresolved, 1ull);
+        double F[8], P[8][3], N[8][3];
+        tmc_corners(field, d, i, j, k, F);
+        for (int c = 0; c < 8; c++) {
+            P[c][0] = geo.x0 + (i + (c & 1)) * geo.dx;
+            P[c][1] = geo.y0 + (j + ((c >> 1) & 1)) * geo.dy;
+            P[c][2] = geo.z0 + (k + (c >> 2)) * geo.dz;
+            tmc_corner_gradient(field, d, geo, F, i, j, k, c, N[c]);
+        }
+        TmcWrite w{P, N, ev, (int32_t)(first + (uint32_t)__popc(tmc_own(code))), vpos, vnrm, tris, (int64_t)tofs[a]};
+        tmc_slice(F, code & 0xFFu, V.iso, w);
+    }
 }
 
 }  // namespace tmc
