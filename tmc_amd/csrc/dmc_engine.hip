@@ -147,6 +147,7 @@ struct dmc_context {
     // overflowed, raised to its exact sizes (the *_min, one extraction long)
     int64_t acap = 0, vcap = 0, qcap = 0, reccap = 0;
     int64_t acap_min = 0, vcap_min = 0, qcap_min = 0;
+    int64_t qexpect = 0;       // quadrilaterals the densities seen so far give (0: none seen)
     double rcell[3] = {0, 0, 0}, rarea[3] = {0, 0, 0};
     Sizes hsz{};               // the last pass's sizes block
     // captured passes (replayed when a pass of the same shape comes again)
@@ -748,6 +749,7 @@ void plan_caps(dmc_context* ctx, const std::vector<HostVol>& hv, int64_t cells) 
     ctx->acap = std::max({cap_step(ctx->acap_min), cap(0), floor});
     ctx->vcap = std::max({cap_step(ctx->vcap_min), cap(1), floor});
     ctx->qcap = std::max({cap_step(ctx->qcap_min), cap(2), floor});
+    ctx->qexpect = (int64_t)std::max(std::ceil(est[2]), (double)ctx->qcap_min);
     ctx->acap = std::min<int64_t>(std::min<int64_t>(ctx->acap, cells), 0xFFFFFFFF);
     ctx->vcap = std::min<int64_t>(ctx->vcap, 0x7FFFFFFF);
     ctx->qcap = std::min<int64_t>(ctx->qcap, 0x1FFFFFFF);
@@ -916,9 +918,6 @@ void finish_halfedges(dmc_context* ctx, bool compacted) {
     check_launch(ctx, "k_finish");
 }
 
-// Meshes of at most this many faces are coloured by one block.
-constexpr int64_t kSmallColourFaces = (int64_t)1 << 14;
-
 // Colour classes that run in one launch.  Class c holds the faces of initial
 // colour c = 3 * parity + direction of their grid edge, and a face reads the
 // colours of its edge neighbours.  Two quadrilaterals share a mesh edge only
@@ -944,6 +943,7 @@ bool classes_touch(int c1, int c2) {
 struct ColourLevels {
     int n = 0;
     int cls[20][2];
+    ClassLevels of{};   // level of each class
 };
 
 const ColourLevels& colour_levels() {
@@ -959,40 +959,47 @@ const ColourLevels& colour_levels() {
                 if (classes_touch(order[i], order[j])) lv = std::max(lv, level[order[j]] + 1);
             level[order[i]] = lv;
             r.n = std::max(r.n, lv + 1);
+            r.of.of[order[i]] = (uint8_t)lv;
             int* slot = r.cls[lv];
             if (slot[0] < 0) slot[0] = order[i];
             else if (slot[1] < 0) slot[1] = order[i];
             else throw std::logic_error("three colour classes in one level");
         }
+        r.of.n = r.n;
         return r;
     }();
     return L;
+}
+
+// One block colours the pass: its faces fit, and no more are expected than
+// the block holds in registers.
+bool small_colouring(const dmc_context* ctx) {
+    return ctx->qcap <= kSmallColourFaces && ctx->qexpect <= kColourHeld;
 }
 
 void color_faces(dmc_context* ctx) {
     const int64_t qcap = ctx->qcap;
     Sizes* S = dsizes(ctx);
     uint8_t* colors = static_cast<uint8_t*>(ctx->colors.p);
+    const int32_t* twin = static_cast<int32_t*>(ctx->twin.p);
+    const ColourLevels& L = colour_levels();
+    if (small_colouring(ctx)) {
+        launch(ctx, "k_color_small", k_color_small, dim3(1), dim3(1024), twin, (const Sizes*)S, L.of, colors);
+        check_launch(ctx, "colour");
+        return;
+    }
     // one histogram block per 4096 faces of capacity, at most kColorBlocks
     const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(kColorBlocks, qcap / 4096));
     uint32_t* hist = ensure<uint32_t>(ctx, ctx->ccnt, (size_t)kColorBlocks * 24);
     int32_t* list = ensure<int32_t>(ctx, ctx->clist, qcap);
     int4* nbr = ensure<int4>(ctx, ctx->cnbr, qcap);
-    const int32_t* twin = static_cast<int32_t*>(ctx->twin.p);
     launch(ctx, "k_color_hist", k_color_hist, dim3(nb), dim3(kBlock), (const uint8_t*)colors, (const Sizes*)S, hist);
     launch(ctx, "k_color_offsets", k_color_offsets, dim3(1), dim3(1024), hist, nb, S->colors);
     launch(ctx, "k_color_scatter", k_color_scatter, dim3(nb), dim3(kBlock), (const uint8_t*)colors, (const Sizes*)S,
            (const uint32_t*)hist, twin, list, nbr);
-    if (qcap <= kSmallColourFaces) {
-        launch(ctx, "k_color_class", k_color_all, dim3(1), dim3(1024), (const int32_t*)list, (const int4*)nbr,
-               (const uint32_t*)S->colors, colors);
-        check_launch(ctx, "colour");
-        return;
-    }
     // a class holds at most a quarter of the faces (four parities of one
     // edge direction), a launch at most two classes
     const int g = grid_for(ctx, qcap / 2 + 1);
-    const ColourLevels& L = colour_levels();
     for (int lv = 0; lv < L.n; lv++)
         launch(ctx, "k_color_class", k_color_class, dim3(g), dim3(kBlock), (const int32_t*)list, (const int4*)nbr,
                (const uint32_t*)S->colors, L.cls[lv][0], L.cls[lv][1], colors);
@@ -1625,6 +1632,7 @@ std::string pass_key(dmc_context* ctx, const std::vector<HostVol>& hv, const Swe
     put(ctx->qcap);
     put(ctx->reccap);
     put(ctx->force_generic);
+    put(small_colouring(ctx));
     put((int64_t)ctx->buf_epoch);
     put((int64_t)hv.size());
     for (const HostVol& h : hv) put(((int64_t)h.g.nx << 42) | ((int64_t)h.g.ny << 21) | h.g.nz);

@@ -397,16 +397,18 @@ __device__ __forceinline__ int4 face_neighbors(const int32_t* __restrict__ twin,
                      t.w >= 0 ? t.w >> 2 : -1);
 }
 
-// First colour in 0..ncol-1 that none of the neighbours nb has.
+// First colour in 0..ncol-1 that none of the neighbours nb has (they have
+// 0..23), if there is one.
 __device__ __forceinline__ void take_free_colour(const int4 nb, int ncol, int32_t f, uint8_t* __restrict__ colors) {
-    const int c0 = nb.x >= 0 ? colors[nb.x] : -1, c1 = nb.y >= 0 ? colors[nb.y] : -1;
-    const int c2 = nb.z >= 0 ? colors[nb.z] : -1, c3 = nb.w >= 0 ? colors[nb.w] : -1;
-    for (int col = 0; col < ncol; col++) {
-        if (c0 != col && c1 != col && c2 != col && c3 != col) {
-            colors[f] = (uint8_t)col;
-            break;
-        }
-    }
+    // all four read, in flight together
+    const uint32_t c0 = colors[max(nb.x, 0)], c1 = colors[max(nb.y, 0)], c2 = colors[max(nb.z, 0)],
+                   c3 = colors[max(nb.w, 0)];
+    uint32_t used = ~0u << ncol;
+    used |= nb.x >= 0 ? 1u << (c0 & 31) : 0u;
+    used |= nb.y >= 0 ? 1u << (c1 & 31) : 0u;
+    used |= nb.z >= 0 ? 1u << (c2 & 31) : 0u;
+    used |= nb.w >= 0 ? 1u << (c3 & 31) : 0u;
+    if (~used) colors[f] = (uint8_t)(__ffs(~used) - 1);
 }
 
 // Face colouring (cpp_dmc/DualMarchingCubes.cpp:714-844).  Colours are
@@ -456,7 +458,8 @@ __global__ void __launch_bounds__(1024) k_color_offsets(uint32_t* __restrict__ h
 #pragma unroll
         for (int q = 0; q < 16; q++) {
             const int b = lane + kWave * q;
-            v[h][q] = (c < 24 && b < nblocks) ? hist[b * 24 + c] : 0u;
+            v[h][q] = 0;
+            if (kWave * q < nblocks) v[h][q] = (c < 24 && b < nblocks) ? hist[b * 24 + c] : 0u;
         }
         uint32_t sum = 0;
 #pragma unroll
@@ -482,6 +485,7 @@ __global__ void __launch_bounds__(1024) k_color_offsets(uint32_t* __restrict__ h
         uint32_t run = start[c];
 #pragma unroll
         for (int q = 0; q < 16; q++) {
+            if (kWave * q >= nblocks) break;
             const int b = lane + kWave * q;
             const uint32_t inc = wave_inclusive_scan(v[h][q]);
             if (b < nblocks) hist[b * 24 + c] = run + inc - v[h][q];
@@ -523,22 +527,58 @@ __global__ void __launch_bounds__(kBlock) k_color_class(const int32_t* __restric
     }
 }
 
-// All classes in one block, in order, for a small mesh (one launch instead
-// of twenty): the same first-free-colour rule, a barrier between classes.
-__global__ void __launch_bounds__(1024) k_color_all(const int32_t* __restrict__ list,
-                                                     const int4* __restrict__ nbr,
-                                                     const uint32_t* __restrict__ totals,
-                                                     uint8_t* __restrict__ colors) {
-    for (int step = 0; step < 20; step++) {
-        const int cls = step < 19 ? 5 + step : 4;
-        const int ncol = step < 19 ? 5 : 4;
-        const int64_t n = totals[cls], start = totals[24 + cls];
-        for (int64_t x = threadIdx.x; x < n; x += blockDim.x)
-            take_free_colour(nbr[start + x], ncol, list[start + x], colors);
-        // the next class reads this one's colours
-        __threadfence_block();
-        __syncthreads();
+// The colouring of a small mesh by one block, level by level with the colours
+// in LDS and a barrier between levels: a launch per level took 2.3 us each,
+// and the lists in class order 20 us before them (32^3, 3,400 faces: 14 + 3
+// launches, 52 us, now 13).  A face's level is that of its initial colour,
+// none for the classes 0..3.  The block's first kColourHeld faces keep their
+// neighbours in registers; further ones (up to kSmallColourFaces) read them
+// again at their level, which is slower than the lists (28^3 noise, 20,000
+// faces: 130 us more), so the caller expects no more than kColourHeld.
+constexpr int kSmallColourFaces = 1 << 15;
+constexpr int kColourIpt = 8, kColourHeld = kColourIpt * 1024;
+struct ClassLevels {
+    uint8_t of[24];
+    int n;
+};
+__global__ void __launch_bounds__(1024) k_color_small(const int32_t* __restrict__ twin, const Sizes* S, ClassLevels L,
+                                                       uint8_t* __restrict__ colors) {
+    constexpr uint8_t kNone = 0x7F;
+    __shared__ uint8_t col[kSmallColourFaces];
+    __shared__ uint8_t todo[kSmallColourFaces - kColourHeld];   // level | 0x80 for class 4
+    const int nq = (int)min((int64_t)S->nq, (int64_t)kSmallColourFaces);
+    auto level_of = [&](int c) { return c < 4 || c >= 24 ? kNone : (uint8_t)(L.of[c] | (c == 4 ? 0x80 : 0)); };
+    int4 nb[kColourIpt];
+    uint8_t mine[kColourIpt];
+#pragma unroll
+    for (int q = 0; q < kColourIpt; q++) {
+        const int f = (int)threadIdx.x + 1024 * q;
+        mine[q] = kNone;
+        if (f < nq) {
+            const int c = colors[f];
+            nb[q] = face_neighbors(twin, f);
+            col[f] = (uint8_t)c;
+            mine[q] = level_of(c);
+        }
     }
+    for (int f = kColourHeld + (int)threadIdx.x; f < nq; f += 1024) {
+        const int c = colors[f];
+        col[f] = (uint8_t)c;
+        todo[f - kColourHeld] = level_of(c);
+    }
+    __syncthreads();
+    for (int level = 0; level < L.n; level++) {
+#pragma unroll
+        for (int q = 0; q < kColourIpt; q++)
+            if (1024 * q < nq && (mine[q] & 0x7F) == level)
+                take_free_colour(nb[q], mine[q] & 0x80 ? 4 : 5, (int)threadIdx.x + 1024 * q, col);
+        for (int f = kColourHeld + (int)threadIdx.x; f < nq; f += 1024) {
+            const int td = todo[f - kColourHeld];
+            if ((td & 0x7F) == level) take_free_colour(face_neighbors(twin, f), td & 0x80 ? 4 : 5, f, col);
+        }
+        __syncthreads();   // the next level reads this one's colours
+    }
+    for (int f = threadIdx.x; f < nq; f += 1024) colors[f] = col[f];
 }
 
 // 3X3Y pattern (cpp_dmc/DualMarchingCubes.cpp:889-913)
