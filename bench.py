@@ -617,15 +617,12 @@ def main():
                                "colour byte (V, Q before simplification)"}
     # per-kernel figures: device ms per extraction (HIP events), bytes by
     # each kernel's own model
-    R = (grid.ny - 1) * (grid.nz - 1)
     models = {
         "k_sweep": (4 * nvox, "4 N (field read once)"),
         "k_cells": (4 * A + 16 * A, "4 A list entries read + 16 A per-cell records written"),
         "k_vertices": (24 * V, "24 V (FP32 position + normal; the engine writes FP64, 48 V)"),
-        "k_quads": (17 * Q + 32 * Q, "17 Q (int4 quad + colour) + 32 Q (first halfedge rows)"),
-        "k_he_twins": (16 * Q + 32 * Q + 20 * Q + 4 * V,
-                       "16 Q quads + 32 Q halfedge rows read, 20 Q twins and flags + 4 V he_v written (the one "
-                       "build through rows, on the cell stage's V, Q; later builds are carried over)"),
+        "k_quads": (16 * A + 17 * Q + 20 * Q + 4 * V,
+                    "16 A records read; 17 Q (int4 quad + colour) + 20 Q (twins and flags) + 4 V he_v written"),
         "k_triangles": (16 * Qf + 24 * Qf + 24 * 4 * Qf, "16 Q quads + 96 Q positions read, 24 Q written"),
     }
     kernels = []

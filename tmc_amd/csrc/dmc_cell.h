@@ -266,22 +266,27 @@ __device__ __forceinline__ void local_coords(int e, float l, double u[3]) {
     }
 }
 
-// Per-contour bounding boxes live in LDS, one column per thread: entry
-// (axis, lo/hi, contour) of thread x is at base[((axis*2 + hi)*4 + t) * 256 + x].
-// All entries are floats widened to double in the reference, so float
-// storage is exact.
+// Bounding boxes of contours live in LDS, one column per thread: entry (axis,
+// lo/hi, contour) of thread x is at base[((axis*2 + hi)*N + t) * 256 + x].  N is
+// 4 where a contour's samples avoid the others' boxes, 1 (t taken as 0) where
+// only its own is needed.  All entries are floats widened to double in the
+// reference, so float storage is exact.
 constexpr int kBoxStride = 256;
-constexpr int kBoxFloats = 24;
-
-struct BoxRef {
-    float* p;   // &box[0][threadIdx.x] of a [24][kBoxStride] LDS array
-    __device__ __forceinline__ float lo(int ax, int t) const { return p[((ax * 2) * 4 + t) * kBoxStride]; }
-    __device__ __forceinline__ float hi(int ax, int t) const { return p[((ax * 2 + 1) * 4 + t) * kBoxStride]; }
+template <int N>
+struct Boxes {
+    static constexpr int kFloats = 6 * N;
+    float* p;   // &box[0][threadIdx.x] of a [kFloats][kBoxStride] LDS array
+    __device__ __forceinline__ float* at(int ax, int hi, int t) const {
+        return p + ((ax * 2 + hi) * N + (N == 1 ? 0 : t)) * kBoxStride;
+    }
+    __device__ __forceinline__ float lo(int ax, int t) const { return *at(ax, 0, t); }
+    __device__ __forceinline__ float hi(int ax, int t) const { return *at(ax, 1, t); }
     __device__ __forceinline__ void set(int ax, int t, float l, float h) const {
-        p[((ax * 2) * 4 + t) * kBoxStride] = l;
-        p[((ax * 2 + 1) * 4 + t) * kBoxStride] = h;
+        *at(ax, 0, t) = l;
+        *at(ax, 1, t) = h;
     }
 };
+using BoxRef = Boxes<4>;
 
 // cpp_dmc/DualMarchingCubes.h:590-597
 __device__ __forceinline__ void trilinear_gradient(const CornerRef& f, double u, double v, double w, double g[3]) {
@@ -302,7 +307,8 @@ struct ProjFrame {
     double umin, vmin, du, dv, wmin, wmax;
 };
 
-__device__ __forceinline__ ProjFrame proj_frame(const BoxRef& B, int axa, int axb, int axc, int t, int ns) {
+template <class Box>
+__device__ __forceinline__ ProjFrame proj_frame(const Box& B, int axa, int axb, int axc, int t, int ns) {
     ProjFrame f;
     const double umax = B.hi(axa, t), vmax = B.hi(axb, t);
     f.umin = B.lo(axa, t);
@@ -341,8 +347,8 @@ __device__ __forceinline__ void proj_row(const CornerRef& Fc, uint32_t cpk, floa
 // exactly as the reference's skip of that sample.
 // kUnroll: how many of a row's 7 samples the compiler interleaves (7: the
 // most instruction-level parallelism, 1: the fewest registers).
-template <int kUnroll>
-__device__ inline bool projection9(const CornerRef& Fc, uint32_t cpk, const BoxRef& B, int axa, int axb, int axc,
+template <int kUnroll, class Box>
+__device__ inline bool projection9(const CornerRef& Fc, uint32_t cpk, const Box& B, int axa, int axb, int axc,
                                    double iso, int t, double p[3]) {
     constexpr int ns = 9;
     constexpr int kIn = ns - 2;  // interior samples per axis: i, j = 1 .. 7
@@ -516,10 +522,17 @@ struct ContourFrame {
     uint32_t cpk;
 };
 
-__device__ inline ContourFrame contour_frame(const CornerRef& Fc, double iso, uint64_t w, int t, const BoxRef& B,
-                                             double p[3], double pt[3]) {
-    // mean of the edge intersections, summed in contour order
+// Mean of the edge intersections of contour t, summed in contour order, and
+// their bounding box (cpp_dmc/DualMarchingCubes.cpp:113-139): one loop, since
+// an intersection costs a division and its placing in the cell.  With a loop
+// for the boxes of all contours and one for the mean, k_vertices took 3.00 ms
+// at 1024^3 (now 2.83), 2.21 on 1,024 small volumes (2.08), 388 us at 385^3 F64
+// (370).  (The mean by the size's reciprocal instead of divisions: 2.87.)
+template <class Box>
+__device__ inline void contour_mean_box(const CornerRef& Fc, double iso, uint64_t w, int t, const Box& B,
+                                        double p[3]) {
     const int start = poly_start(w, t), size = poly_size(w, t);
+    float lo[3] = {1.f, 1.f, 1.f}, hi[3] = {0.f, 0.f, 0.f};
     p[0] = 0;
     p[1] = 0;
     p[2] = 0;
@@ -527,13 +540,24 @@ __device__ inline ContourFrame contour_frame(const CornerRef& Fc, double iso, ui
         const int e = poly_edge_at(w, start + m);
         double ui[3];
         local_coords(e, edge_param(e, Fc, iso), ui);
-        p[0] += ui[0];
-        p[1] += ui[1];
-        p[2] += ui[2];
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            p[c] += ui[c];
+            const float x = (float)ui[c];
+            lo[c] = lo[c] > x ? x : lo[c];
+            hi[c] = hi[c] < x ? x : hi[c];
+        }
     }
     p[0] /= size;
     p[1] /= size;
     p[2] /= size;
+#pragma unroll
+    for (int c = 0; c < 3; c++) B.set(c, t, lo[c], hi[c]);
+}
+
+template <class Box>
+__device__ inline ContourFrame contour_frame(const CornerRef& Fc, int size, int t, const Box& B, const double p[3],
+                                             double pt[3]) {
     // projection axis: W = 1, V = 2, U = 3
     int prj;
     if (size >= 6) {
@@ -596,11 +620,12 @@ __device__ __forceinline__ bool cell_needs_box_test(uint64_t w, int cnt) {
 // Representative of contour t of a cell without the box test, from the 9 x 9
 // sampling; false when that sampling finds no point (the caller then takes
 // the general path, which also samples at 28 x 28).
-template <int kUnroll>
-__device__ inline bool contour_representative9(const CornerRef& Fc, double iso, uint64_t w, int t, const BoxRef& B,
+template <int kUnroll, class Box>
+__device__ inline bool contour_representative9(const CornerRef& Fc, double iso, uint64_t w, int t, const Box& B,
                                                double p[3]) {
     double pt[3];
-    const ContourFrame f = contour_frame(Fc, iso, w, t, B, p, pt);
+    contour_mean_box(Fc, iso, w, t, B, p);
+    const ContourFrame f = contour_frame(Fc, poly_size(w, t), t, B, p, pt);
     if (!projection9<kUnroll>(Fc, f.cpk, B, f.axa, f.axb, f.axc, iso, t, pt)) return false;
     contour_unframe(f, pt, p);
     return true;
@@ -612,7 +637,8 @@ __device__ inline bool contour_representative9(const CornerRef& Fc, double iso, 
 __device__ inline int contour_representative(const CornerRef& Fc, double iso, uint64_t w, int cnt, int t,
                                              const BoxRef& B, double p[3]) {
     double pt[3];
-    const ContourFrame f = contour_frame(Fc, iso, w, t, B, p, pt);
+    contour_mean_box(Fc, iso, w, t, B, p);
+    const ContourFrame f = contour_frame(Fc, poly_size(w, t), t, B, p, pt);
     // size-3 contours of the cell other than t whose boxes samples must avoid
     unsigned nbmask = 0;
 #pragma unroll
@@ -625,27 +651,6 @@ __device__ inline int contour_representative(const CornerRef& Fc, double iso, ui
     }
     contour_unframe(f, pt, p);
     return fails;
-}
-
-// Bounding boxes of all contours (cpp_dmc/DualMarchingCubes.cpp:113-139).
-__device__ inline void cell_boxes(const CornerRef& Fc, double iso, uint64_t w, int cnt, const BoxRef& B) {
-    for (int t = 0; t < cnt; t++) {
-        const int start = poly_start(w, t), size = poly_size(w, t);
-        float lo[3] = {1.f, 1.f, 1.f}, hi[3] = {0.f, 0.f, 0.f};
-        for (int m = 0; m < size; m++) {
-            const int e = poly_edge_at(w, start + m);
-            double ui[3];
-            local_coords(e, edge_param(e, Fc, iso), ui);
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                const float x = (float)ui[c];
-                lo[c] = lo[c] > x ? x : lo[c];
-                hi[c] = hi[c] < x ? x : hi[c];
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < 3; c++) B.set(c, t, lo[c], hi[c]);
-    }
 }
 
 }  // namespace tmc

@@ -56,7 +56,7 @@ constexpr size_t kMaxSeen = 4096;
 constexpr int kCaptureAfter = 2;
 // capacity floor of a pass: its cells, up to this many
 constexpr int64_t kSmallPassCells = (int64_t)1 << 18;
-// k_vertices blocks: 256 CUs x 2 resident blocks (40 KB of LDS, 256 VGPRs
+// k_vertices blocks: 256 CUs x 2 resident blocks (22 KB of LDS, 235 VGPRs
 // each) x 4 rounds
 constexpr int64_t kVerticesBlocks = 2048;
 
@@ -2137,8 +2137,7 @@ static void diag_mesh_ok(dmc_context* ctx) {
 }
 
 // The final mesh's halfedge rows (off/adj), counted from the quadrilaterals
-// when the final build was carried over from a compaction and paired
-// without them.
+// when its twins were written without them.
 static void ensure_rows(dmc_context* ctx) {
     if (ctx->rows_live) return;
     Sizes* S = dsizes(ctx);

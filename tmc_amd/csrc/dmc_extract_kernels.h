@@ -723,9 +723,9 @@ __device__ __forceinline__ void vertices_run(const VolTable& vt, const uint4* __
                                              uint32_t* __restrict__ slow, unsigned long long* qhead) {
     static_assert(kBlock == kBoxStride && kBlock == kCornerStride, "LDS columns are one per thread");
     const int64_t A = dA.get();
-    __shared__ float boxes[kBoxFloats * kBoxStride];
+    __shared__ float boxes[Boxes<1>::kFloats * kBoxStride];
     __shared__ double corners[8 * kCornerStride];
-    const BoxRef B{boxes + threadIdx.x};
+    const Boxes<1> B{boxes + threadIdx.x};
     const CornerRef Fc{corners + threadIdx.x};
     // Persistent blocks pull chunks of kVerticesChunk x kBlock active cells
     // from a device work queue (*qhead, ascending): cells cost unevenly (one
@@ -763,7 +763,6 @@ __device__ __forceinline__ void vertices_run(const VolTable& vt, const uint4* __
             // issued before the sampling, which hides their latency
             OuterValues<T> o;
             if (!V.grads) load_outer<T>(V, i, j, k, o);
-            cell_boxes(Fc, iso, w, cnt, B);
             const uint32_t aux = R.aux;
             const unsigned used = R.used();
             uint32_t out = first_vertex(V, r, i, R, grpV);
@@ -827,7 +826,7 @@ __global__ void __launch_bounds__(kBlock) k_vertices_slow(VolTable vt, const uin
                                                           double* __restrict__ vpos, double* __restrict__ vnrm,
                                                           VertexOut vo,
                                                           VolStat* __restrict__ vstat) {
-    __shared__ float boxes[kBoxFloats * kBoxStride];
+    __shared__ float boxes[BoxRef::kFloats * kBoxStride];
     __shared__ double corners[8 * kCornerStride];
     const BoxRef B{boxes + threadIdx.x};
     const CornerRef Fc{corners + threadIdx.x};
@@ -847,7 +846,11 @@ __global__ void __launch_bounds__(kBlock) k_vertices_slow(VolTable vt, const uin
         const int cnt = poly_count(w);
         OuterValues<T> o;
         if (!V.grads) load_outer<T>(V, i, j, k, o);
-        cell_boxes(Fc, iso, w, cnt, B);
+        // the boxes of all contours, which the samples of any may have to avoid
+        for (int t = 0; cnt > 1 && t < cnt; t++) {
+            double mean[3];
+            contour_mean_box(Fc, iso, w, t, B, mean);
+        }
         const uint32_t aux = R.aux;
         const unsigned used = R.used();
         uint32_t out = first_vertex(V, r, i, R, grpV);

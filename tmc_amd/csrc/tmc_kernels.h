@@ -665,8 +665,9 @@ __device__ __forceinline__ double tmc_slope(T lo, T hi, int x, int n, double h, 
 // given a thread each: consecutive threads write consecutive vertices, and a
 // vertex's 14 field values are in flight together.
 //
-// Bound by memory: at 1024^3 3.9 GB read (nearly the whole field again, in
-// lines of which a surface needs a few points) and 2.3 GB written, 3.0 TB/s.
+// Bound by memory: at 1024^3 7.9 GB read (the field's lines around the surface,
+// of which it needs a few points, by more than one L2) and 2.4 GB written, 4.9
+// TB/s.
 // (12 loads a vertex instead of 14, rows read as vectors, or stores staged
 // through LDS changed nothing.)  One thread
 // per cell that walked its twelve edges in turn ran vertices and lookups
