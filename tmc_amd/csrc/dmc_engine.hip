@@ -829,10 +829,10 @@ void run_cells(dmc_context* ctx, const SweepPlan& P, bool live) {
     // threads (F32 fields: the F64 form would spill at 3 waves)
     const dim3 gv(grid_for(ctx, acap, kBlock, kVerticesBlocks));
     if (std::is_same<T, float>::value && acap > kVerticesBlocks * kBlock)
-        launch(ctx, "k_vertices", k_vertices_wide<T>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, vo, slow,
+        launch(ctx, "k_vertices", n > 1 ? k_vertices_wide<T, true> : k_vertices_wide<T, false>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, vo, slow,
                &S->qhead);
     else
-        launch(ctx, "k_vertices", k_vertices<T>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, vo, slow,
+        launch(ctx, "k_vertices", n > 1 ? k_vertices<T, true> : k_vertices<T, false>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, vo, slow,
                &S->qhead);
     check_launch(ctx, "k_vertices");
     launch(ctx, "k_vertices_slow", k_vertices_slow<T>, dim3(grid_for(ctx, acap, kBlock, 1024)), dim3(kBlock), vt,

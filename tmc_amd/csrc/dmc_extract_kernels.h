@@ -715,7 +715,7 @@ __device__ __forceinline__ void store_vertex(const VolDesc& V, int i, int j, int
     }
 }
 
-template <class T, int kUnroll>
+template <class T, int kUnroll, bool MANY>
 __device__ __forceinline__ void vertices_run(const VolTable& vt, const uint4* __restrict__ rec,
                                              const uint32_t* __restrict__ grpV, DevN dA,
                                              double* __restrict__ vpos, double* __restrict__ vnrm,
@@ -723,6 +723,11 @@ __device__ __forceinline__ void vertices_run(const VolTable& vt, const uint4* __
                                              uint32_t* __restrict__ slow, unsigned long long* qhead) {
     static_assert(kBlock == kBoxStride && kBlock == kCornerStride, "LDS columns are one per thread");
     const int64_t A = dA.get();
+    // one volume (MANY false): its descriptor in scalar registers, instead of
+    // vector loads from the table after every store -- 1024^3 2.82 -> 2.70 ms,
+    // 385^3 F64 370 -> 354 us, 128^3 22.3 -> 20.5 (the general path gets slower
+    // with it: 256 VGPRs, 512^3 blobs 380 -> 578 us)
+    const VolDesc V0 = vt.desc[0];
     __shared__ float boxes[Boxes<1>::kFloats * kBoxStride];
     __shared__ double corners[8 * kCornerStride];
     const Boxes<1> B{boxes + threadIdx.x};
@@ -747,8 +752,8 @@ __device__ __forceinline__ void vertices_run(const VolTable& vt, const uint4* __
         for (int round = 0; round < rounds; round++) {
         const int64_t a = c0 + (int64_t)round * kBlock + threadIdx.x;
         if (a >= A) continue;
-        const int vol = vol_of(vt.aBase, vt.n, a);
-        const VolDesc& V = vt.desc[vol];
+        const int vol = MANY ? vol_of(vt.aBase, vt.n, a) : 0;
+        const VolDesc& V = MANY ? vt.desc[vol] : V0;
         const double iso = V.iso;
         const ActRec R = load_rec(rec, a);
         const uint32_t code = R.code;
@@ -794,13 +799,13 @@ __device__ __forceinline__ void vertices_run(const VolTable& vt, const uint4* __
 // K3 for passes of up to one round of the persistent grid's threads per
 // active cell: a row's samples interleaved (the latency of one cell matters
 // most), 2 waves per SIMD.
-template <class T>
+template <class T, bool MANY>
 __global__ void __launch_bounds__(kBlock) TMC_VERTICES_ATTR k_vertices(VolTable vt, const uint4* __restrict__ rec,
                                                       const uint32_t* __restrict__ grpV, DevN dA,
                                                       double* __restrict__ vpos, double* __restrict__ vnrm,
                                                       VertexOut vo,
                                                       uint32_t* __restrict__ slow, unsigned long long* qhead) {
-    vertices_run<T, 7>(vt, rec, grpV, dA, vpos, vnrm, vo, slow, qhead);
+    vertices_run<T, 7, MANY>(vt, rec, grpV, dA, vpos, vnrm, vo, slow, qhead);
 }
 
 // K3 for larger passes: samples one at a time, which fits 3 waves per SIMD
@@ -808,12 +813,12 @@ __global__ void __launch_bounds__(kBlock) TMC_VERTICES_ATTR k_vertices(VolTable 
 // memory waits (1024^3 Schwarz-P: 20.25 -> 19.85 ms per extraction; one
 // 128^3 volume: 0.401 -> 0.407 ms, hence the two forms).  The same
 // arithmetic in the same order as k_vertices.
-template <class T>
+template <class T, bool MANY>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 3)))
 k_vertices_wide(VolTable vt, const uint4* __restrict__ rec, const uint32_t* __restrict__ grpV, DevN dA,
                 double* __restrict__ vpos, double* __restrict__ vnrm, VertexOut vo, uint32_t* __restrict__ slow,
                 unsigned long long* qhead) {
-    vertices_run<T, 1>(vt, rec, grpV, dA, vpos, vnrm, vo, slow, qhead);
+    vertices_run<T, 1, MANY>(vt, rec, grpV, dA, vpos, vnrm, vo, slow, qhead);
 }
 
 // General path of K3 for the cells k_vertices deferred: every contour is
