@@ -1,0 +1,33 @@
+"""The engine's host rules (tmc_amd/csrc/dmc_plan.h), compiled for the CPU."""
+import itertools
+import os
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+
+@pytest.fixture(scope="module")
+def probe(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("plan") / "plan_probe")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-o", exe,
+                    os.path.join(ROOT, "tests", "cpp", "plan_probe.cpp")], check=True)
+
+    def run(*args):
+        return subprocess.run([exe, *map(str, args)], capture_output=True, text=True, check=True).stdout.strip()
+    return run
+
+
+# axes up to 2^24 points: shapes whose axes ran into each other when they were
+# packed into 21 bits each, and batches that differ in the order of their axes
+SHAPES = [(2, 2, 10485759), (2, 6, 2097151), (6, 2, 2097151), (2, 2097154, 2), (3, 2, 2), (2, 3, 2), (2, 2, 3),
+          (2, 2, 1 << 24), (2, 10, 2), (4, 1 << 21, 2), (5, 2, 2), (2, 2, 2, 3, 3, 3), (3, 3, 3, 2, 2, 2),
+          (2, 2, 2, 3, 3, 3, 2, 2, 2)]
+
+
+def test_shapes_have_keys_of_their_own(probe):
+    keys = {s: probe("key", *s) for s in SHAPES}
+    for a, b in itertools.combinations(SHAPES, 2):
+        assert keys[a] != keys[b], (a, b)
+    assert probe("key", 2, 2, 3) == keys[(2, 2, 3)]

@@ -25,6 +25,7 @@
 #include "../../include/tmc_dmc.h"
 #include "dmc_extract_kernels.h"
 #include "dmc_mesh_kernels.h"
+#include "dmc_plan.h"
 #include "dmc_quad_kernels.h"
 #include "dmc_simplify_kernels.h"
 #include "tmc_kernels.h"
@@ -1617,26 +1618,26 @@ bool finish_pass(dmc_context* ctx, const std::vector<HostVol>& hv, uint32_t flag
 // launches leave (which double buffers hold the mesh) is recorded with the
 // graph and restored after a replay.
 // ---------------------------------------------------------------------------
-std::string pass_key(dmc_context* ctx, const std::vector<HostVol>& hv, const SweepPlan& P, int field_type,
-                     uint32_t flags) {
-    std::string k;
-    auto put = [&](int64_t x) { k.append(reinterpret_cast<const char*>(&x), sizeof(x)); };
-    put(field_type);
-    put(flags & (DMC_SIMPLIFY_ALL | DMC_TRIANGLES));
-    put(P.J);
-    put(P.rows);
-    put(ctx->grid_cap);
-    put(ctx->sweep_waves);
-    put(ctx->acap);
-    put(ctx->vcap);
-    put(ctx->qcap);
-    put(ctx->reccap);
-    put(ctx->force_generic);
-    put(small_colouring(ctx));
-    put((int64_t)ctx->buf_epoch);
-    put((int64_t)hv.size());
-    for (const HostVol& h : hv) put(((int64_t)h.g.nx << 42) | ((int64_t)h.g.ny << 21) | h.g.nz);
-    return k;
+std::string pass_key(dmc_context* ctx, const SweepPlan& P, int field_type, uint32_t flags) {
+    PassShape s{};
+    s.field_type = field_type;
+    s.flags = flags & (DMC_SIMPLIFY_ALL | DMC_TRIANGLES);
+    s.sweep_rows = P.J;
+    s.row_form = P.rows;
+    s.waves = P.W;
+    s.groups = P.groups;
+    s.grid_cap = ctx->grid_cap;
+    s.sweep_waves = ctx->sweep_waves;
+    s.acap = ctx->acap;
+    s.vcap = ctx->vcap;
+    s.qcap = ctx->qcap;
+    s.reccap = ctx->reccap;
+    s.generic = ctx->force_generic;
+    s.small_colouring = small_colouring(ctx);
+    s.buf_epoch = (int64_t)ctx->buf_epoch;
+    const VolDesc* d = reinterpret_cast<const VolDesc*>(ctx->vtab_host.data());
+    for (int v = 0; v < ctx->nvol; v++) s.dims.insert(s.dims.end(), {d[v].d.nx, d[v].d.ny, d[v].d.nz});
+    return tmc::pass_key(s);
 }
 
 void save_post(dmc_context* ctx, dmc_context::PassGraph& g) {
@@ -1666,11 +1667,7 @@ void run_pass(dmc_context* ctx, const SweepPlan& P, int field_type, uint32_t fla
     const bool graphs = ctx->use_graphs && !ctx->timing && !ctx->arena;
     std::string key;
     if (graphs) {
-        // hv is only needed for the key: rebuild it from the volume table
-        std::vector<HostVol> hv(ctx->nvol);
-        const VolDesc* d = reinterpret_cast<const VolDesc*>(ctx->vtab_host.data());
-        for (int v = 0; v < ctx->nvol; v++) hv[v].g = dmc_grid{d[v].d.nx, d[v].d.ny, d[v].d.nz, 0, 0, 0, 0, 0, 0};
-        key = pass_key(ctx, hv, P, field_type, flags);
+        key = pass_key(ctx, P, field_type, flags);
         for (auto& g : ctx->graphs) {
             if (g.key != key) continue;
             upload_vtab(ctx, P);
