@@ -31,3 +31,17 @@ def test_shapes_have_keys_of_their_own(probe):
     for a, b in itertools.combinations(SHAPES, 2):
         assert keys[a] != keys[b], (a, b)
     assert probe("key", 2, 2, 3) == keys[(2, 2, 3)]
+
+
+@pytest.mark.parametrize("volumes,shift", [
+    # one volume: the limits of the group sizes
+    ([(1, 1)], 0), ([(1, 8191)], 0), ([(1, 8192)], 2), ([(1, 65535)], 2), ([(1, 65536)], 4),
+    # many small ones: whole groups of 16, 8, 4, 2 and 1 within an eighth
+    ([(8000, 30)], 4), ([(10000, 8)], 3), ([(10000, 25)], 2), ([(8000, 9)], 1), ([(70000, 1)], 0),
+    # a large one among them carries their padding
+    ([(100, 1), (1, 65536)], 4), ([(1000, 1), (1, 65536)], 3)])
+def test_groups_pad_little(probe, volumes, shift):
+    total = sum(n * rs for n, rs in volumes)
+    got, padded = map(int, probe("groups", *itertools.chain(*volumes)).split())
+    assert got == shift
+    assert total <= padded <= total + total // 8

@@ -25,7 +25,6 @@
 #include "../../include/tmc_dmc.h"
 #include "dmc_extract_kernels.h"
 #include "dmc_mesh_kernels.h"
-#include "dmc_plan.h"
 #include "dmc_quad_kernels.h"
 #include "dmc_simplify_kernels.h"
 #include "tmc_kernels.h"
@@ -598,14 +597,6 @@ struct SweepPlan {
     size_t tab_bytes;
 };
 
-// (row, segment)s per wave of k_cells and k_tmc_cells (2^n), from their total:
-// enough waves to fill the chip come first, cells per wave second.  k_cells
-// with 1 / 2 / 4 / 8 / 16 of them per wave, us: 32^3 (961 in all) 4.6 / 4.6 /
-// 5.2 / 6.4 / 8.0; 201x174x149 (25,752) 17 / 13 / 13 / 18 / 29; 301x257x283
-// (144,384) 107 / 68 / 48 / 39 / 36; 1024^3 (4.2 M) 1606 / 1008 / 799 / 620 /
-// 511.
-int group_shift(int64_t rs) { return rs >= (1 << 16) ? 4 : rs >= (1 << 13) ? 2 : 0; }
-
 template <class T, int J>
 auto sweep_kernel(int rows) {
     return rows == kVectorRows ? k_sweep<T, kVectorRows, J>
@@ -653,9 +644,9 @@ SweepPlan plan_sweep(dmc_context* ctx, const std::vector<HostVol>& hv) {
     int64_t* grpBase = waveBase + (n + 1);
     int64_t W = 0, RS = 0;
     int rows = kVectorRows;
-    int64_t rs_all = 0;
-    for (int v = 0; v < n; v++) rs_all += desc[v].d.R * desc[v].S;
-    const int gsh = group_shift(rs_all);
+    std::vector<int64_t> rs(n);
+    for (int v = 0; v < n; v++) rs[v] = desc[v].d.R * desc[v].S;
+    const int gsh = group_shift(rs);
     for (int v = 0; v < n; v++) {
         VolDesc& D = desc[v];
         D.K = std::min(Kg, D.d.nz - 1);
@@ -665,7 +656,7 @@ SweepPlan plan_sweep(dmc_context* ctx, const std::vector<HostVol>& hv) {
         waveBase[v] = W;
         grpBase[v] = RS >> gsh;
         W += (int64_t)D.S * D.ntj * D.ntk;
-        RS += (D.d.R * D.S + kGroup - 1) / kGroup * kGroup;
+        RS += in_groups(rs[v], gsh);
         const bool whole = D.d.nx % 4 == 0 && (uintptr_t)D.field % (4 * sizeof(T)) == 0;
         rows = std::min<int>(rows, whole ? kVectorRows : D.d.nx >= 4 ? kLongRows : kShortRows);
     }

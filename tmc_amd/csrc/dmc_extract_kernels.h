@@ -20,6 +20,7 @@
 
 #include "dmc_cell.h"
 #include "dmc_kernels.h"
+#include "dmc_plan.h"
 
 namespace tmc {
 
@@ -48,7 +49,7 @@ struct VolDesc {
     double iso_t;          // comparison threshold, exact in the field type
     double rdx2[3];        // 1 / (2 dx), 1 / (2 dy), 1 / (2 dz) correctly rounded, or 0 (divide instead)
     int S, ntj, K, ntk;    // sweep tiling: segments per row, row tiles, planes per wave, plane tiles
-    int64_t rsBase;        // first global (row, segment), a multiple of kGroup
+    int64_t rsBase;        // first global (row, segment), a multiple of 2^gsh
     int gsh;               // (row, segment)s per group (wave of k_cells): 2^gsh, the same for all volumes
 };
 
@@ -90,7 +91,7 @@ struct VolTable {
 constexpr int kSweepRowsFew = 4, kSweepRowsMany = 8;
 constexpr int64_t kSweepManyPoints = (int64_t)1 << 28;   // points of a pass from which a wave takes many
 constexpr int kSeg = 256;           // cells per segment (one wave) and list slots per (row, segment)
-constexpr int kGroup = 16;          // most (row, segment)s per wave of k_cells; a volume is padded to whole ones
+constexpr int kGroup = 1 << kMaxGroupShift;   // most (row, segment)s per wave of k_cells; a volume is padded to whole groups
 #ifndef TMC_VERTICES_ATTR
 #define TMC_VERTICES_ATTR
 #endif
@@ -317,7 +318,7 @@ __global__ void __launch_bounds__(kBlock) k_sweep(VolTable vt, int64_t waves, ui
     // the volume's last wave empties the padding of its last group
     if (wave == vt.waveBase[v + 1] - vt.waveBase[v] - 1) {
         const int64_t rs = d.R * S + lane;
-        if (rs < (d.R * S + kGroup - 1) / kGroup * kGroup) segCount[rs] = 0;
+        if (rs < in_groups(d.R * S, V.gsh)) segCount[rs] = 0;
     }
 }
 
