@@ -745,7 +745,7 @@ void plan_caps(dmc_context* ctx, const std::vector<HostVol>& hv, int64_t cells) 
     ctx->acap = std::min<int64_t>(std::min<int64_t>(ctx->acap, cells), 0xFFFFFFFF);
     ctx->vcap = std::min<int64_t>(ctx->vcap, 0x7FFFFFFF);
     ctx->qcap = std::min<int64_t>(ctx->qcap, 0x1FFFFFFF);
-    ctx->reccap = std::max<int64_t>(ctx->reccap, 1024);
+    ctx->reccap = std::max<int64_t>(ctx->reccap, kFinishRecords);
 }
 
 // live: simplifications follow on the live mesh, whose per-vertex and
@@ -903,10 +903,18 @@ void build_halfedges(dmc_context* ctx, bool final_pass, const StageClears& clear
 // replace the live mesh's.
 void finish_halfedges(dmc_context* ctx, bool compacted) {
     Sizes* S = dsizes(ctx);
-    unsigned long long* ovr = ensure<unsigned long long>(ctx, ctx->ovr, ctx->vcap);
-    launch(ctx, "k_finish", k_finish, dim3(1), dim3(1024), S, static_cast<const BndRec*>(ctx->bndrec.p),
-           (uint32_t)ctx->reccap, static_cast<const int32_t*>(ctx->quads[ctx->cur].p), ovr,
-           static_cast<int32_t*>(ctx->hev.p), compacted ? 1 : 0);
+    const Overrides o{S,
+                      static_cast<const BndRec*>(ctx->bndrec.p),
+                      (uint32_t)ctx->reccap,
+                      static_cast<const int32_t*>(ctx->quads[ctx->cur].p),
+                      ensure<unsigned long long>(ctx, ctx->ovr, ctx->vcap),
+                      static_cast<int32_t*>(ctx->hev.p),
+                      compacted ? 1 : 0};
+    if (ctx->reccap <= kFinishRecords)
+        launch(ctx, "k_finish", k_finish, dim3(1), dim3(1024), o);
+    else
+        for (int which = 0; which < 3; which++)
+            launch(ctx, "k_finish", k_finish_step, dim3(grid_for(ctx, ctx->reccap)), dim3(kBlock), o, which);
     check_launch(ctx, "k_finish");
 }
 

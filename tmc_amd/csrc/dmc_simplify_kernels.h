@@ -732,50 +732,62 @@ __global__ void __launch_bounds__(kBlock) k_final_faces(Live m, const int32_t* _
     }
 }
 
-// Last of the halfedges, one block: the 3-face overrides of he_v
+// Last of the halfedges: the 3-face overrides of he_v
 // (cpp_dmc/DualMarchingCubes.cpp:603-637) -- of the records on a lone vertex
 // the largest key writes -- and, after a simplification, the compacted counts
-// become the mesh's.  Records are few (none on a smooth surface).  Its own
-// stores and atomics meet in this block's L2; the waits order them.
-__global__ void __launch_bounds__(1024) k_finish(Sizes* S, const BndRec* __restrict__ recs, uint32_t reccap,
-                                                  const int32_t* __restrict__ quads,
-                                                  unsigned long long* __restrict__ ovr, int32_t* __restrict__ he_v,
-                                                  int compacted) {
-    const int64_t n = min((int64_t)(compacted ? S->nrec_final : S->nrec), (int64_t)reccap);
-    const int64_t nv = (int64_t)(compacted ? S->nn : S->nv);
-    auto lone = [&](int64_t i, BndRec& r) {
-        r = recs[i];
+// become the mesh's.  Three steps over the records: clear the lone vertices'
+// keys, take the largest, let its record write.
+struct Overrides {
+    Sizes* S;
+    const BndRec* recs;
+    uint32_t reccap;
+    const int32_t* quads;
+    unsigned long long* ovr;
+    int32_t* he_v;
+    int compacted;
+    __device__ __forceinline__ int64_t count() const {
+        return min((int64_t)(compacted ? S->nrec_final : S->nrec), (int64_t)reccap);
+    }
+    __device__ __forceinline__ void step(int which, int64_t i, int64_t nv) const {
+        const BndRec r = recs[i];
         const int32_t v = quads[r.lone];
-        return vid_ok(v, nv) ? v : -1;
-    };
-    auto settle = [] {
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __builtin_amdgcn_s_waitcnt(0);
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __syncthreads();
-    };
-    BndRec r;
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-        const int32_t v = lone(i, r);
-        if (v >= 0) __hip_atomic_store(&ovr[v], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (!vid_ok(v, nv)) return;
+        if (which == 0) __hip_atomic_store(&ovr[v], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else if (which == 1) atomicMax(&ovr[v], r.key + 1ull);
+        else if (__hip_atomic_load(&ovr[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == r.key + 1ull) he_v[v] = r.lone;
     }
-    if (n > 0) settle();
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-        const int32_t v = lone(i, r);
-        if (v >= 0) atomicMax(&ovr[v], r.key + 1ull);
-    }
-    if (n > 0) settle();
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-        const int32_t v = lone(i, r);
-        if (v >= 0 && __hip_atomic_load(&ovr[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == r.key + 1ull)
-            he_v[v] = r.lone;
-    }
-    if (threadIdx.x == 0 && compacted) {
+    // (none of these counts is read by a thread that may still run)
+    __device__ __forceinline__ void commit() const {
+        if (!compacted) return;
         S->nv = S->nn;
         S->nq = S->qn;
         S->recmax = S->nrec > S->recmax ? S->nrec : S->recmax;
         S->nrec = S->nrec_final;
     }
+};
+
+// A pass with room for at most kFinishRecords records, the room that a context
+// starts with (a smooth surface has none): one block does all three steps.  Its
+// own stores and atomics meet in this block's L2; the waits order them.
+constexpr int64_t kFinishRecords = 1024;
+__global__ void __launch_bounds__(1024) k_finish(Overrides o) {
+    const int64_t n = o.count(), nv = (int64_t)(o.compacted ? o.S->nn : o.S->nv);
+    for (int which = 0; which < 3 && n > 0; which++) {
+        for (int64_t i = threadIdx.x; i < n; i += blockDim.x) o.step(which, i, nv);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __builtin_amdgcn_s_waitcnt(0);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) o.commit();
+}
+// More, as noisy fields have: a launch per step.  223 / 1,003 / 1,903 / 7,995 /
+// 23,565 records (noise three points thick) in one block 4.5 / 9.4 / 16.5 / 67
+// / 274 us, in three launches 13.7 to 14.2.
+__global__ void __launch_bounds__(kBlock) k_finish_step(Overrides o, int which) {
+    const int64_t n = o.count(), nv = (int64_t)(o.compacted ? o.S->nn : o.S->nv);
+    TMC_GRID_STRIDE(i, n) o.step(which, i, nv);
+    if (which == 2 && blockIdx.x == 0 && threadIdx.x == 0) o.commit();
 }
 
 }  // namespace tmc
