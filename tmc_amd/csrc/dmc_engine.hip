@@ -1038,7 +1038,6 @@ uint32_t* compact_vertices(dmc_context* ctx, const uint8_t* removed, int32_t* vs
     check_launch(ctx, "k_compact_slots");
     ctx->scur = 1 - ctx->scur;
     ctx->slots = true;
-    remap_bounds(ctx, ctx->vbound, newidx, &S->nv, &S->nn);
     return newidx;
 }
 
@@ -1116,10 +1115,11 @@ void simplify3x3y(dmc_context* ctx, bool colored) {
            static_cast<double*>(ctx->pos[ctx->pcur].p), static_cast<double*>(ctx->nrm[ctx->pcur].p),
            ctx->slots ? static_cast<const uint32_t*>(ctx->vslot[ctx->scur].p) : nullptr, vsecond);
     check_launch(ctx, "k_merge_apply");
-    compact_vertices(ctx, vfirst, vsecond);
+    const uint32_t* newv = compact_vertices(ctx, vfirst, vsecond);
     int32_t* vmap = ensure<int32_t>(ctx, ctx->vmap, vcap);
     launch(ctx, "k_vmap3x3y", k_vmap3x3y, dim3(grid_for(ctx, vcap)), dim3(kBlock), (const uint8_t*)vfirst,
-           (const int32_t*)vsecond, (const Sizes*)S, vmap);
+           (const int32_t*)vsecond, (const Sizes*)S, static_cast<const int64_t*>(ctx->vbound.p), ctx->nvol, newv, vmap);
+    remap_bounds(ctx, ctx->vbound, newv, &S->nv, &S->nn);
     compact_quads(ctx, newQ, vmap, nullptr, nullptr);
 }
 
@@ -1158,6 +1158,7 @@ void simplify3333(dmc_context* ctx) {
     int32_t* vmap = ensure<int32_t>(ctx, ctx->vmap, vcap);
     launch(ctx, "k_vmap3333", k_vmap3333, dim3(grid_for(ctx, vcap)), dim3(kBlock), (const uint8_t*)vflag,
            (const uint32_t*)newv, (const Sizes*)S, vmap);
+    remap_bounds(ctx, ctx->vbound, newv, &S->nv, &S->nn);
     compact_quads(ctx, newQ, vmap, p3333, vtwin);
 }
 

@@ -984,6 +984,10 @@ __device__ __forceinline__ int vol_from(const int64_t* __restrict__ base, int n,
     return v;
 }
 
+// A vertex id of a batch as the volume's own; -2 - id is an id that the volume
+// does not have (k_vmap3x3y), -1 stays.
+__device__ __forceinline__ int32_t own_id(int32_t x, int32_t v0) { return x >= 0 ? x - v0 : x < -1 ? -2 - x : x; }
+
 __global__ void __launch_bounds__(kBlock) k_rebase(const int64_t* __restrict__ vb, const int64_t* __restrict__ qb,
                                                     int n, int32_t* __restrict__ quads, int32_t* __restrict__ twin,
                                                     int32_t* __restrict__ tris, const Sizes* S,
@@ -999,7 +1003,7 @@ __global__ void __launch_bounds__(kBlock) k_rebase(const int64_t* __restrict__ v
             const int vol = vol_from(qb, n, first, x);
             const int32_t v0 = (int32_t)vb[vol], h0 = (int32_t)(4 * qb[vol]);
             int4 q = reinterpret_cast<const int4*>(quads)[x], t = reinterpret_cast<const int4*>(twin)[x];
-            q = make_int4(q.x - v0, q.y - v0, q.z - v0, q.w - v0);
+            q = make_int4(own_id(q.x, v0), own_id(q.y, v0), own_id(q.z, v0), own_id(q.w, v0));
             t = make_int4(t.x >= 0 ? t.x - h0 : t.x, t.y >= 0 ? t.y - h0 : t.y, t.z >= 0 ? t.z - h0 : t.z,
                           t.w >= 0 ? t.w - h0 : t.w);
             reinterpret_cast<int4*>(quads)[x] = q;
@@ -1009,7 +1013,7 @@ __global__ void __launch_bounds__(kBlock) k_rebase(const int64_t* __restrict__ v
 #pragma unroll
                 for (int k = 0; k < 3; k++) {
                     const int2 e = tr[k];
-                    tr[k] = make_int2(e.x - v0, e.y - v0);
+                    tr[k] = make_int2(own_id(e.x, v0), own_id(e.y, v0));
                 }
             }
         }

@@ -836,14 +836,29 @@ __global__ void __launch_bounds__(kBlock) k_twin3333(const int32_t* __restrict__
 
 // The compactions of a pass run stage by stage (generic rows).
 // 3X3Y: vmap[x] = vsecond[x] for a kept x (its new id after the vertex
-// compaction), vsecond[vsecond[x]] for a removed one (its target's).
+// compaction), vsecond[vsecond[x]] for a removed one: its target's new id or,
+// where the target is removed too, the old id of the target's target, which the
+// reference takes for a new one.  In a batch that id is the volume's own: vb
+// holds each volume's first old vertex, newidx the scan of the kept ones, and an
+// id that the volume no longer has becomes -2 - id, which no vertex has.
 __global__ void __launch_bounds__(kBlock) k_vmap3x3y(const uint8_t* __restrict__ vfirst,
                                                       const int32_t* __restrict__ vsecond, const Sizes* S,
+                                                      const int64_t* __restrict__ vb, int nvol,
+                                                      const uint32_t* __restrict__ newidx,
                                                       int32_t* __restrict__ vmap) {
-    const int64_t nv = (int64_t)S->nv;
+    const int64_t nv = (int64_t)S->nv, nn = (int64_t)S->nn;
     TMC_GRID_STRIDE(x, nv) {
         int32_t y = vsecond[x];
-        if (vfirst[x] != 0) y = vid_ok(y, nv) ? vsecond[y] : -1;
+        if (vfirst[x] != 0) {
+            const bool ok = vid_ok(y, nv), chain = ok && vfirst[y] != 0;
+            y = ok ? vsecond[y] : -1;
+            if (chain && nvol > 1) {
+                const int v = vol_of(vb, nvol, y);
+                auto first = [&](int64_t b) { return b < nv ? (int64_t)newidx[b] : nn; };
+                const int64_t id = y - vb[v], n0 = first(vb[v]);
+                y = id < first(vb[v + 1]) - n0 ? (int32_t)(n0 + id) : (int32_t)(-2 - id);
+            }
+        }
         vmap[x] = y;
     }
 }
