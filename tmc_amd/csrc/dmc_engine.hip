@@ -19,6 +19,7 @@
 #include <stdexcept>
 #include <string>
 #include <unordered_map>
+#include <unordered_set>
 #include <utility>
 #include <vector>
 
@@ -147,6 +148,7 @@ struct dmc_context {
     // overflowed, raised to its exact sizes (the *_min, one extraction long)
     int64_t acap = 0, vcap = 0, qcap = 0, reccap = 0;
     int64_t acap_min = 0, vcap_min = 0, qcap_min = 0;
+    std::string shape;         // shape_key of the running extraction
     int64_t qexpect = 0;       // quadrilaterals the densities seen so far give (0: none seen)
     double rcell[3] = {0, 0, 0}, rarea[3] = {0, 0, 0};
     Sizes hsz{};               // the last pass's sizes block
@@ -161,6 +163,7 @@ struct dmc_context {
     };
     std::vector<PassGraph> graphs;
     std::unordered_map<std::string, int> seen;   // passes run per shape (bounded)
+    std::unordered_set<std::string> staged;      // shapes whose last pass needed to be run stage by stage (bounded)
     uint64_t buf_epoch = 0;    // bumped by every buffer (re)allocation
     uint64_t graph_clock = 0;
     bool use_graphs = true;
@@ -1066,7 +1069,7 @@ void compact_quads(dmc_context* ctx, const uint32_t* newQ, const int32_t* vmap, 
     int32_t* q2 = ensure<int32_t>(ctx, ctx->quads[1 - ctx->cur], 4 * qcap);
     remap_bounds(ctx, ctx->qbound, newQ, &S->nq, &S->qn);
     launch(ctx, "k_compact_quads", k_compact_quads, dim3(grid_for(ctx, qcap)), dim3(kBlock),
-           static_cast<const int32_t*>(ctx->quads[ctx->cur].p), (const Sizes*)S, p3333, vtwin, vmap,
+           static_cast<const int32_t*>(ctx->quads[ctx->cur].p), S, p3333, vtwin, vmap,
            reinterpret_cast<const int32_t*>(newQ), q2);
     check_launch(ctx, "k_compact_quads");
     ctx->commit_pending = true;
@@ -1118,7 +1121,7 @@ void simplify3x3y(dmc_context* ctx, bool colored) {
     const uint32_t* newv = compact_vertices(ctx, vfirst, vsecond);
     int32_t* vmap = ensure<int32_t>(ctx, ctx->vmap, vcap);
     launch(ctx, "k_vmap3x3y", k_vmap3x3y, dim3(grid_for(ctx, vcap)), dim3(kBlock), (const uint8_t*)vfirst,
-           (const int32_t*)vsecond, (const Sizes*)S, static_cast<const int64_t*>(ctx->vbound.p), ctx->nvol, newv, vmap);
+           (const int32_t*)vsecond, S, static_cast<const int64_t*>(ctx->vbound.p), ctx->nvol, newv, vmap);
     remap_bounds(ctx, ctx->vbound, newv, &S->nv, &S->nn);
     compact_quads(ctx, newQ, vmap, nullptr, nullptr);
 }
@@ -1500,8 +1503,14 @@ bool finish_pass(dmc_context* ctx, const std::vector<HostVol>& hv, uint32_t flag
     }
     if (!ctx->force_generic && (hs.need_generic || hs.unresolved)) {
         // the live mesh could not express the pass: the same stage by stage
+        if (hs.need_generic) {
+            if (ctx->staged.size() >= kMaxSeen) ctx->staged.clear();
+            ctx->staged.insert(ctx->shape);
+        }
         ctx->force_generic = true;
         if (!hs.ovf) return false;
+    } else if (!hs.ovf && !hs.need_generic && !ctx->staged.empty()) {
+        ctx->staged.erase(ctx->shape);
     }
     if (hs.ovf) {
         // exceeded a capacity: the same pass again with room for the exact
@@ -1606,6 +1615,15 @@ bool finish_pass(dmc_context* ctx, const std::vector<HostVol>& hv, uint32_t flag
     }
     ctx->have_mesh = true;
     return true;
+}
+
+// What a caller sees of a pass: element type, stages and volumes.
+std::string shape_key(int field_type, uint32_t flags, const std::vector<HostVol>& hv) {
+    PassShape s{};
+    s.field_type = field_type;
+    s.flags = flags & DMC_SIMPLIFY_ALL;
+    for (const HostVol& h : hv) s.dims.insert(s.dims.end(), {h.g.nx, h.g.ny, h.g.nz});
+    return tmc::pass_key(s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1788,7 +1806,12 @@ void do_extract(dmc_context* ctx, void* a_) {
     }
     // a pass that outgrew a capacity learned the exact sizes, and one that
     // needed generic halfedge rows asks for them: once more
-    ctx->force_generic = ctx->always_generic;
+    // (a shape that needed them last time starts with them: a slab of noise one
+    // cell thick, 4000x600x2 points, 2.3 ms a pass instead of 1.7 + 2.3; the
+    // pass says when it did not)
+    ctx->shape.clear();
+    if (a.flags & DMC_SIMPLIFY_ALL) ctx->shape = shape_key(a.field_type, a.flags, hv);
+    ctx->force_generic = ctx->always_generic || ctx->staged.count(ctx->shape) != 0;
     // exact sizes learned from an overflow hold for that extraction's rerun
     // only: later passes plan from the densities, which the overflow raised
     ctx->acap_min = ctx->vcap_min = ctx->qcap_min = 0;

@@ -842,7 +842,7 @@ __global__ void __launch_bounds__(kBlock) k_twin3333(const int32_t* __restrict__
 // holds each volume's first old vertex, newidx the scan of the kept ones, and an
 // id that the volume no longer has becomes -2 - id, which no vertex has.
 __global__ void __launch_bounds__(kBlock) k_vmap3x3y(const uint8_t* __restrict__ vfirst,
-                                                      const int32_t* __restrict__ vsecond, const Sizes* S,
+                                                      const int32_t* __restrict__ vsecond, Sizes* S,
                                                       const int64_t* __restrict__ vb, int nvol,
                                                       const uint32_t* __restrict__ newidx,
                                                       int32_t* __restrict__ vmap) {
@@ -852,6 +852,7 @@ __global__ void __launch_bounds__(kBlock) k_vmap3x3y(const uint8_t* __restrict__
         if (vfirst[x] != 0) {
             const bool ok = vid_ok(y, nv), chain = ok && vfirst[y] != 0;
             y = ok ? vsecond[y] : -1;
+            if (chain) S->need_generic = 1u;   // the live mesh does not express it
             if (chain && nvol > 1) {
                 const int v = vol_of(vb, nvol, y);
                 auto first = [&](int64_t b) { return b < nv ? (int64_t)newidx[b] : nn; };
@@ -876,7 +877,7 @@ __global__ void __launch_bounds__(kBlock) k_vmap3333(const uint8_t* __restrict__
 // qmap[f] (negative: dropped).  The vertex ids come from vmap, for 3X3Y
 // vm[vm[x]]-style lookups of a removed vertex x, exactly as the reference
 // composes them; a pattern face's corners go through vtwin first.
-__global__ void __launch_bounds__(kBlock) k_compact_quads(const int32_t* __restrict__ quads, const Sizes* S,
+__global__ void __launch_bounds__(kBlock) k_compact_quads(const int32_t* __restrict__ quads, Sizes* S,
                                                            const uint8_t* __restrict__ p3333,
                                                            const int32_t* __restrict__ vtwin,
                                                            const int32_t* __restrict__ vmap,
@@ -892,6 +893,7 @@ __global__ void __launch_bounds__(kBlock) k_compact_quads(const int32_t* __restr
         for (int k = 0; k < 4; k++) {
             if (p3333 && p3333[f] && vid_ok(x[k], nv)) x[k] = vtwin[x[k]];
             x[k] = vid_ok(x[k], nv) ? vmap[x[k]] : -1;
+            if (x[k] < 0) S->need_generic = 1u;   // nor this
         }
         reinterpret_cast<int4*>(quads2)[m] = make_int4(x[0], x[1], x[2], x[3]);
     }
