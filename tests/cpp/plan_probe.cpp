@@ -1,6 +1,7 @@
 // Prints what the engine's host rules (tmc_amd/csrc/dmc_plan.h) answer.
 //   plan_probe key nx ny nz [nx ny nz ...]   the pass key of volumes, everything else equal (hex)
 //   plan_probe groups n rs [n rs ...]        group shift of n volumes of rs (row, segment)s each, and these padded
+//   plan_probe blocks n per_block limit grid_cap
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -13,6 +14,10 @@ int main(int argc, char** argv) {
         for (int i = 2; i < argc; i++) s.dims.push_back(atoi(argv[i]));
         for (unsigned char c : tmc::pass_key(s)) printf("%02x", c);
         printf("\n");
+        return 0;
+    }
+    if (argc == 6 && !strcmp(argv[1], "blocks")) {
+        printf("%lld\n", (long long)tmc::blocks_for(atoll(argv[2]), atoll(argv[3]), atoll(argv[4]), atoll(argv[5])));
         return 0;
     }
     if (argc > 3 && !strcmp(argv[1], "groups")) {

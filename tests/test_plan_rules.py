@@ -45,3 +45,11 @@ def test_groups_pad_little(probe, volumes, shift):
     got, padded = map(int, probe("groups", *itertools.chain(*volumes)).split())
     assert got == shift
     assert total <= padded <= total + total // 8
+
+
+@pytest.mark.parametrize("args,blocks", [
+    ((0, 256, 0, 32768), 1), ((256, 256, 0, 32768), 1), ((257, 256, 0, 32768), 2), ((1 << 30, 256, 0, 32768), 32768),
+    # a kernel's own limit never lifts the caller's cap
+    ((1 << 30, 256, 4096, 32768), 4096), ((1 << 30, 256, 4096, 64), 64), ((1000, 256, 4096, 64), 4)])
+def test_blocks_of_a_launch(probe, args, blocks):
+    assert int(probe("blocks", *args)) == blocks

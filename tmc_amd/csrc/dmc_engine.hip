@@ -266,10 +266,8 @@ T* ensure(dmc_context* ctx, Buf& b, size_t n) {
     return static_cast<T*>(b.p);
 }
 
-int grid_for(const dmc_context* ctx, int64_t n, int per_block = kBlock, int64_t cap = 0) {
-    if (cap <= 0) cap = ctx->grid_cap;
-    int64_t g = (n + per_block - 1) / per_block;
-    return (int)std::max<int64_t>(1, std::min<int64_t>(g, cap));
+int grid_for(const dmc_context* ctx, int64_t n, int per_block = kBlock, int64_t limit = 0) {
+    return (int)blocks_for(n, per_block, limit, ctx->grid_cap);
 }
 
 hipEvent_t take_event(dmc_context* ctx) {
@@ -1199,7 +1197,8 @@ Live live_mesh(dmc_context* ctx) {
 }
 
 // Blocks of the kernels that gather a stage's list (a contiguous share of the
-// faces each): one add on the list's counter per block and 768 entries.
+// faces each): an add on the list's counter per block, and another one each time
+// a block holds more than kListBuf - kListTurn entries.
 constexpr int kListBlocks = 4096;
 
 void stage_rest(dmc_context* ctx, const Live& m, bool is3333) {

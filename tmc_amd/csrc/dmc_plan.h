@@ -1,6 +1,8 @@
 // dmc_plan.h -- host rules of the engine that need no device: what makes two
-// passes the same pass, and how the cells' rows are grouped.
+// passes the same pass, how the cells' rows are grouped, and how many blocks a
+// launch takes.
 #pragma once
+#include <algorithm>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -53,6 +55,14 @@ inline int group_shift(const std::vector<int64_t>& rs) {
         if (padded - total <= total / 8) break;
     }
     return shift;
+}
+
+// Blocks of a launch over n items, per_block of them a block and turn: at most
+// grid_cap (the caller's, dmc_launch) and, where a kernel has a limit of its own,
+// at most that (0: none).
+inline int64_t blocks_for(int64_t n, int64_t per_block, int64_t limit, int64_t grid_cap) {
+    const int64_t cap = limit > 0 ? std::min(limit, grid_cap) : grid_cap;
+    return std::max<int64_t>(1, std::min((n + per_block - 1) / per_block, cap));
 }
 
 }  // namespace tmc
