@@ -54,11 +54,6 @@ __device__ __forceinline__ int edge_axis(int e) { return (int)((kEdgeAxisPacked 
 __device__ __forceinline__ int edge_slot(int e, int bit) {
     return (int)((kEdgeSlotPacked >> (4 * e + 2 * bit)) & 3);
 }
-// Does the iso-surface cross edge e of a cell with case `icase`?
-__device__ __forceinline__ bool edge_cut(unsigned icase, int e) {
-    return ((icase >> edge_v0(e)) ^ (icase >> edge_v1(e))) & 1u;
-}
-
 // Is the grid edge e of cell (i,j,k) shared by four existing cells?  Only
 // such edges yield complete quadrilaterals (DualMarchingCubes.h:663-676).
 __device__ __forceinline__ bool edge_interior(int e, int i, int j, int k, int nx, int ny, int nz) {
@@ -222,18 +217,6 @@ __device__ __forceinline__ unsigned case_decisions(unsigned icase, double iso, c
 __device__ __forceinline__ bool undecided(unsigned dec) { return dec >= 1u << kMaxDecisions; }
 __device__ inline uint64_t chained_contours(unsigned icase, unsigned dec) {
     return ContourTable::chain(icase, dec & ((1u << kMaxDecisions) - 1u), dec >> kMaxDecisions);
-}
-
-// Pick element t of a 4-array without dynamic register indexing.
-template <class T>
-__device__ __forceinline__ T pick4(const T (&a)[4], int t) {
-    return t == 0 ? a[0] : t == 1 ? a[1] : t == 2 ? a[2] : a[3];
-}
-template <class T>
-__device__ __forceinline__ T pick8(const T* a, int t) {
-    const T lo = (t & 2) ? ((t & 1) ? a[3] : a[2]) : ((t & 1) ? a[1] : a[0]);
-    const T hi = (t & 2) ? ((t & 1) ? a[7] : a[6]) : ((t & 1) ? a[5] : a[4]);
-    return (t & 4) ? hi : lo;
 }
 
 // Corner values of one cell kept in LDS (one column per thread) for reads

@@ -417,15 +417,10 @@ void swap_pairs(dmc_context* ctx) {
 DevN dn(const uint64_t* p, int64_t cap) { return DevN{p, cap}; }
 DevN hn(int64_t n) { return DevN{nullptr, n}; }
 
-// Fill n (device count, capped) 32-bit words or bytes with a value.
-void fill_u32(dmc_context* ctx, void* p, DevN n, uint32_t value, const uint32_t* gate = nullptr) {
+// Fill n (device count, capped) 32-bit words with a value.
+void fill_u32(dmc_context* ctx, void* p, DevN n, uint32_t value) {
     if (n.cap <= 0) return;
-    launch(ctx, "k_fill", k_fill_u32, dim3(grid_for(ctx, n.cap)), dim3(kBlock), static_cast<uint32_t*>(p), n, value,
-           gate);
-}
-void fill_u8(dmc_context* ctx, void* p, DevN n, uint8_t value) {
-    if (n.cap <= 0) return;
-    launch(ctx, "k_fill", k_fill_u8, dim3(grid_for(ctx, n.cap)), dim3(kBlock), static_cast<uint8_t*>(p), n, value);
+    launch(ctx, "k_fill", k_fill_u32, dim3(grid_for(ctx, n.cap)), dim3(kBlock), static_cast<uint32_t*>(p), n, value);
 }
 
 // Fills gathered into one launch (k_fill_many).
@@ -435,12 +430,10 @@ struct Fills {
     int n = 0;
     int64_t cap = 0;
     explicit Fills(dmc_context* c) : ctx(c) {}
-    Fills& u32(void* p, DevN d, uint32_t value, const uint32_t* gate = nullptr) { return add(p, d, value, gate, 4); }
-    Fills& u8(void* p, DevN d, uint8_t value, const uint32_t* gate = nullptr) { return add(p, d, value, gate, 1); }
-    Fills& add(void* p, DevN d, uint32_t value, const uint32_t* gate, int bytes) {
+    Fills& u32(void* p, DevN d, uint32_t value) {
         if (d.cap <= 0) return *this;
         if (n == kMaxFillJobs) run();
-        s.j[n++] = FillJob{p, d, value, gate, bytes};
+        s.j[n++] = FillJob{static_cast<uint32_t*>(p), d, value};
         cap = std::max(cap, d.cap);
         return *this;
     }
@@ -469,14 +462,14 @@ unsigned long long* scan_state(dmc_context* ctx, int64_t tiles) {
 
 // Exclusive scan of n.get() uint32 items into out (launched for n.cap); the
 // 64-bit total goes to *dtotal (device memory); row_end: also the total's low
-// 32 bits to row_end[n] (the end of a CSR's last row).  Nothing runs when
-// *gate is 0.  One block for a few tiles, one launch of look-back tiles for
-// up to kScanOnePassTiles, three launches beyond.
+// 32 bits to row_end[n] (the end of a CSR's last row).  One block for a few
+// tiles, one launch of look-back tiles for up to kScanOnePassTiles, three
+// launches beyond.
 template <class In>
 void scan_to(dmc_context* ctx, In in, uint32_t* out, DevN n, uint64_t* dtotal, const char* name = "k_scan",
-             const uint32_t* gate = nullptr, uint32_t* row_end = nullptr) {
+             uint32_t* row_end = nullptr) {
     if (n.cap <= kScanSmallItems) {
-        launch(ctx, name, k_scan_small<In>, dim3(1), dim3(1024), in, out, n, gate, dtotal, row_end);
+        launch(ctx, name, k_scan_small<In>, dim3(1), dim3(1024), in, out, n, dtotal, row_end);
         check_launch(ctx, "scan");
         return;
     }
@@ -485,27 +478,24 @@ void scan_to(dmc_context* ctx, In in, uint32_t* out, DevN n, uint64_t* dtotal, c
         // a stalled look-back re-reads the input
         if (static_cast<const void*>(in.p) == static_cast<const void*>(out))
             fail(ctx, DMC_ERR_STATE, "%s: a scan in place", name);
-        launch(ctx, name, k_scan<In>, dim3((unsigned)tiles), dim3(kBlock), in, out, n, gate, dtotal, row_end,
+        launch(ctx, name, k_scan<In>, dim3((unsigned)tiles), dim3(kBlock), in, out, n, dtotal, row_end,
                scan_state(ctx, tiles), tiles, ctx->scan_spin);
     } else {
         uint64_t* part = ensure<uint64_t>(ctx, ctx->scanPartial, tiles);
-        launch(ctx, name, k_scan_reduce<In>, dim3((unsigned)tiles), dim3(kBlock), in, n, gate, part);
-        launch(ctx, name, k_scan_partials, dim3(1), dim3(1024), part, tiles, gate, dtotal, row_end, n);
-        launch(ctx, name, k_scan_down<In>, dim3((unsigned)tiles), dim3(kBlock), in, out, n, gate, part);
+        launch(ctx, name, k_scan_reduce<In>, dim3((unsigned)tiles), dim3(kBlock), in, n, part);
+        launch(ctx, name, k_scan_partials, dim3(1), dim3(1024), part, tiles, dtotal, row_end, n);
+        launch(ctx, name, k_scan_down<In>, dim3((unsigned)tiles), dim3(kBlock), in, out, n, part);
     }
     check_launch(ctx, "scan");
 }
 
 template <class In>
-ScanJob<In> scan_job(In in, uint32_t* out, DevN n, uint64_t* dtotal, const uint32_t* gate = nullptr,
-                     uint32_t* row_end = nullptr) {
+ScanJob<In> scan_job(In in, uint32_t* out, DevN n, uint64_t* dtotal) {
     ScanJob<In> j{};
     j.in = in;
     j.out = out;
     j.dn = n;
-    j.gate = gate;
     j.total = dtotal;
-    j.row_end = row_end;
     j.ntiles = (n.cap + kScanTile - 1) / kScanTile;
     return j;
 }
@@ -821,12 +811,10 @@ void run_cells(dmc_context* ctx, const SweepPlan& P, bool live) {
     // 3-wave form once there are more cells than one round of the grid's
     // threads (F32 fields: the F64 form would spill at 3 waves)
     const dim3 gv(grid_for(ctx, acap, kBlock, kVerticesBlocks));
-    if (std::is_same<T, float>::value && acap > kVerticesBlocks * kBlock)
-        launch(ctx, "k_vertices", n > 1 ? k_vertices_wide<T, true> : k_vertices_wide<T, false>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, vo, slow,
-               &S->qhead);
-    else
-        launch(ctx, "k_vertices", n > 1 ? k_vertices<T, true> : k_vertices<T, false>, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, vo, slow,
-               &S->qhead);
+    auto vertices = n > 1 ? k_vertices<T, true> : k_vertices<T, false>;
+    if constexpr (std::is_same<T, float>::value)
+        if (acap > kVerticesBlocks * kBlock) vertices = n > 1 ? k_vertices_wide<T, true> : k_vertices_wide<T, false>;
+    launch(ctx, "k_vertices", vertices, gv, dim3(kBlock), vt, rec, grpV, A, pos, nrm, vo, slow, &S->qhead);
     check_launch(ctx, "k_vertices");
     launch(ctx, "k_vertices_slow", k_vertices_slow<T>, dim3(grid_for(ctx, acap, kBlock, 1024)), dim3(kBlock), vt,
            rec, grpV, slow, pos, nrm, vo, sw.vstat);
@@ -875,7 +863,7 @@ void pair_rows(dmc_context* ctx, bool final_pass) {
     fl.run();
     launch(ctx, "k_he_degree", k_he_degree, dim3(grid_for(ctx, hcap)), dim3(kBlock), quads, (const Sizes*)S, deg,
            &S->he.bad);
-    scan_to(ctx, ScanCounts{deg}, off, nv, &S->tot, "k_scan", nullptr, off);
+    scan_to(ctx, ScanCounts{deg}, off, nv, &S->tot, "k_scan", off);
     launch(ctx, "k_he_scatter", k_he_scatter, dim3(grid_for(ctx, qcap)), dim3(kBlock), quads, (const Sizes*)S, off,
            cursor, adj);
     launch(ctx, "k_he_twins", k_he_twins, dim3(grid_for(ctx, hcap)), dim3(kBlock), quads, (const Sizes*)S, off, adj,
@@ -2171,7 +2159,7 @@ static void ensure_rows(dmc_context* ctx) {
     fill_u32(ctx, cursor, nv, 0u);
     launch(ctx, "k_he_degree", k_he_degree, dim3(grid_for(ctx, hcap)), dim3(kBlock), quads, (const Sizes*)S, deg,
            &S->he.pad);
-    scan_to(ctx, ScanCounts{deg}, off, nv, &S->tot, "k_scan", nullptr, off);
+    scan_to(ctx, ScanCounts{deg}, off, nv, &S->tot, "k_scan", off);
     launch(ctx, "k_he_scatter", k_he_scatter, dim3(grid_for(ctx, qcap)), dim3(kBlock), quads, (const Sizes*)S, off,
            cursor, adj);
     check_launch(ctx, "rows");

@@ -46,11 +46,9 @@ struct DevN {
     }
 };
 
-// Statistics of one halfedge build, counted per halfedge so that a build
-// that carries most groups over from the last one can count them too:
-// non-manifold edges = nm4 / 4 + nm3 / 3, 3-face edges = nm3 / 3.
-// Halfedge statistics of a build.  On the device only bad and pad are kept
-// here; the counts of flagged halfedges live in Sizes::hep (spread over
+// Halfedge statistics of a build, counted per halfedge: non-manifold edges =
+// nm4 / 4 + nm3 / 3, 3-face edges = nm3 / 3.  On the device only bad and pad are
+// kept here; the counts of flagged halfedges live in Sizes::hep (spread over
 // kHeParts slots) and the host writes their sums into nm4, errors, nm3.
 struct HeStats {
     unsigned long long nm4;      // halfedges flagged non-manifold (groups of 4)
@@ -98,23 +96,12 @@ struct Sizes {
     unsigned long long hep[kHeParts][3];      // the build's flagged halfedges per slot: groups of 4, of 3, error groups
 };
 
-// The build's count of error groups (groups of more than 4 halfedges).
-__device__ __forceinline__ unsigned long long he_errors(const Sizes* S) {
-    unsigned long long e = 0;
-    for (int p = 0; p < kHeParts; p++) e += S->hep[p][2];
-    return e;
-}
-
 // Fresh counts for a new build (one thread).
 __device__ __forceinline__ void he_clear(Sizes* S) {
     for (int p = 0; p < kHeParts; p++) S->hep[p][0] = S->hep[p][1] = S->hep[p][2] = 0;
     S->he.bad = 0;
     S->he.pad = 0;
 }
-
-// A launch whose work is conditional on device data: it runs only when
-// *gate != 0 (gate == nullptr: always).
-__device__ __forceinline__ bool gated_off(const uint32_t* gate) { return gate && *gate == 0u; }
 
 template <class T>
 __device__ __forceinline__ T wave_inclusive_scan(T x) {
@@ -181,17 +168,6 @@ struct ScanCounts {
         }
     }
 };
-struct ScanSet {
-    static constexpr bool kMap = false;
-    const uint8_t* p;   // set flags
-    __device__ __forceinline__ uint32_t at(int64_t i) const { return p[i] ? 1u : 0u; }
-    __device__ __forceinline__ void vec16(int64_t base, uint32_t v[kScanIPT]) const {
-        const uint4 t = *reinterpret_cast<const uint4*>(p + base);
-        const uint32_t w[4] = {t.x, t.y, t.z, t.w};
-#pragma unroll
-        for (int q = 0; q < kScanIPT; q++) v[q] = ((w[q >> 2] >> (8 * (q & 3))) & 0xFFu) ? 1u : 0u;
-    }
-};
 struct ScanKeep {
     static constexpr bool kMap = false;
     const uint8_t* p;   // removed flags
@@ -241,13 +217,12 @@ __device__ __forceinline__ void scan_items(const In& in, int64_t n, int64_t base
 }
 
 // Device-wide exclusive scan over n = dn.get() items in three launches over
-// ceil(dn.cap / kScanTile) tiles (tile sums, their scan, the tiles again);
-// skipped entirely when gated off.  For inputs of many tiles.
+// ceil(dn.cap / kScanTile) tiles (tile sums, their scan, the tiles again).  For
+// inputs of many tiles.
 template <class In>
-__device__ __forceinline__ void scan_reduce_tile(const In& in, DevN dn, const uint32_t* __restrict__ gate,
-                                                 uint64_t* __restrict__ partial, int64_t tile) {
+__device__ __forceinline__ void scan_reduce_tile(const In& in, DevN dn, uint64_t* __restrict__ partial,
+                                                 int64_t tile) {
     __shared__ uint64_t sm[kBlock / kWave + 1];
-    if (gated_off(gate)) return;
     const int64_t n = dn.get();
     uint32_t v[kScanIPT];
     scan_items(in, n, tile * kScanTile + (int64_t)threadIdx.x * kScanIPT, v);
@@ -266,18 +241,15 @@ __device__ __forceinline__ void scan_reduce_tile(const In& in, DevN dn, const ui
 }
 
 template <class In>
-__global__ void __launch_bounds__(kBlock) k_scan_reduce(In in, DevN dn, const uint32_t* __restrict__ gate,
-                                                       uint64_t* __restrict__ partial) {
-    scan_reduce_tile(in, dn, gate, partial, (int64_t)blockIdx.x);
+__global__ void __launch_bounds__(kBlock) k_scan_reduce(In in, DevN dn, uint64_t* __restrict__ partial) {
+    scan_reduce_tile(in, dn, partial, (int64_t)blockIdx.x);
 }
 
 // Single block: exclusive scan of the tile sums in place, total to *total
 // (and, for a CSR, its low 32 bits to row_end[n], the end of the last row).
 __device__ __forceinline__ void scan_partials_run(uint64_t* __restrict__ partial, int64_t ntiles,
-                                                  const uint32_t* __restrict__ gate, uint64_t* __restrict__ total,
-                                                  uint32_t* __restrict__ row_end, DevN dn) {
+                                                  uint64_t* __restrict__ total, uint32_t* __restrict__ row_end, DevN dn) {
     __shared__ uint64_t sm[1024 / kWave + 1];
-    if (gated_off(gate)) return;
     uint64_t carry = 0;
     for (int64_t b = 0; b < ntiles; b += 1024) {
         const int64_t idx = b + threadIdx.x;
@@ -294,17 +266,15 @@ __device__ __forceinline__ void scan_partials_run(uint64_t* __restrict__ partial
 }
 
 __global__ void __launch_bounds__(1024) k_scan_partials(uint64_t* __restrict__ partial, int64_t ntiles,
-                                                         const uint32_t* __restrict__ gate, uint64_t* __restrict__ total,
+                                                         uint64_t* __restrict__ total,
                                                          uint32_t* __restrict__ row_end, DevN dn) {
-    scan_partials_run(partial, ntiles, gate, total, row_end, dn);
+    scan_partials_run(partial, ntiles, total, row_end, dn);
 }
 
 template <class In>
 __device__ __forceinline__ void scan_down_tile(const In& in, uint32_t* __restrict__ out, DevN dn,
-                                               const uint32_t* __restrict__ gate,
                                                const uint64_t* __restrict__ partial, int64_t tile) {
     __shared__ uint32_t sm[kBlock / kWave + 1];
-    if (gated_off(gate)) return;
     const int64_t n = dn.get();
     const int64_t base = tile * kScanTile + (int64_t)threadIdx.x * kScanIPT;
     const bool full = base + kScanIPT <= n;
@@ -334,16 +304,15 @@ __device__ __forceinline__ void scan_down_tile(const In& in, uint32_t* __restric
 
 template <class In>
 __global__ void __launch_bounds__(kBlock) k_scan_down(In in, uint32_t* __restrict__ out, DevN dn,
-                                                       const uint32_t* __restrict__ gate,
                                                        const uint64_t* __restrict__ partial) {
-    scan_down_tile(in, out, dn, gate, partial, (int64_t)blockIdx.x);
+    scan_down_tile(in, out, dn, partial, (int64_t)blockIdx.x);
 }
 
 // The same in one launch of ceil(dn.cap / kScanTile) blocks (decoupled
 // look-back), for inputs of up to kScanOnePassTiles tiles, so that a
-// look-back never spans more than one wave's window; skipped entirely when
-// gated off.  Each block takes the next tile from a ticket counter, so a tile
-// only waits on tiles whose blocks already run.  It publishes its sum
+// look-back never spans more than one wave's window.  Each block takes the next
+// tile from a ticket counter, so a tile only waits on tiles whose blocks already
+// run.  It publishes its sum
 // (kScanAgg); wave 0 looks back over the predecessors, adding sums until it
 // meets a tile that holds its inclusive prefix (kScanInc); the tile then
 // publishes its own.  Waits are bounded: a tile whose predecessors are not
@@ -368,14 +337,13 @@ __device__ __forceinline__ void scan_flag_store(unsigned long long* p, uint64_t 
 
 template <class In>
 __device__ __forceinline__ void scan_onepass_run(const In& in, uint32_t* __restrict__ out, DevN dn,
-                                                 const uint32_t* __restrict__ gate, uint64_t* __restrict__ total,
+                                                 uint64_t* __restrict__ total,
                                                  uint32_t* __restrict__ row_end, unsigned long long* __restrict__ st,
                                                  int64_t ntiles, int spin) {
     __shared__ uint64_t sm[kBlock / kWave + 1];
     __shared__ int64_t s_tile;
     __shared__ uint64_t s_excl;
     __shared__ int s_stalled, s_last;
-    if (gated_off(gate)) return;
     const int64_t n = dn.get();
     if (threadIdx.x == 0) s_tile = (int64_t)atomicAdd(&st[0], 1ull);
     __syncthreads();
@@ -478,10 +446,10 @@ __device__ __forceinline__ void scan_onepass_run(const In& in, uint32_t* __restr
 
 template <class In>
 __global__ void __launch_bounds__(kBlock) k_scan(In in, uint32_t* __restrict__ out, DevN dn,
-                                                  const uint32_t* __restrict__ gate, uint64_t* __restrict__ total,
+                                                  uint64_t* __restrict__ total,
                                                   uint32_t* __restrict__ row_end, unsigned long long* __restrict__ st,
                                                   int64_t ntiles, int spin) {
-    scan_onepass_run(in, out, dn, gate, total, row_end, st, ntiles, spin);
+    scan_onepass_run(in, out, dn, total, row_end, st, ntiles, spin);
 }
 
 // Two independent scans in one launch (a pair of the kernels above): the
@@ -492,9 +460,7 @@ struct ScanJob {
     In in;
     uint32_t* out;
     DevN dn;
-    const uint32_t* gate;
     uint64_t* total;
-    uint32_t* row_end;
     unsigned long long* st;
     uint64_t* partial;
     int64_t ntiles;
@@ -503,39 +469,38 @@ struct ScanJob {
 template <class A, class B>
 __global__ void __launch_bounds__(kBlock) k_scan_pair(ScanJob<A> a, ScanJob<B> b, int spin) {
     if ((int64_t)blockIdx.x < a.ntiles)
-        scan_onepass_run(a.in, a.out, a.dn, a.gate, a.total, a.row_end, a.st, a.ntiles, spin);
+        scan_onepass_run(a.in, a.out, a.dn, a.total, nullptr, a.st, a.ntiles, spin);
     else
-        scan_onepass_run(b.in, b.out, b.dn, b.gate, b.total, b.row_end, b.st, b.ntiles, spin);
+        scan_onepass_run(b.in, b.out, b.dn, b.total, nullptr, b.st, b.ntiles, spin);
 }
 
 template <class A, class B>
 __global__ void __launch_bounds__(kBlock) k_scan_reduce_pair(ScanJob<A> a, ScanJob<B> b) {
     const int64_t t = blockIdx.x;
-    if (t < a.ntiles) scan_reduce_tile(a.in, a.dn, a.gate, a.partial, t);
-    else scan_reduce_tile(b.in, b.dn, b.gate, b.partial, t - a.ntiles);
+    if (t < a.ntiles) scan_reduce_tile(a.in, a.dn, a.partial, t);
+    else scan_reduce_tile(b.in, b.dn, b.partial, t - a.ntiles);
 }
 
 template <class A, class B>
 __global__ void __launch_bounds__(1024) k_scan_partials_pair(ScanJob<A> a, ScanJob<B> b) {
-    if (blockIdx.x == 0) scan_partials_run(a.partial, a.ntiles, a.gate, a.total, a.row_end, a.dn);
-    else scan_partials_run(b.partial, b.ntiles, b.gate, b.total, b.row_end, b.dn);
+    if (blockIdx.x == 0) scan_partials_run(a.partial, a.ntiles, a.total, nullptr, a.dn);
+    else scan_partials_run(b.partial, b.ntiles, b.total, nullptr, b.dn);
 }
 
 template <class A, class B>
 __global__ void __launch_bounds__(kBlock) k_scan_down_pair(ScanJob<A> a, ScanJob<B> b) {
     const int64_t t = blockIdx.x;
-    if (t < a.ntiles) scan_down_tile(a.in, a.out, a.dn, a.gate, a.partial, t);
-    else scan_down_tile(b.in, b.out, b.dn, b.gate, b.partial, t - a.ntiles);
+    if (t < a.ntiles) scan_down_tile(a.in, a.out, a.dn, a.partial, t);
+    else scan_down_tile(b.in, b.out, b.dn, b.partial, t - a.ntiles);
 }
 
 // The whole scan in one block, for short inputs (one launch, no state):
 // tiles of 1024 x kScanIPT items in turn, carrying the running sum.
 template <class In>
 __global__ void __launch_bounds__(1024) k_scan_small(In in, uint32_t* __restrict__ out, DevN dn,
-                                                      const uint32_t* __restrict__ gate, uint64_t* __restrict__ total,
+                                                      uint64_t* __restrict__ total,
                                                       uint32_t* __restrict__ row_end) {
     __shared__ uint32_t sm[1024 / kWave + 1];
-    if (gated_off(gate)) return;
     const int64_t n = dn.get();
     uint32_t carry = 0;
     uint64_t carry64 = 0;
@@ -564,26 +529,16 @@ __global__ void __launch_bounds__(1024) k_scan_small(In in, uint32_t* __restrict
 
 // Fill n = dn.get() 32-bit words with `value` (a kernel rather than a memset
 // node, so that a captured pass replays it as a kernel).
-__global__ void __launch_bounds__(kBlock) k_fill_u32(uint32_t* __restrict__ p, DevN dn, uint32_t value,
-                                                    const uint32_t* __restrict__ gate) {
-    if (gated_off(gate)) return;
+__global__ void __launch_bounds__(kBlock) k_fill_u32(uint32_t* __restrict__ p, DevN dn, uint32_t value) {
     const int64_t n = dn.get();
     for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) p[i] = value;
 }
 
-__global__ void __launch_bounds__(kBlock) k_fill_u8(uint8_t* __restrict__ p, DevN dn, uint8_t value) {
-    const int64_t n = dn.get();
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) p[i] = value;
-}
-
-// Several fills in one launch: fill y of the grid is job y (32-bit words or
-// bytes), each gated on its own.
+// Several fills in one launch: fill y of the grid is job y.
 struct FillJob {
-    void* p;
+    uint32_t* p;
     DevN n;
     uint32_t value;
-    const uint32_t* gate;
-    int bytes;   // 4 or 1
 };
 constexpr int kMaxFillJobs = 6;
 struct FillSet {
@@ -592,24 +547,8 @@ struct FillSet {
 
 __global__ void __launch_bounds__(kBlock) k_fill_many(FillSet s) {
     const FillJob& J = s.j[blockIdx.y];
-    if (gated_off(J.gate)) return;
     const int64_t n = J.n.get();
-    if (J.bytes == 4) {
-        uint32_t* p = static_cast<uint32_t*>(J.p);
-        for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
-            p[i] = J.value;
-    } else {
-        uint8_t* p = static_cast<uint8_t*>(J.p);
-        for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
-            p[i] = (uint8_t)J.value;
-    }
-}
-
-// off[n] = the low 32 bits of a scan total (the end of the last CSR row).
-__global__ void k_set_row_end(uint32_t* __restrict__ off, DevN dn, const uint64_t* __restrict__ total,
-                              const uint32_t* __restrict__ gate) {
-    if (gated_off(gate)) return;
-    if (blockIdx.x == 0 && threadIdx.x == 0) off[dn.get()] = (uint32_t)*total;
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) J.p[i] = J.value;
 }
 
 }  // namespace tmc
