@@ -116,6 +116,27 @@ def test_slabs_in_a_batch():
         eng.close()
 
 
+def test_capacities_and_rerun_together():
+    """A new context learns the cells' sizes, then the records', and that the
+    pass has to be run stage by stage, within its three attempts."""
+    flags = SIMPLIFY_ALL | TRIANGLES
+    f = np.random.default_rng(8).standard_normal((3, 3, 100000)).astype(np.float32)
+    vols = [(f, ISO, tmc_amd.Grid.make(f.shape))] + [(s, iso, g) for s, g, iso in (_slab("6x8"), _slab("6x6", 12))]
+    eng, ref = tmc_amd.Engine(0), tmc_amd.Engine(0)
+    try:
+        print("[gpu] capacities and rerun together", flush=True)
+        ms = eng.extract_batch(vols, flags=flags)
+        assert ms[0].host_syncs == 3 + 1   # the last for the records
+        for i, (v, iso, g) in enumerate(vols):
+            ref.extract(v, iso, g, flags=flags)
+            exp, got = ref.download(), eng.download_batch(i)
+            for k in KEYS:
+                assert_same(got[k], exp[k], f"volume {i}: {k}")
+    finally:
+        eng.close()
+        ref.close()
+
+
 def test_slab_without_allocation():
     flags = SIMPLIFY_ALL | TRIANGLES
     f, g, iso = _slab("6x8")
