@@ -57,8 +57,8 @@ constexpr size_t kMaxSeen = 4096;
 constexpr int kCaptureAfter = 2;
 // capacity floor of a pass: its cells, up to this many
 constexpr int64_t kSmallPassCells = (int64_t)1 << 18;
-// k_vertices blocks: 256 CUs x 2 resident blocks (22 KB of LDS, 235 VGPRs
-// each) x 4 rounds
+// k_vertices blocks: 256 CUs x 2 resident blocks (22 KB of LDS; 252 VGPRs for
+// one volume of floats, 235 for a batch) x 4 rounds
 constexpr int64_t kVerticesBlocks = 2048;
 
 struct StageMark {

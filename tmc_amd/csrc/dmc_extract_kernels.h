@@ -809,11 +809,12 @@ __global__ void __launch_bounds__(kBlock) TMC_VERTICES_ATTR k_vertices(VolTable 
     vertices_run<T, 7, MANY>(vt, rec, grpV, dA, vpos, vnrm, vo, slow, qhead);
 }
 
-// K3 for larger passes: samples one at a time, which fits 3 waves per SIMD
-// (166 VGPRs for F32 fields, no scratch), so more cells hide each other's
-// memory waits (1024^3 Schwarz-P: 20.25 -> 19.85 ms per extraction; one
-// 128^3 volume: 0.401 -> 0.407 ms, hence the two forms).  The same
-// arithmetic in the same order as k_vertices.
+// K3 for larger passes of floats: samples one at a time, which fits 3 waves per
+// SIMD (a batch: 165 VGPRs; one volume, whose descriptor is in registers: 168
+// with four spilled, 20 B of scratch a lane, and faster all the same), so more
+// cells hide each other's memory waits (when it was added, 1024^3 Schwarz-P:
+// 20.25 -> 19.85 ms per extraction; one 128^3 volume: 0.401 -> 0.407 ms, hence
+// the two forms).  The same arithmetic in the same order as k_vertices.
 template <class T, bool MANY>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 3)))
 k_vertices_wide(VolTable vt, const uint4* __restrict__ rec, const uint32_t* __restrict__ grpV, DevN dA,
@@ -824,7 +825,8 @@ k_vertices_wide(VolTable vt, const uint4* __restrict__ rec, const uint32_t* __re
 
 // General path of K3 for the cells k_vertices deferred: every contour is
 // sampled with the box test at 9 x 9 and, where that finds no point, at
-// 28 x 28; failed projections are counted per volume.
+// 28 x 28; failed projections are counted per volume.  237 VGPRs for floats, two
+// waves per SIMD; doubles take 255 and 2 AGPRs, one wave.
 template <class T>
 __global__ void __launch_bounds__(kBlock) k_vertices_slow(VolTable vt, const uint4* __restrict__ rec,
                                                           const uint32_t* __restrict__ grpV,

@@ -3,11 +3,15 @@
 //
 // Halfedge h = 4q + k runs from quads[4q+k] to quads[4q+(k+1)%4]; face and
 // next are implicit, twins and flags are stored (4 B + 1 B per halfedge).
-// Twins are found through a per-vertex CSR of outgoing (halfedge,
-// destination) pairs instead of the reference's map keyed by the vertex pair
-// (cpp_dmc/DualMarchingCubes.cpp:488-671): the halfedges sharing an edge
-// {a, b} are the out-halfedges of a ending at b plus those of b ending at a,
-// taken in ascending halfedge order, which is the map's insertion order.
+// The usual pass writes the first twins with the quadrilaterals
+// (dmc_quad_kernels.h) and keeps them up to date while it simplifies
+// (dmc_simplify_kernels.h); the kernels here pair a mesh as it stands, for the
+// passes run stage by stage and the diagnostics.  They find twins through a
+// per-vertex CSR of outgoing (halfedge, destination) pairs instead of the
+// reference's map keyed by the vertex pair (cpp_dmc/DualMarchingCubes.cpp:
+// 488-671): the halfedges sharing an edge {a, b} are the out-halfedges of a
+// ending at b plus those of b ending at a, taken in ascending halfedge order,
+// which is the map's insertion order.
 #pragma once
 #include "dmc_kernels.h"
 
@@ -110,10 +114,10 @@ __device__ __forceinline__ int he_group(const int32_t* __restrict__ quads, const
 // Flag bytes are the reference's: 0 manifold, 1 non-manifold (4 faces),
 // 2 boundary multiple edge (3 faces).  A group of more than 4 faces (the
 // reference's error case) keeps 0 in the output; inside the engine its
-// members carry kFlagErr (its first member kFlagErrFirst) so that a build
-// that carries the group over can still count it.  Every test of a flag
-// compares with 1 or 2, which the markers never equal; the final build
-// clears them.
+// members carry kFlagErr (its first member kFlagErrFirst) so that a stage that
+// takes a face away can still count the group.  Every test of a flag
+// compares with 1 or 2, which the markers never equal; the final mesh has them
+// cleared (k_final_faces, the last k_he_twins).
 constexpr uint8_t kFlagErr = 0x80, kFlagErrFirst = 0xC0;
 
 // Twin and flag from a sorted group (cpp_dmc/DualMarchingCubes.cpp:574-669).
