@@ -38,10 +38,10 @@ HBM_PEAK_GBS = 8000.0
 # Bytes per extraction the cell-stage kernels move between L2 and the fabric
 # (HBM and Infinity Cache), from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE
 # scaled by the copy-kernel calibration
-# (profiles/dmc_schwarz_1024_kernel_traffic.md): k_sweep 5.51 GB, k_cells
-# 0.94 GB, k_vertices (its 3-wave form) 11.62 GB, k_quads 4.59 GB, the cell
-# scans 0.06 GB.
-TRAFFIC = {"schwarz_1024": 22_700_000_000}
+# (profiles/dmc_schwarz_1024_kernel_traffic.md): k_sweep 5.52 GB, k_cells
+# 0.94 GB, k_vertices (its 3-wave form) 11.98 GB, k_quads 4.53 GB, the cell
+# scans 0.05 GB.
+TRAFFIC = {"schwarz_1024": 23_030_000_000}
 CELL_KERNELS = ("k_sweep", "k_scan_cells", "k_vol_abase", "k_cells", "k_vol_bounds", "k_vertices", "k_vertices_slow",
                 "k_quads")
 

@@ -145,7 +145,8 @@ dmc_status dmc_extract_batch(dmc_context* ctx, const dmc_volume* vols, int32_t n
  *
  * Limits: at most 2,097,152 grid points (128^3); the working set of the
  * field's surface must fit the 64 MiB scratch (a smooth surface on 128^3
- * does, about 40 MiB; dense noise fits up to about 64^3).  Beyond either,
+ * does, about 40 MiB; white noise fits to 49^3 with all simplifications and
+ * triangles, to 74^3 with neither).  Beyond either,
  * DMC_ERR_CAPACITY with the reason in dmc_last_error.  The field (and
  * gradients, DMC_GRADIENTS_SUPPLIED) must be device pointers; the flag
  * DMC_FIELD_ON_DEVICE is implied and DMC_STAGE_TIMING is ignored.
@@ -347,13 +348,12 @@ dmc_status tmc_download(dmc_context* ctx, double* positions, double* normals, in
  * kernels launch with fixed block sizes over one thread per item,
  * dmc/DualMarchingCubes.cu).  Results never depend on the launch shape,
  * only the time does.
- *   grid_cap     blocks (256 threads) of every grid-stride kernel, which
- *                loops over its items: 64 .. 2^24, default 32768 (env
- *                TMC_GRID_CAP);
+ *   grid_cap     at most this many blocks (256 threads) of every grid-stride
+ *                kernel, which loops over its items: 64 .. 2^24, default
+ *                32768 (env TMC_GRID_CAP); some kernels take fewer;
  *   sweep_waves  waves the field sweep aims for, one 256-cell x 4-row tile
  *                (8 rows from 2^28 points on) of K planes each; sets K:
- *                256 .. 2^24,
- *                default 32768 (env TMC_SWEEP_WAVES).
+ *                256 .. 2^24, default 32768 (env TMC_SWEEP_WAVES).
  * There is no hash-table load factor to choose: vertex and quadrilateral
  * ids come from prefix sums over the cells, not from hash tables.
  * ---------------------------------------------------------------------- */
